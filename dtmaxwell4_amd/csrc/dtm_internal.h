@@ -325,24 +325,17 @@ void fail_launch(const char* kernel, const char* why);
 // 1 and the message when a failure was recorded since the last call (cleared).
 int take_launch_error(char* msg, int cap);
 
-// Launchers (dtm_kernels.hip).  All enqueue on `st`; each sweep is one
-// launch of the kernel variant with every boundary rule over `regs`.
-// fold non-null: add a plane-wave TF/SF source along x inside the sweep,
-// from this half-step's per-plane factor table (launch_tfsf_fold); ignored
-// with an FP32 zone
-// side: with an FP32 zone, the zone's column runs on side.st between the
-// fork and join events (concurrently with the rest of the grid on st); null:
-// both launches on st.
-struct SideStream {
-  hipStream_t st;
-  hipEvent_t fork, join;
-};
-void launch_update_h(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                     const Region* regs, int nreg, hipStream_t st, const float* fold = nullptr,
-                     const SideStream* side = nullptr);
-void launch_update_e(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                     const Materials& mt, const Ade& ade, const Region* regs, int nreg, hipStream_t st,
-                     const float* fold = nullptr, const SideStream* side = nullptr);
+// Launchers; all enqueue on `st`.
+// One half-step (up 0: H, 1: E) of the x planes [i0, i1) (dtm_sweep.hip).
+// fold non-null: add a plane-wave TF/SF source along x inside the sweep, from
+// this half-step's per-plane factors (launch_tfsf_fold) and the weights of
+// every chunk of cells (launch_fold_weights); none with an FP32 zone.
+void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
+                  const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
+                  hipStream_t st);
+// entries of the weights, both half-steps
+long long fold_weights_size(const Grid& g);
+void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t st);
 // floats per half-step of the fold factor table: (nx + 1) * 8
 void launch_tfsf_fold(const Tfsf& tf, const double* tables, float* out, int nsteps, const Grid& g,
                       hipStream_t st);

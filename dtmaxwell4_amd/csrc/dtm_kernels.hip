@@ -1,20 +1,6 @@
-// dtm_kernels.hip — hand-written gfx950 kernels of the FDTD stepping path.
-//
-// One launch per half-step ("two-pass" sweep).  Each launch covers a set of
-// boxes (regions): the interior box where every x/y stencil neighbour exists
-// and only z can touch a boundary or a CPML slab, and up to four x/y edge
-// slabs handled with full boundary logic — the zone split of the reference's
-// Window::calcDtorres (window.hpp:126-145) without its host loop.
-//
-// Thread mapping: 256 threads = 64 (z, one wavefront) x 4 (y).  Blocks are
-// remapped so that each of the 8 XCDs sweeps a contiguous run of (x,y) rows,
-// keeping the x/y stencil neighbours of a block in that XCD's L2.
-//
-// Update equations (genAlg.py:182-301, constants defs.h:3-13), on the cell
-// lattice of include/dtmaxwell4.h:
-//   H^{n+1/2} = H^{n-1/2} - dt curl E^n          (body diamond, time 0)
-//   E^{n+1}   = E^n + dt/eps curl H^{n+1/2}      (nose diamond, time 1/2)
-// with the (2,4) difference D f = [27 (f_{+1/2} - f_{-1/2}) - (f_{+3/2} - f_{-3/2})]/(24 d).
+// dtm_kernels.hip — the kernels around the half-step sweeps (dtm_sweep.hip):
+// TF/SF corrections and their tables, dispersive and gyrotropic cells, soft
+// sources, probes, and conversion of half-precision fields.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -25,10 +11,6 @@
 #include "dtm_internal.h"
 
 namespace dtm {
-
-constexpr int BZ = 64;  // z extent of a block (one wavefront)
-constexpr int BY = 4;   // y extent of a block
-constexpr int NXCD = 8;
 
 // ------------------------------------------------------- storage helpers
 __device__ __forceinline__ float ld(const float* F, long long q, float) { return F[q]; }
@@ -230,549 +212,12 @@ __device__ __forceinline__ long long psi_index(const Grid& g, const Cpml& p, int
   return ((long long)i * g.ny + j) * P + s;
 }
 
-// Split-field part update (genAlg.py:117-148): F = P1 + P2 with P2 stored,
-// P1 <- k1a P1 + k2a ua and P2 <- k1b P2 + k2b ub, ua / ub the increments of
-// the first and second curl term.  Outside every slab of the component
-// (k2 = 1 on both axes) it is the plain update F + ua + ub.
-__device__ __forceinline__ float split_step(float* P2, long long q, float f0, float k1a, float k2a, float ua,
-                                            float k1b, float k2b, float ub) {
-  if (k2a == 1.0f && k2b == 1.0f) return f0 + ua + ub;
-  const float p2 = P2[q], p1 = f0 - p2;
-  const float n1 = k1a * p1 + k2a * ua, n2 = k1b * p2 + k2b * ub;
-  P2[q] = n2;
-  return n1 + n2;
-}
-
-// 32-bit psi indices of the sweeps (psi arrays are far below 2^32 floats):
-// z slab: base + slab index; x and y slabs: base + (k - k_lane0).
-__device__ __forceinline__ unsigned psi_base_z(const Grid& g, const Cpml& p, int i, int j) {
-  return ((unsigned)i * (unsigned)g.ny + (unsigned)j) * (unsigned)(p.plo[2] + p.phi[2]);
-}
-__device__ __forceinline__ unsigned psi_base_y(const Grid& g, const Cpml& p, int ys, int i, int k) {
-  return ys < 0 ? 0u : ((unsigned)i * (unsigned)(p.plo[1] + p.phi[1]) + (unsigned)ys) * (unsigned)g.nz + (unsigned)k;
-}
-__device__ __forceinline__ unsigned psi_base_x(const Grid& g, const Cpml& p, int xs, int j, int k) {
-  (void)p;
-  return ((unsigned)xs * (unsigned)g.ny + (unsigned)j) * (unsigned)g.nz + (unsigned)k;
-}
-
 // psi <- b psi + c D ; D <- D + psi   (CPML, kappa=1, alpha=0)
 __device__ __forceinline__ void cpml_apply(float* psi, long long pq, float b, float c, float& D) {
   float v = b * psi[pq] + c * D;
   psi[pq] = v;
   D += v;
 }
-// The same with the old psi value already loaded.
-__device__ __forceinline__ void cpml_step(float* psi, long long pq, float old, float b, float c, float& D) {
-  const float v = b * old + c * D;
-  psi[pq] = v;
-  D += v;
-}
-
-// ===================================================== marching sweeps
-// A block owns a tile of 64 (z) x ROWS (y) columns and marches along x over
-// a segment of planes (the tilted space-time march of the reference's torre,
-// genAlg.py:420-499, with the rag shuffles of copyrags.cuh replaced by an
-// LDS ring): the x stencil reads a 5-plane ring of the two transverse
-// components, the y/z stencils a double-buffered LDS tile of the current
-// plane with a 3-cell halo, and operands are prefetched PF planes ahead in
-// registers.  One barrier per plane.
-// y rows per block (ROWS): 8, or 16 with one cell per lane when the launch
-// then fills the chip as well (see upd_h).  At 512x256x256 the FP32 E sweep
-// ran 7% faster with 16 rows (the H sweep 1%); the paired FP16 sweeps ran 8%
-// slower, and at 400x200x200 the 16-row launch left a fifth of the CUs idle.
-constexpr int MLZ = 67;   // LDS row length: 64 + 3 halo columns
-
-struct MarchSet {
-  int n;
-  Region r[6];
-  int nbk[6], nbj[6], nbs[6];
-  int start[7];
-  int total, per, seg;
-  int bz;  // z extent of a tile: BZ * (cells per lane)
-  int by;  // y extent of a tile: the kernel's ROWS
-};
-
-static MarchSet make_march(const Region* regs, int nreg, int seg, int bz, int by) {
-  MarchSet s{};
-  s.seg = seg;
-  s.bz = bz;
-  s.by = by;
-  int acc = 0, m = 0;
-  for (int t = 0; t < nreg && m < 6; t++) {
-    const Region& r = regs[t];
-    if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) continue;
-    s.r[m] = r;
-    s.nbk[m] = (r.k1 - r.k0 + bz - 1) / bz;
-    s.nbj[m] = (r.j1 - r.j0 + by - 1) / by;
-    s.nbs[m] = (r.i1 - r.i0 + seg - 1) / seg;
-    s.start[m] = acc;
-    acc += s.nbk[m] * s.nbj[m] * s.nbs[m];
-    m++;
-  }
-  s.n = m;
-  s.start[m] = acc;
-  s.total = acc;
-  s.per = (acc + NXCD - 1) / NXCD;
-  return s;
-}
-
-struct MarchTile {
-  int r, i0, i1, j0, k0;
-};
-
-__device__ __forceinline__ bool march_locate(const MarchSet& ms, MarchTile& t) {
-  const int b = blockIdx.x;
-  const int L = (b % NXCD) * ms.per + b / NXCD;  // XCD-contiguous logical id
-  if (L >= ms.total) return false;
-  int r = 0;
-  while (r + 1 < ms.n && L >= ms.start[r + 1]) r++;
-  int loc = L - ms.start[r];
-  const int bk = loc % ms.nbk[r];
-  loc /= ms.nbk[r];
-  const int bj = loc % ms.nbj[r];
-  const int bs = loc / ms.nbj[r];
-  const Region& R = ms.r[r];
-  t.r = r;
-  t.k0 = R.k0 + bk * ms.bz;
-  t.j0 = R.j0 + bj * ms.by;
-  t.i0 = R.i0 + bs * ms.seg;
-  t.i1 = min(t.i0 + ms.seg, R.i1);
-  return true;
-}
-
-// In-plane offset (j*sy + k) of a position under the boundary rule, or -1.
-__device__ __forceinline__ long long plane_off(const Grid& g, int j, int k) {
-  const int jj = nbr(j, 0, g.ny, g.per[1]), kk = nbr(k, 0, g.nz, g.per[2]);
-  return (jj < 0 || kk < 0) ? -1LL : (long long)jj * g.sy + kk;
-}
-template <bool GEN>
-__device__ __forceinline__ long long plane_base(const Grid& g, int i) {
-  if (!GEN) return (long long)i * g.sx;
-  const int ii = nbr(i, 0, g.nx, g.per[0]);
-  return ii < 0 ? -1LL : (long long)ii * g.sx;
-}
-template <typename T>
-__device__ __forceinline__ float ldp(const T* F, long long base, long long off, float inv) {
-  return (base < 0 || off < 0) ? 0.0f : ld(F, base + off, inv);
-}
-
-// Barrier that waits only for this wave's LDS traffic, so global loads
-// issued for the next plane stay in flight across it (__syncthreads would
-// also drain every outstanding global load).  The "memory" clobber keeps the
-// compiler from moving LDS accesses across it.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Raw storage element and its conversion: prefetched operands stay in the
-// storage type until they are published to LDS, so no conversion (and no
-// wait for the load) sits next to the load that produced them.
-template <int STORE> struct Raw;
-template <> struct Raw<0> { using T = float; };
-template <> struct Raw<1> { using T = __half; };
-__device__ __forceinline__ float cvt(float v, float) { return v; }
-__device__ __forceinline__ float cvt(__half v, float inv) { return __builtin_fmaf(__half2float(v), inv, 0.0f); }
-template <typename T> __device__ __forceinline__ T rzero();
-template <> __device__ __forceinline__ float rzero<float>() { return 0.0f; }
-template <> __device__ __forceinline__ __half rzero<__half>() { return __ushort_as_half((unsigned short)0); }
-template <typename T>
-__device__ __forceinline__ T ldr(const T* F, long long base, long long off) {
-  return (base < 0 || off < 0) ? rzero<T>() : F[base + off];
-}
-// Address of a position under the boundary rule: outside the grid (base or
-// off < 0) it is the array's zero pad, so the load itself is unconditional
-// and its destination register never needs a merge (a merge would force a
-// wait for the load before the next plane).  The index type I is 32-bit
-// below 2^32 - kPad cells, which keeps the select out of 64-bit registers,
-// and 64-bit in the wide variants (IxT).
-template <bool W> struct IxT { using T = unsigned; };
-template <> struct IxT<true> { using T = unsigned long long; };
-template <typename T, typename I>
-__device__ __forceinline__ const T* at(const T* F, long long base, long long off, I zidx) {
-  const I idx = (base < 0 || off < 0) ? zidx : (I)(base + off);
-  return F + idx;
-}
-
-// Ring slot of plane p in a 5-plane LDS ring (p >= -3).
-__device__ __forceinline__ int ring5(int p) { return (p + 10) % 5; }
-
-// ================================================================ H sweep
-// V consecutive z cells per lane (V = 2 for FP16 storage on an even nz: the
-// lane loads one __half2, so a prefetch register carries two cells, the
-// same bytes in flight per register as FP32).  Raw word of V cells:
-template <int STORE, int V> struct Vec;
-template <> struct Vec<0, 1> { using P = float; };
-template <> struct Vec<1, 1> { using P = __half; };
-template <> struct Vec<1, 2> { using P = __half2; };
-__device__ __forceinline__ void unpackv(float p, float, float* o) { o[0] = p; }
-__device__ __forceinline__ void unpackv(__half p, float inv, float* o) {
-  o[0] = __builtin_fmaf(__half2float(p), inv, 0.0f);
-}
-// The conversions are written as fma(x, scale, 0): one mixed-precision
-// v_fma_mix (half operand, float result) per value instead of a convert and
-// a multiply.  The scale is a power of two, so the product is exact and the
-// result is the same as the convert-then-multiply.
-__device__ __forceinline__ void unpackv(__half2 p, float inv, float* o) {
-  const float2 f = __half22float2(p);
-  o[0] = __builtin_fmaf(f.x, inv, 0.0f);
-  o[1] = __builtin_fmaf(f.y, inv, 0.0f);
-}
-template <typename P> __device__ __forceinline__ P pzero();
-template <> __device__ __forceinline__ float pzero<float>() { return 0.0f; }
-template <> __device__ __forceinline__ __half pzero<__half>() { return __ushort_as_half((unsigned short)0); }
-template <> __device__ __forceinline__ __half2 pzero<__half2>() { return __half2(pzero<__half>(), pzero<__half>()); }
-// store V values at element q (q even for V = 2)
-__device__ __forceinline__ void stv(float* F, long long q, const float* v, float) { F[q] = v[0]; }
-__device__ __forceinline__ void stv(__half* F, long long q, const float* v, float s) {
-  F[q] = __float2half_rn(__builtin_fmaf(v[0], s, 0.0f));
-}
-__device__ __forceinline__ void stv2(__half* F, long long q, const float* v, float s) {
-  *reinterpret_cast<__half2*>(F + q) =
-      __floats2half2_rn(__builtin_fmaf(v[0], s, 0.0f), __builtin_fmaf(v[1], s, 0.0f));
-}
-// word of V cells at a position under the boundary rule (see at())
-template <typename P, typename T, typename I>
-__device__ __forceinline__ P ldv(const T* F, long long base, long long off, I zidx) {
-  const I idx = (base < 0 || off < 0) ? zidx : (I)(base + off);
-  return *reinterpret_cast<const P*>(F + idx);
-}
-
-// Operands of one plane, loaded PF planes ahead: the Ex tile words of
-// plane p (own, y-halo row) and the Ex z-halo value, the H read-modify-write
-// words of plane p, and the Ey / Ez tile values of plane p+1 (the x stencil
-// of H reaches one plane ahead).
-template <typename P, typename T> struct PreH {
-  P ex, exy, hx, hy, hz, ey, ez, ezy;
-  T exz, eyz;
-};
-
-// GEN bit 0: x boundary rule and x CPML (per plane, block-uniform);
-// bit 1: y CPML (per row).  The y and z boundary rules and the z CPML are
-// always on: they are per-thread constants.
-// SP: split-field absorbing layer instead of the CPML (one cell per lane).
-// TF: a plane-wave TF/SF source along x folded in: the correction of
-// genAlg.py:219-221 is added to the derivative it belongs to before the CPML
-// and split-field updates, which are linear in it (the k_tfsf kernel applies
-// the same terms after a sweep); fold: this half-step's factor table.
-// W: 64-bit cell indices (grids of 2^32 - kPad cells and more).
-template <int STORE, int GEN, int V, bool SP = false, int ROWS = 8, bool XZ = false, bool TF = false, bool W = false>
-__global__ __launch_bounds__(BZ* ROWS, 4) void k_update_h(Grid g, Fields<STORE> f, Scales sc, Cpml pm, MarchSet ms,
-                                                         const float* fold) {
-  using T = typename Raw<STORE>::T;
-  using P = typename Vec<STORE, V>::P;
-  constexpr bool GX = GEN & 1, GY = GEN & 2;
-  constexpr int BZV = BZ * V, LZ = BZV + 3, MBY = ROWS;
-  __shared__ float sEx[2][MBY + 3][LZ];  // [row j-j0+2][col k-k0+2], plane i
-  __shared__ float rEy[5][MBY][LZ];      // [row j-j0][col k-k0+2], ring of planes
-  __shared__ float rEz[5][MBY + 3][BZV]; // [row j-j0+2][col k-k0], ring of planes
-  __shared__ float sHo[3][MBY][BZV];     // this thread's H operands of plane i
-  MarchTile t;
-  if (!march_locate(ms, t)) return;
-  const Region& R = ms.r[t.r];
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int j = t.j0 + ty, k = t.k0 + V * tx;  // first of this lane's V cells
-  const int c0 = V * tx;                       // its tile column
-  const bool inreg = j < R.j1 && k < R.k1;     // V = 2 needs an even nz: cells pair up
-  const long long own = plane_off(g, j, k);
-  // halo positions: rows j0-2, j0-1, j0+MBY (waves ty<3); columns k0-2, k0-1, k0+BZV (lanes tx<3)
-  const bool yw = ty < 3, zl = tx < 3;
-  const int yrow = ty < 2 ? ty : MBY + 2;
-  const long long yh = yw ? plane_off(g, t.j0 + (ty < 2 ? ty - 2 : MBY), k) : -1;
-  const int zcol = tx < 2 ? tx : BZV + 2;
-  const long long zh = zl ? plane_off(g, j, t.k0 + (tx < 2 ? tx - 2 : BZV)) : -1;
-  const T* Ex = f.E[0];
-  const T* Ey = f.E[1];
-  const T* Ez = f.E[2];
-  T* Hx = f.H[0];
-  T* Hy = f.H[1];
-  T* Hz = f.H[2];
-  const float iex = sc.ie[0], iey = sc.ie[1], iez = sc.ie[2];
-  const float ihx = sc.ih[0], ihy = sc.ih[1], ihz = sc.ih[2];
-  using Ix = typename IxT<W>::T;
-  const Ix zi = W ? (Ix)g.zidxw : (Ix)g.zidx;  // zero pad index
-
-  const long long hq = inreg ? own : -1;  // H operands: owned cells only
-  // FP32 zone (FP16 storage): a block whose tile (with its halo) meets the
-  // zone replaces the LDS values of zone cells by their FP32 copies and
-  // writes its new zone values there too
-  static_assert(!XZ || STORE == 1, "the FP32 zone applies to FP16 storage");
-  const Exact& xz = sc.xz;
-  bool xtile = false;
-  if constexpr (XZ)
-    xtile = xz.on && (g.per[1] || g.per[2] ||
-                      (xz.j0 < t.j0 + MBY + 3 && xz.j1 > t.j0 - 3 && xz.k0 < t.k0 + BZV + 3 && xz.k1 > t.k0 - 3));
-  const int jo = j;
-  const int jy = yw ? nbr(t.j0 + (ty < 2 ? ty - 2 : MBY), 0, g.ny, g.per[1]) : -1;
-  const int kz = zl ? nbr(t.k0 + (tx < 2 ? tx - 2 : BZV), 0, g.nz, g.per[2]) : -1;
-  auto ov = [&](float& dst, int comp, int pi, int pj, int pk) {
-    // rows and lanes past the grid's edge hold the wrapped cells on a
-    // periodic axis (plane_off), nothing otherwise
-    pj = nbr(pj, 0, g.ny, g.per[1]);
-    pk = nbr(pk, 0, g.nz, g.per[2]);
-    const int xq = (pi < 0 || pj < 0 || pk < 0) ? -1 : exact_idx(xz, pi, pj, pk);
-    if (xq >= 0) dst = xz.f[comp][xq];
-  };
-  auto fetch = [&](PreH<P, T>& S, int p) {
-    const long long pb = plane_base<GX>(g, p);
-    const long long pn = plane_base<GX>(g, p + 1);
-    S.ex = ldv<P>(Ex, pb, own, zi);
-    S.ey = ldv<P>(Ey, pn, own, zi);
-    S.ez = ldv<P>(Ez, pn, own, zi);
-    S.exy = ldv<P>(Ex, pb, yh, zi);
-    S.ezy = ldv<P>(Ez, pn, yh, zi);
-    S.exz = *at(Ex, pb, zh, zi);
-    S.eyz = *at(Ey, pn, zh, zi);
-    S.hx = ldv<P>((const T*)Hx, pb, hq, zi);
-    S.hy = ldv<P>((const T*)Hy, pb, hq, zi);
-    S.hz = ldv<P>((const T*)Hz, pb, hq, zi);
-  };
-  // Ey / Ez tile of plane p straight into its ring slot (prologue only)
-  auto ring_direct = [&](int p) {
-    const long long pb = plane_base<GX>(g, p);
-    const int s = ring5(p);
-    float v[V];
-    unpackv(ldv<P>(Ey, pb, own, zi), iey, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rEy[s][ty][c0 + q + 2] = v[q];
-    unpackv(ldv<P>(Ez, pb, own, zi), iez, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rEz[s][ty + 2][c0 + q] = v[q];
-    if (yw) {
-      unpackv(ldv<P>(Ez, pb, yh, zi), iez, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) rEz[s][yrow][c0 + q] = v[q];
-    }
-    if (zl) rEy[s][ty][zcol] = cvt(ldr(Ey, pb, zh), iey);
-    if constexpr (XZ) {
-      if (xtile) {
-        const int pp = GX ? nbr(p, 0, g.nx, g.per[0]) : p;
-#pragma unroll
-        for (int q = 0; q < V; q++) {
-          ov(rEy[s][ty][c0 + q + 2], 1, pp, jo, k + q);
-          ov(rEz[s][ty + 2][c0 + q], 2, pp, jo, k + q);
-          if (yw) ov(rEz[s][yrow][c0 + q], 2, pp, jy, k + q);
-        }
-        if (zl) ov(rEy[s][ty][zcol], 1, pp, jo, kz);
-      }
-    }
-  };
-
-  const int ysl = (GY && pm.on) ? slab_index(j, g.ny, pm.plo[1], pm.phi[1]) : -1;
-  const float rd0 = g.rd[0], rd1 = g.rd[1], rd2 = g.rd[2], dt = g.dt;
-  // CPML state of this lane's cells (z and y are fixed per thread)
-  int zs[V];
-  float bz[V], cz[V];
-#pragma unroll
-  for (int q = 0; q < V; q++) {
-    zs[q] = pm.on ? slab_index(k + q, g.nz, pm.plo[2], pm.phi[2]) : -1;
-    bz[q] = zs[q] >= 0 ? pm.bH[2][k + q] : 0.f;
-    cz[q] = zs[q] >= 0 ? pm.cH[2][k + q] : 0.f;
-  }
-  const float by = ysl >= 0 ? pm.bH[1][j] : 0.f, cy = ysl >= 0 ? pm.cH[1][j] : 0.f;
-  // TF/SF fold: this lane's packed weights (zero away from the y and z faces)
-  int tfw[V];
-#pragma unroll
-  for (int q = 0; q < V; q++) tfw[q] = 0;
-  if constexpr (TF) {
-    const int* hd = reinterpret_cast<const int*>(fold);
-#pragma unroll
-    for (int q = 0; q < V; q++) tfw[q] = fold_pack(0, j, k + q, hd);
-  }
-
-  // PF prefetch sets, each a plane ahead of the next: two planes in flight in
-  // the launched variants, which carry the y-CPML (three would spill).
-  constexpr int PF = (GY || V == 2) ? 2 : 3;
-  PreH<P, T> S[PF];
-#pragma unroll
-  for (int u = 0; u < PF; u++) {
-    S[u].ex = S[u].exy = S[u].hx = S[u].hy = S[u].hz = S[u].ey = S[u].ez = S[u].ezy = pzero<P>();
-    S[u].exz = S[u].eyz = rzero<T>();
-  }
-  ring_direct(t.i0 - 2);
-  ring_direct(t.i0 - 1);
-  ring_direct(t.i0);
-  // Prefetches are unconditional (a plane past the segment is clamped to
-  // its last plane): with no branch around them the compiler's in-order
-  // wait counts stay exact and a wait never reaches the other sets.
-#pragma unroll
-  for (int u = 0; u < PF; u++) fetch(S[u], min(t.i0 + u, t.i1 - 1));
-
-  auto step = [&](int i, PreH<P, T>& Q) {
-    const int b = i & 1;
-    const int s0 = ring5(i - 2), s1 = ring5(i - 1), s2 = ring5(i), s3 = ring5(i + 1);
-    // publish plane i (Ex) and plane i+1 (Ey, Ez); H operands to the own slots
-    float v[V];
-    unpackv(Q.ex, iex, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sEx[b][ty + 2][c0 + q + 2] = v[q];
-    unpackv(Q.ey, iey, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rEy[s3][ty][c0 + q + 2] = v[q];
-    unpackv(Q.ez, iez, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rEz[s3][ty + 2][c0 + q] = v[q];
-    if (yw) {
-      unpackv(Q.exy, iex, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) sEx[b][yrow][c0 + q + 2] = v[q];
-      unpackv(Q.ezy, iez, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) rEz[s3][yrow][c0 + q] = v[q];
-    }
-    if (zl) {
-      sEx[b][ty + 2][zcol] = cvt(Q.exz, iex);
-      rEy[s3][ty][zcol] = cvt(Q.eyz, iey);
-    }
-    // the H operands go through this thread's own LDS slots: no register of
-    // the prefetch set is live across its refetch
-    unpackv(Q.hx, ihx, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sHo[0][ty][c0 + q] = v[q];
-    unpackv(Q.hy, ihy, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sHo[1][ty][c0 + q] = v[q];
-    unpackv(Q.hz, ihz, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sHo[2][ty][c0 + q] = v[q];
-    if constexpr (XZ) {
-      if (xtile && (g.per[0] || (i + 1 >= xz.i0 && i - 1 < xz.i1))) {  // Ex of plane i, Ey / Ez of i+1, own H of i
-        const int ii = GX ? nbr(i, 0, g.nx, g.per[0]) : i;
-        const int i1n = GX ? nbr(i + 1, 0, g.nx, g.per[0]) : i + 1;
-#pragma unroll
-        for (int q = 0; q < V; q++) {
-          ov(sEx[b][ty + 2][c0 + q + 2], 0, ii, jo, k + q);
-          ov(rEy[s3][ty][c0 + q + 2], 1, i1n, jo, k + q);
-          ov(rEz[s3][ty + 2][c0 + q], 2, i1n, jo, k + q);
-          ov(sHo[0][ty][c0 + q], 3, ii, jo, k + q);
-          ov(sHo[1][ty][c0 + q], 4, ii, jo, k + q);
-          ov(sHo[2][ty][c0 + q], 5, ii, jo, k + q);
-          if (yw) {
-            ov(sEx[b][yrow][c0 + q + 2], 0, ii, jy, k + q);
-            ov(rEz[s3][yrow][c0 + q], 2, i1n, jy, k + q);
-          }
-        }
-        if (zl) {
-          ov(sEx[b][ty + 2][zcol], 0, ii, jo, kz);
-          ov(rEy[s3][ty][zcol], 1, i1n, jo, kz);
-        }
-      }
-    }
-    // CPML psi of plane i, loaded before the prefetch so that waiting for
-    // psi does not wait for it (loads complete in issue order)
-    // (z and y slabs; the x slab is a few planes, its psi is read in place)
-    float pz0[V], pz1[V], py0[V], py1[V];
-    const unsigned zb = psi_base_z(g, pm, i, j), yb = psi_base_y(g, pm, ysl, i, k);
-#pragma unroll
-    for (int q = 0; q < V; q++) {
-      pz0[q] = pz1[q] = py0[q] = py1[q] = 0.f;
-      if (!SP && inreg && zs[q] >= 0) {
-        pz0[q] = pm.psiH[2][0][zb + zs[q]];
-        pz1[q] = pm.psiH[2][1][zb + zs[q]];
-      }
-      if (!SP && GY && inreg && ysl >= 0) {
-        py0[q] = pm.psiH[1][0][yb + q];
-        py1[q] = pm.psiH[1][1][yb + q];
-      }
-    }
-    const int xsl = (GX && pm.on) ? slab_index(i, g.nx, pm.plo[0], pm.phi[0]) : -1;
-    // this plane's fold factors, loaded before the barrier (whose wait covers
-    // them) rather than inside the band branch
-    float fu[6];
-#pragma unroll
-    for (int t6 = 0; t6 < 6; t6++) fu[t6] = 0.f;
-    if constexpr (TF) {
-#pragma unroll
-      for (int t6 = 0; t6 < 6; t6++) fu[t6] = fold[kFoldStride * (1 + i) + t6];
-    }
-    fetch(Q, min(i + PF, t.i1 - 1));
-    lds_barrier();
-    if (inreg) {
-      float nx_[V], ny_[V], nz_[V];
-#pragma unroll
-      for (int q = 0; q < V; q++) {
-        const int c = c0 + q;
-        const float hx0 = sHo[0][ty][c], hy0 = sHo[1][ty][c], hz0 = sHo[2][ty][c];
-        const float exo = sEx[b][ty + 2][c + 2];
-        float dyEz = rd1 * d24(rEz[s2][ty][c], rEz[s2][ty + 1][c], rEz[s2][ty + 2][c], rEz[s2][ty + 3][c]);
-        float dyEx = rd1 * d24(sEx[b][ty][c + 2], sEx[b][ty + 1][c + 2], exo, sEx[b][ty + 3][c + 2]);
-        float dzEy = rd2 * d24(rEy[s2][ty][c], rEy[s2][ty][c + 1], rEy[s2][ty][c + 2], rEy[s2][ty][c + 3]);
-        float dzEx = rd2 * d24(sEx[b][ty + 2][c], sEx[b][ty + 2][c + 1], exo, sEx[b][ty + 2][c + 3]);
-        float dxEz = rd0 * d24(rEz[s0][ty + 2][c], rEz[s1][ty + 2][c], rEz[s2][ty + 2][c], rEz[s3][ty + 2][c]);
-        float dxEy = rd0 * d24(rEy[s0][ty][c + 2], rEy[s1][ty][c + 2], rEy[s2][ty][c + 2], rEy[s3][ty][c + 2]);
-        if constexpr (TF) {
-          if (tfw[q]) {  // a lane next to a y or z face (or inside the box on both)
-            const int w = tfw[q];
-            dyEz += fold_f(w, 0) * fu[0];   // Hx, y faces
-            dzEy += fold_f(w, 6) * fu[1];   // Hx, z faces
-            dzEx += fold_f(w, 12) * fu[2];  // Hy, z faces
-            dxEz += fold_b(w, 24) * fu[3];  // Hy, x faces
-            dxEy += fold_b(w, 25) * fu[4];  // Hz, x faces
-            dyEx += fold_f(w, 18) * fu[5];  // Hz, y faces
-          }
-        }
-        if constexpr (SP) {
-          // split parts, (k1, k2) = (1, 1) off the slab: Hx (y, z), Hy (z, x), Hz (x, y)
-          const bool sx = GX && xsl >= 0;
-          const float k1x = sx ? pm.bH[0][i] : 1.f, k2x = sx ? pm.cH[0][i] : 1.f;
-          const float k1y = (GY && ysl >= 0) ? by : 1.f, k2y = (GY && ysl >= 0) ? cy : 1.f;
-          const float k1z = zs[q] >= 0 ? bz[q] : 1.f, k2z = zs[q] >= 0 ? cz[q] : 1.f;
-          const long long qs = plane_base<GX>(g, i) + own + q;
-          nx_[q] = split_step(pm.p2H[0], qs, hx0, k1y, k2y, -dt * dyEz, k1z, k2z, dt * dzEy);
-          ny_[q] = split_step(pm.p2H[1], qs, hy0, k1z, k2z, -dt * dzEx, k1x, k2x, dt * dxEz);
-          nz_[q] = split_step(pm.p2H[2], qs, hz0, k1x, k2x, -dt * dxEy, k1y, k2y, dt * dyEx);
-        } else {
-          if (zs[q] >= 0) {  // z axis: slot 0 = Hx (D_z Ey), slot 1 = Hy (D_z Ex)
-            cpml_step(pm.psiH[2][0], zb + zs[q], pz0[q], bz[q], cz[q], dzEy);
-            cpml_step(pm.psiH[2][1], zb + zs[q], pz1[q], bz[q], cz[q], dzEx);
-          }
-          if (GX && xsl >= 0) {  // x axis: slot 0 = Hy (D_x Ez), slot 1 = Hz (D_x Ey)
-            const unsigned qx = psi_base_x(g, pm, xsl, j, k) + q;
-            cpml_apply(pm.psiH[0][0], qx, pm.bH[0][i], pm.cH[0][i], dxEz);
-            cpml_apply(pm.psiH[0][1], qx, pm.bH[0][i], pm.cH[0][i], dxEy);
-          }
-          if (GY && ysl >= 0) {  // y axis: slot 0 = Hz (D_y Ex), slot 1 = Hx (D_y Ez)
-            cpml_step(pm.psiH[1][0], yb + q, py0[q], by, cy, dyEx);
-            cpml_step(pm.psiH[1][1], yb + q, py1[q], by, cy, dyEz);
-          }
-          nx_[q] = hx0 - dt * (dyEz - dzEy);
-          ny_[q] = hy0 - dt * (dzEx - dxEz);
-          nz_[q] = hz0 - dt * (dxEy - dyEx);
-        }
-      }
-      const long long qq = plane_base<GX>(g, i) + own;
-      if constexpr (XZ) {
-        if (xtile) {  // new H of zone cells to the FP32 copy
-#pragma unroll
-          for (int q = 0; q < V; q++) {
-            const int xq = exact_idx(xz, i, j, k + q);
-            if (xq >= 0) {
-              xz.f[3][xq] = nx_[q];
-              xz.f[4][xq] = ny_[q];
-              xz.f[5][xq] = nz_[q];
-            }
-          }
-        }
-      }
-      if constexpr (V == 2) {
-        stv2(Hx, qq, nx_, sc.sh[0]);
-        stv2(Hy, qq, ny_, sc.sh[1]);
-        stv2(Hz, qq, nz_, sc.sh[2]);
-      } else {
-        stv(Hx, qq, nx_, sc.sh[0]);
-        stv(Hy, qq, ny_, sc.sh[1]);
-        stv(Hz, qq, nz_, sc.sh[2]);
-      }
-    }
-  };
-  int i = t.i0;
-  for (; i + PF - 1 < t.i1; i += PF) {
-#pragma unroll
-    for (int u = 0; u < PF; u++) step(i + u, S[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < PF - 1; u++)
-    if (i + u < t.i1) step(i + u, S[u]);
-}
-
 // ============================================================ ADE cells
 // Dispersive / gyrotropic cells: countDisp (dispersion.cpp:85-99) and the
 // magnetised-plasma current, from the curl H the E sweep stored.
@@ -982,384 +427,6 @@ __global__ __launch_bounds__(256) void k_tfsf_table(Tfsf tf, double* out, long l
   out[idx] = tf.amp * f0;
 }
 
-// ================================================================ E sweep
-// Operands of one plane, loaded PF planes ahead: the Hx tile words of
-// plane p (own, y-halo row) and the Hx z-halo value, the E read-modify-write
-// words and class bytes of plane p, and the Hy / Hz tile values of plane p+2
-// (the x stencil of E reaches two planes ahead).
-template <typename P, typename T, typename CL> struct PreE {
-  P hx, hxy, hy, hz, hzy, ex, ey, ez;
-  T hxz, hyz;
-  CL cls;
-};
-template <int V> struct ClsWord;
-template <> struct ClsWord<1> { using T = uint8_t; };
-template <> struct ClsWord<2> { using T = unsigned short; };
-
-// MAT: the grid may hold dispersive / gyrotropic cells or a design box; the
-// variants without (MAT false) carry none of their branches and pointers.
-template <int STORE, int GEN, int V, bool SP = false, int ROWS = 8, bool XZ = false, bool TF = false, bool MAT = true,
-          bool W = false>
-__global__ __launch_bounds__(BZ* ROWS, 4) void k_update_e(Grid g, Fields<STORE> f, Scales sc, Cpml pm, Materials mt,
-                                                         Ade ade, MarchSet ms, const float* fold) {
-  using T = typename Raw<STORE>::T;
-  using P = typename Vec<STORE, V>::P;
-  using CL = typename ClsWord<V>::T;
-  constexpr bool GX = GEN & 1, GY = GEN & 2;
-  constexpr bool DES = MAT && V == 1;  // design-box support (its launches use one cell per lane)
-  constexpr int BZV = BZ * V, LZ = BZV + 3, MBY = ROWS;
-  __shared__ ClassEntry tbl[kMaxClasses];
-  __shared__ float sHx[2][MBY + 3][LZ];  // [row j-j0+1][col k-k0+1], plane i
-  __shared__ float rHy[5][MBY][LZ];      // [row j-j0][col k-k0+1], ring of planes
-  __shared__ float rHz[5][MBY + 3][BZV]; // [row j-j0+1][col k-k0], ring of planes
-  __shared__ float sEo[3][MBY][BZV];     // this thread's E operands of plane i
-  __shared__ uint8_t sCl[MBY][BZV];      // and its class bytes
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  for (int q = tx + ty * BZ; q < mt.nclass; q += BZ * MBY) tbl[q] = mt.table[q];
-  MarchTile t;
-  if (!march_locate(ms, t)) return;  // block-uniform
-  const Region& R = ms.r[t.r];
-  const int j = t.j0 + ty, k = t.k0 + V * tx;
-  const int c0 = V * tx;
-  const bool inreg = j < R.j1 && k < R.k1;
-  const long long own = plane_off(g, j, k);
-  // halo rows j0-1, j0+MBY, j0+MBY+1 (waves ty<3); columns k0-1, k0+BZV, k0+BZV+1 (lanes tx<3)
-  const bool yw = ty < 3, zl = tx < 3;
-  const int yrow = ty == 0 ? 0 : MBY + ty;
-  const long long yh = yw ? plane_off(g, t.j0 + (ty == 0 ? -1 : MBY + ty - 1), k) : -1;
-  const int zcol = tx == 0 ? 0 : BZV + tx;
-  const long long zh = zl ? plane_off(g, j, t.k0 + (tx == 0 ? -1 : BZV + tx - 1)) : -1;
-  const T* Hx = f.H[0];
-  const T* Hy = f.H[1];
-  const T* Hz = f.H[2];
-  T* Ex = f.E[0];
-  T* Ey = f.E[1];
-  T* Ez = f.E[2];
-  const float ihx = sc.ih[0], ihy = sc.ih[1], ihz = sc.ih[2];
-  const float iex = sc.ie[0], iey = sc.ie[1], iez = sc.ie[2];
-  using Ix = typename IxT<W>::T;
-  const Ix zi = W ? (Ix)g.zidxw : (Ix)g.zidx;  // zero pad index
-
-  const long long eq = inreg ? own : -1;  // E operands: owned cells only
-  // FP32 zone (FP16 storage), as in the H sweep
-  static_assert(!XZ || STORE == 1, "the FP32 zone applies to FP16 storage");
-  const Exact& xz = sc.xz;
-  bool xtile = false;
-  if constexpr (XZ)
-    xtile = xz.on && (g.per[1] || g.per[2] ||
-                      (xz.j0 < t.j0 + MBY + 3 && xz.j1 > t.j0 - 3 && xz.k0 < t.k0 + BZV + 3 && xz.k1 > t.k0 - 3));
-  const int jo = j;
-  const int jy = yw ? nbr(t.j0 + (ty == 0 ? -1 : MBY + ty - 1), 0, g.ny, g.per[1]) : -1;
-  const int kz = zl ? nbr(t.k0 + (tx == 0 ? -1 : BZV + tx - 1), 0, g.nz, g.per[2]) : -1;
-  auto ov = [&](float& dst, int comp, int pi, int pj, int pk) {
-    // rows and lanes past the grid's edge hold the wrapped cells on a
-    // periodic axis (plane_off), nothing otherwise
-    pj = nbr(pj, 0, g.ny, g.per[1]);
-    pk = nbr(pk, 0, g.nz, g.per[2]);
-    const int xq = (pi < 0 || pj < 0 || pk < 0) ? -1 : exact_idx(xz, pi, pj, pk);
-    if (xq >= 0) dst = xz.f[comp][xq];
-  };
-  // with no class array every cell is class 0: read the zero page
-  const uint8_t* clsp = mt.cls ? mt.cls : static_cast<const uint8_t*>(g.zero);
-  const long long cq = mt.cls ? eq : 0;
-  const Ix czidx = mt.cls ? zi : (Ix)0;
-  auto fetch = [&](PreE<P, T, CL>& S, int p) {
-    const long long pb = plane_base<GX>(g, p);
-    const long long pn = plane_base<GX>(g, p + 2);
-    S.hx = ldv<P>(Hx, pb, own, zi);
-    S.hy = ldv<P>(Hy, pn, own, zi);
-    S.hz = ldv<P>(Hz, pn, own, zi);
-    S.hxy = ldv<P>(Hx, pb, yh, zi);
-    S.hzy = ldv<P>(Hz, pn, yh, zi);
-    S.hxz = *at(Hx, pb, zh, zi);
-    S.hyz = *at(Hy, pn, zh, zi);
-    S.ex = ldv<P>((const T*)Ex, pb, eq, zi);
-    S.ey = ldv<P>((const T*)Ey, pb, eq, zi);
-    S.ez = ldv<P>((const T*)Ez, pb, eq, zi);
-    // planes without a class other than 0 read the class array's zero pad
-    // (one cached line) instead of a byte per cell
-    const int pw = GX ? nbr(p, 0, g.nx, g.per[0]) : p;
-    S.cls = ldv<CL>(clsp, mt.cls ? (pw >= mt.cx0 && pw < mt.cx1 ? pb : -1) : 0, cq, czidx);
-  };
-  auto ring_direct = [&](int p) {  // Hy / Hz tile of plane p into its slot
-    const long long pb = plane_base<GX>(g, p);
-    const int s = ring5(p);
-    float v[V];
-    unpackv(ldv<P>(Hy, pb, own, zi), ihy, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rHy[s][ty][c0 + q + 1] = v[q];
-    unpackv(ldv<P>(Hz, pb, own, zi), ihz, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rHz[s][ty + 1][c0 + q] = v[q];
-    if (yw) {
-      unpackv(ldv<P>(Hz, pb, yh, zi), ihz, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) rHz[s][yrow][c0 + q] = v[q];
-    }
-    if (zl) rHy[s][ty][zcol] = cvt(ldr(Hy, pb, zh), ihy);
-    if constexpr (XZ) {
-      if (xtile) {
-        const int pp = GX ? nbr(p, 0, g.nx, g.per[0]) : p;
-#pragma unroll
-        for (int q = 0; q < V; q++) {
-          ov(rHy[s][ty][c0 + q + 1], 4, pp, jo, k + q);
-          ov(rHz[s][ty + 1][c0 + q], 5, pp, jo, k + q);
-          if (yw) ov(rHz[s][yrow][c0 + q], 5, pp, jy, k + q);
-        }
-        if (zl) ov(rHy[s][ty][zcol], 4, pp, jo, kz);
-      }
-    }
-  };
-
-  const int ysl = (GY && pm.on) ? slab_index(j, g.ny, pm.plo[1], pm.phi[1]) : -1;
-  bool design_col[V];
-  int zs[V];
-  float bz[V], cz[V];
-#pragma unroll
-  for (int q = 0; q < V; q++) {
-    design_col[q] = DES && mt.d_on && j >= mt.d_j0 && j < mt.d_j0 + mt.d_nj && k + q >= mt.d_k0 &&
-                    k + q < mt.d_k0 + mt.d_nk;
-    zs[q] = pm.on ? slab_index(k + q, g.nz, pm.plo[2], pm.phi[2]) : -1;
-    bz[q] = zs[q] >= 0 ? pm.bE[2][k + q] : 0.f;
-    cz[q] = zs[q] >= 0 ? pm.cE[2][k + q] : 0.f;
-  }
-  const float rd0 = g.rd[0], rd1 = g.rd[1], rd2 = g.rd[2], dt = g.dt;
-  const float by = ysl >= 0 ? pm.bE[1][j] : 0.f, cy = ysl >= 0 ? pm.cE[1][j] : 0.f;
-  // TF/SF fold: this lane's packed weights (zero away from the y and z faces)
-  int tfw[V];
-#pragma unroll
-  for (int q = 0; q < V; q++) tfw[q] = 0;
-  if constexpr (TF) {
-    const int* hd = reinterpret_cast<const int*>(fold);
-#pragma unroll
-    for (int q = 0; q < V; q++) tfw[q] = fold_pack(1, j, k + q, hd);
-  }
-
-  // prefetch depth, as in the H sweep; the paired variant with the folded
-  // plane wave keeps one set (two spill 30 VGPRs; one set measured 5% faster)
-  constexpr int PF = (V == 2 && TF) ? 1 : ((GY || V == 2) ? 2 : 3);
-  PreE<P, T, CL> S[PF];
-#pragma unroll
-  for (int u = 0; u < PF; u++) {
-    S[u].hx = S[u].hxy = S[u].hy = S[u].hz = S[u].hzy = S[u].ex = S[u].ey = S[u].ez = pzero<P>();
-    S[u].hxz = S[u].hyz = rzero<T>();
-    S[u].cls = 0;
-  }
-  ring_direct(t.i0 - 1);
-  ring_direct(t.i0);
-  ring_direct(t.i0 + 1);
-#pragma unroll
-  for (int u = 0; u < PF; u++) fetch(S[u], min(t.i0 + u, t.i1 - 1));  // unconditional, as in the H sweep
-
-  auto step = [&](int i, PreE<P, T, CL>& Q) {
-    const int b = i & 1;
-    const int s0 = ring5(i - 1), s1 = ring5(i), s2 = ring5(i + 1), s3 = ring5(i + 2);
-    // publish plane i (Hx) and plane i+2 (Hy, Hz); E operands to the own slots
-    float v[V];
-    unpackv(Q.hx, ihx, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sHx[b][ty + 1][c0 + q + 1] = v[q];
-    unpackv(Q.hy, ihy, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rHy[s3][ty][c0 + q + 1] = v[q];
-    unpackv(Q.hz, ihz, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) rHz[s3][ty + 1][c0 + q] = v[q];
-    if (yw) {
-      unpackv(Q.hxy, ihx, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) sHx[b][yrow][c0 + q + 1] = v[q];
-      unpackv(Q.hzy, ihz, v);
-#pragma unroll
-      for (int q = 0; q < V; q++) rHz[s3][yrow][c0 + q] = v[q];
-    }
-    if (zl) {
-      sHx[b][ty + 1][zcol] = cvt(Q.hxz, ihx);
-      rHy[s3][ty][zcol] = cvt(Q.hyz, ihy);
-    }
-    unpackv(Q.ex, iex, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sEo[0][ty][c0 + q] = v[q];
-    unpackv(Q.ey, iey, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sEo[1][ty][c0 + q] = v[q];
-    unpackv(Q.ez, iez, v);
-#pragma unroll
-    for (int q = 0; q < V; q++) sEo[2][ty][c0 + q] = v[q];
-#pragma unroll
-    for (int q = 0; q < V; q++) sCl[ty][c0 + q] = (uint8_t)(Q.cls >> (8 * q));
-    if constexpr (XZ) {
-      if (xtile && (g.per[0] || (i + 2 >= xz.i0 && i < xz.i1))) {  // Hx and own E of plane i, Hy / Hz of i+2
-        const int ii = GX ? nbr(i, 0, g.nx, g.per[0]) : i;
-        const int i2n = GX ? nbr(i + 2, 0, g.nx, g.per[0]) : i + 2;
-#pragma unroll
-        for (int q = 0; q < V; q++) {
-          ov(sHx[b][ty + 1][c0 + q + 1], 3, ii, jo, k + q);
-          ov(rHy[s3][ty][c0 + q + 1], 4, i2n, jo, k + q);
-          ov(rHz[s3][ty + 1][c0 + q], 5, i2n, jo, k + q);
-          ov(sEo[0][ty][c0 + q], 0, ii, jo, k + q);
-          ov(sEo[1][ty][c0 + q], 1, ii, jo, k + q);
-          ov(sEo[2][ty][c0 + q], 2, ii, jo, k + q);
-          if (yw) {
-            ov(sHx[b][yrow][c0 + q + 1], 3, ii, jy, k + q);
-            ov(rHz[s3][yrow][c0 + q], 5, i2n, jy, k + q);
-          }
-        }
-        if (zl) {
-          ov(sHx[b][ty + 1][zcol], 3, ii, jo, kz);
-          ov(rHy[s3][ty][zcol], 4, i2n, jo, kz);
-        }
-      }
-    }
-    // psi and design-box operands of plane i before the prefetch
-    float pz0[V], pz1[V], py0[V], py1[V], dv[V];
-    bool over[V];
-    const unsigned zb = psi_base_z(g, pm, i, j), yb = psi_base_y(g, pm, ysl, i, k);
-#pragma unroll
-    for (int q = 0; q < V; q++) {
-      pz0[q] = pz1[q] = py0[q] = py1[q] = dv[q] = 0.f;
-      if (!SP && inreg && zs[q] >= 0) {
-        pz0[q] = pm.psiE[2][0][zb + zs[q]];
-        pz1[q] = pm.psiE[2][1][zb + zs[q]];
-      }
-      if (!SP && GY && inreg && ysl >= 0) {
-        py0[q] = pm.psiE[1][0][yb + q];
-        py1[q] = pm.psiE[1][1][yb + q];
-      }
-      over[q] = DES && inreg && design_col[q] && i >= mt.d_i0 && i < mt.d_i0 + mt.d_ni;
-      if (DES && over[q])
-        dv[q] = mt.d_inv_eps[((long long)(i - mt.d_i0) * mt.d_nj + (j - mt.d_j0)) * mt.d_nk + (k + q - mt.d_k0)];
-    }
-    const int xsl = (GX && pm.on) ? slab_index(i, g.nx, pm.plo[0], pm.phi[0]) : -1;
-    // this plane's fold factors, loaded before the barrier (whose wait covers
-    // them) rather than inside the band branch
-    float fu[6];
-#pragma unroll
-    for (int t6 = 0; t6 < 6; t6++) fu[t6] = 0.f;
-    if constexpr (TF) {
-#pragma unroll
-      for (int t6 = 0; t6 < 6; t6++) fu[t6] = fold[kFoldStride * (1 + i) + t6];
-    }
-    fetch(Q, min(i + PF, t.i1 - 1));
-    lds_barrier();
-    if (inreg) {
-      float nE[3][V];
-      bool plain = true;
-#pragma unroll
-      for (int q = 0; q < V; q++) {
-        const int c = c0 + q;
-        const float ex0 = sEo[0][ty][c], ey0 = sEo[1][ty][c], ez0 = sEo[2][ty][c];
-        const int cls = sCl[ty][c];
-        const float hxo = sHx[b][ty + 1][c + 1];
-        float dyHz = rd1 * d24(rHz[s1][ty][c], rHz[s1][ty + 1][c], rHz[s1][ty + 2][c], rHz[s1][ty + 3][c]);
-        float dyHx = rd1 * d24(sHx[b][ty][c + 1], hxo, sHx[b][ty + 2][c + 1], sHx[b][ty + 3][c + 1]);
-        float dzHy = rd2 * d24(rHy[s1][ty][c], rHy[s1][ty][c + 1], rHy[s1][ty][c + 2], rHy[s1][ty][c + 3]);
-        float dzHx = rd2 * d24(sHx[b][ty + 1][c], hxo, sHx[b][ty + 1][c + 2], sHx[b][ty + 1][c + 3]);
-        float dxHz = rd0 * d24(rHz[s0][ty + 1][c], rHz[s1][ty + 1][c], rHz[s2][ty + 1][c], rHz[s3][ty + 1][c]);
-        float dxHy = rd0 * d24(rHy[s0][ty][c + 1], rHy[s1][ty][c + 1], rHy[s2][ty][c + 1], rHy[s3][ty][c + 1]);
-        if constexpr (TF) {
-          if (tfw[q]) {
-            const int w = tfw[q];
-            dyHz += fold_f(w, 0) * fu[0];   // Ex, y faces
-            dzHy += fold_f(w, 6) * fu[1];   // Ex, z faces
-            dzHx += fold_f(w, 12) * fu[2];  // Ey, z faces
-            dxHz += fold_b(w, 24) * fu[3];  // Ey, x faces
-            dxHy += fold_b(w, 25) * fu[4];  // Ez, x faces
-            dyHx += fold_f(w, 18) * fu[5];  // Ez, y faces
-          }
-        }
-        if (!SP && zs[q] >= 0) {  // z axis: slot 0 = Ex (D_z Hy), slot 1 = Ey (D_z Hx)
-          cpml_step(pm.psiE[2][0], zb + zs[q], pz0[q], bz[q], cz[q], dzHy);
-          cpml_step(pm.psiE[2][1], zb + zs[q], pz1[q], bz[q], cz[q], dzHx);
-        }
-        if (!SP && GX && xsl >= 0) {  // x axis: slot 0 = Ey (D_x Hz), slot 1 = Ez (D_x Hy)
-          const unsigned qx = psi_base_x(g, pm, xsl, j, k) + q;
-          cpml_apply(pm.psiE[0][0], qx, pm.bE[0][i], pm.cE[0][i], dxHz);
-          cpml_apply(pm.psiE[0][1], qx, pm.bE[0][i], pm.cE[0][i], dxHy);
-        }
-        if (!SP && GY && ysl >= 0) {  // y axis: slot 0 = Ez (D_y Hx), slot 1 = Ex (D_y Hz)
-          cpml_step(pm.psiE[1][0], yb + q, py0[q], by, cy, dyHx);
-          cpml_step(pm.psiE[1][1], yb + q, py1[q], by, cy, dyHz);
-        }
-        const float crx = dyHz - dzHy, cry = dzHx - dxHz, crz = dxHy - dyHx;
-        const ClassEntry& ce = tbl[cls];
-        float ie0 = ce.inv_eps[0], ie1 = ce.inv_eps[1], ie2 = ce.inv_eps[2];
-        if (over[q]) ie0 = ie1 = ie2 = dv[q];
-        if (MAT && ce.special && !over[q]) {  // finished by k_ade; its E word keeps the old value here
-          const long long bq =
-              (long long)(i - ade.i0) * ade.bsx + (long long)(j - ade.j0) * ade.bsy + (k + q - ade.k0);
-          ade.curl[0][bq] = crx;
-          ade.curl[1][bq] = cry;
-          ade.curl[2][bq] = crz;
-          nE[0][q] = ex0;
-          nE[1][q] = ey0;
-          nE[2][q] = ez0;
-          plain = false;
-        } else if constexpr (SP) {
-          // split parts: Ex (y, z), Ey (z, x), Ez (x, y); dispersive cells never sit in the layer
-          const bool sx = GX && xsl >= 0;
-          const float k1x = sx ? pm.bE[0][i] : 1.f, k2x = sx ? pm.cE[0][i] : 1.f;
-          const float k1y = (GY && ysl >= 0) ? by : 1.f, k2y = (GY && ysl >= 0) ? cy : 1.f;
-          const float k1z = zs[q] >= 0 ? bz[q] : 1.f, k2z = zs[q] >= 0 ? cz[q] : 1.f;
-          const long long qs = plane_base<GX>(g, i) + own + q;
-          nE[0][q] = split_step(pm.p2E[0], qs, ex0, k1y, k2y, dt * ie0 * dyHz, k1z, k2z, -dt * ie0 * dzHy);
-          nE[1][q] = split_step(pm.p2E[1], qs, ey0, k1z, k2z, dt * ie1 * dzHx, k1x, k2x, -dt * ie1 * dxHz);
-          nE[2][q] = split_step(pm.p2E[2], qs, ez0, k1x, k2x, dt * ie2 * dxHy, k1y, k2y, -dt * ie2 * dyHx);
-        } else {
-          nE[0][q] = ex0 + dt * ie0 * crx;
-          nE[1][q] = ey0 + dt * ie1 * cry;
-          nE[2][q] = ez0 + dt * ie2 * crz;
-        }
-      }
-      const long long qq = plane_base<GX>(g, i) + own;
-      if constexpr (XZ) {
-        if (xtile) {  // new E of zone cells to the FP32 copy (a dispersive cell keeps its old value for k_ade)
-#pragma unroll
-          for (int q = 0; q < V; q++) {
-            const int xq = exact_idx(xz, i, j, k + q);
-            if (xq >= 0) {
-              xz.f[0][xq] = nE[0][q];
-              xz.f[1][xq] = nE[1][q];
-              xz.f[2][xq] = nE[2][q];
-            }
-          }
-        }
-      }
-      if constexpr (V == 2) {
-        // a pair with a dispersive cell stores only its plain cells: k_ade
-        // writes the other one (from the old value it reads)
-        if (plain) {
-          stv2(Ex, qq, nE[0], sc.se[0]);
-          stv2(Ey, qq, nE[1], sc.se[1]);
-          stv2(Ez, qq, nE[2], sc.se[2]);
-        } else {
-#pragma unroll
-          for (int q = 0; q < V; q++) {
-            if (tbl[sCl[ty][c0 + q]].special && !over[q]) continue;
-            stv(Ex + q, qq, &nE[0][q], sc.se[0]);
-            stv(Ey + q, qq, &nE[1][q], sc.se[1]);
-            stv(Ez + q, qq, &nE[2][q], sc.se[2]);
-          }
-        }
-      } else {
-        if (plain) {
-          stv(Ex, qq, nE[0], sc.se[0]);
-          stv(Ey, qq, nE[1], sc.se[1]);
-          stv(Ez, qq, nE[2], sc.se[2]);
-        }
-      }
-    }
-  };
-  int i = t.i0;
-  for (; i + PF - 1 < t.i1; i += PF) {
-#pragma unroll
-    for (int u = 0; u < PF; u++) step(i + u, S[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < PF - 1; u++)
-    if (i + u < t.i1) step(i + u, S[u]);
-}
-
 // ======================================================== small kernels
 template <int STORE>
 __global__ void k_soft(Fields<STORE> f, Scales sc, Soft so) {
@@ -1459,289 +526,6 @@ int take_launch_error(char* msg, int cap) {
 }
 
 static void check_launch(const char* what) { note_launch(what); }
-
-// Blocks of one launch that fit on the device at once.
-template <typename K>
-static int resident_blocks(K kernel, int threads) {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    hipDeviceProp_t p;
-    if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&p, dev) != hipSuccess) return 512;
-    cus = p.multiProcessorCount;
-  }
-  int per = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per < 1) per = 1;
-  return per * cus;
-}
-
-// Segment length along x: a block marches seg planes after a warm-up of
-// about kWarm planes (three ring planes loaded synchronously, then the
-// two-plane prefetch filling), and the launch runs in ceil(blocks / slots)
-// rounds.  Minimise rounds * (seg + kWarm); *cost receives the minimum.
-static int march_seg(const Region* regs, int nreg, int slots, int bz, int by, long long* cost_out = nullptr) {
-  constexpr int kWarm = 6;
-  int maxlen = 1;
-  for (int t = 0; t < nreg; t++) {
-    const Region& r = regs[t];
-    if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) continue;
-    maxlen = std::max(maxlen, r.i1 - r.i0);
-  }
-  int best = maxlen;
-  long long best_cost = -1;
-  for (int nseg = 1; nseg <= maxlen; nseg++) {
-    const int seg = (maxlen + nseg - 1) / nseg;
-    if (nseg > 1 && seg == (maxlen + nseg - 2) / (nseg - 1)) continue;  // same seg as nseg-1
-    long long blocks = 0;
-    for (int t = 0; t < nreg; t++) {
-      const Region& r = regs[t];
-      if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) continue;
-      blocks += (long long)((r.k1 - r.k0 + bz - 1) / bz) * ((r.j1 - r.j0 + by - 1) / by) *
-                ((r.i1 - r.i0 + seg - 1) / seg);
-    }
-    const long long rounds = (blocks + slots - 1) / slots;
-    const long long cost = rounds * (seg + kWarm);
-    if (best_cost < 0 || cost < best_cost) {
-      best_cost = cost;
-      best = seg;
-    }
-    if (seg <= 4) break;
-  }
-  if (cost_out) *cost_out = best_cost;
-  return best;
-}
-
-// Tile height of a one-cell-per-lane sweep: 16 rows (one 1024-lane block per
-// CU) unless the 8-row launch (two blocks per CU) has a lower march cost.  A
-// block of either height keeps its CU equally busy per plane, so the costs
-// compare directly.
-static bool use_16_rows(int slots8, int slots16, const Region* regs, int nreg, int bz, int& seg8, int& seg16) {
-  long long c8 = 0, c16 = 0;
-  seg8 = march_seg(regs, nreg, slots8, bz, 8, &c8);
-  seg16 = march_seg(regs, nreg, slots16, bz, 16, &c16);
-  return c16 <= c8;
-}
-
-template <int STORE, int V, bool SP, bool XZ, bool TF, bool W = false>
-static void upd_h(const Grid& g, const void* fields, const Scales& sc, const Cpml& pm, const Region* regs, int nreg,
-                  const float* fold, hipStream_t st) {
-  const Fields<STORE>& f = *static_cast<const Fields<STORE>*>(fields);
-  int seg8 = 0, seg16 = 0;
-  if constexpr (V == 1) {
-    static const int slots8 = resident_blocks(k_update_h<STORE, 3, V, SP, 8, XZ, TF, W>, BZ * 8);
-    static const int slots16 = resident_blocks(k_update_h<STORE, 3, V, SP, 16, XZ, TF, W>, BZ * 16);
-    if (use_16_rows(slots8, slots16, regs, nreg, BZ, seg8, seg16)) {
-      MarchSet rg = make_march(regs, nreg, seg16, BZ, 16);
-      if (rg.total <= 0) return;
-      hipLaunchKernelGGL((k_update_h<STORE, 3, V, SP, 16, XZ, TF, W>), dim3(rg.per * NXCD), dim3(BZ, 16, 1), 0, st, g, f,
-                         sc, pm, rg, fold);
-      check_launch("k_update_h");
-      return;
-    }
-  } else {
-    static const int slots = resident_blocks(k_update_h<STORE, 3, V, SP, 8, XZ, TF, W>, BZ * 8);
-    seg8 = march_seg(regs, nreg, slots, BZ * V, 8);
-  }
-  MarchSet rg = make_march(regs, nreg, seg8, BZ * V, 8);
-  if (rg.total <= 0) return;
-  hipLaunchKernelGGL((k_update_h<STORE, 3, V, SP, 8, XZ, TF, W>), dim3(rg.per * NXCD), dim3(BZ, 8, 1), 0, st, g, f, sc, pm,
-                     rg, fold);
-  check_launch("k_update_h");
-}
-
-template <int STORE, int V, bool SP, bool XZ, bool TF, bool MAT = true, bool W = false>
-static void upd_e(const Grid& g, const void* fields, const Scales& sc, const Cpml& pm, const Materials& mt,
-                  const Ade& ade, const Region* regs, int nreg, const float* fold, hipStream_t st) {
-  const Fields<STORE>& f = *static_cast<const Fields<STORE>*>(fields);
-  int seg8 = 0, seg16 = 0;
-  if constexpr (V == 1) {
-    static const int slots8 = resident_blocks(k_update_e<STORE, 3, V, SP, 8, XZ, TF, MAT, W>, BZ * 8);
-    static const int slots16 = resident_blocks(k_update_e<STORE, 3, V, SP, 16, XZ, TF, MAT, W>, BZ * 16);
-    if (use_16_rows(slots8, slots16, regs, nreg, BZ, seg8, seg16)) {
-      MarchSet rg = make_march(regs, nreg, seg16, BZ, 16);
-      if (rg.total <= 0) return;
-      hipLaunchKernelGGL((k_update_e<STORE, 3, V, SP, 16, XZ, TF, MAT, W>), dim3(rg.per * NXCD), dim3(BZ, 16, 1), 0, st, g,
-                         f, sc, pm, mt, ade, rg, fold);
-      check_launch("k_update_e");
-      return;
-    }
-  } else {
-    static const int slots = resident_blocks(k_update_e<STORE, 3, V, SP, 8, XZ, TF, MAT, W>, BZ * 8);
-    seg8 = march_seg(regs, nreg, slots, BZ * V, 8);
-  }
-  MarchSet rg = make_march(regs, nreg, seg8, BZ * V, 8);
-  if (rg.total <= 0) return;
-  hipLaunchKernelGGL((k_update_e<STORE, 3, V, SP, 8, XZ, TF, MAT, W>), dim3(rg.per * NXCD), dim3(BZ, 8, 1), 0, st, g, f, sc,
-                     pm, mt, ade, rg, fold);
-  check_launch("k_update_e");
-}
-
-// FP16 storage on an even nz runs two z cells per lane (__half2 words);
-// a design box (FP32 inverse design) keeps one cell per lane.
-static bool pair_cells(int store, const Grid& g, const Materials* mt) {
-  return store == 1 && g.nz % 2 == 0 && !(mt && mt->d_on);
-}
-// pairs start at an even k: every region must too (the __half2 words)
-static bool even_k(const Region* regs, int nreg) {
-  for (int r = 0; r < nreg; r++)
-    if (regs[r].k0 & 1) return false;
-  return true;
-}
-
-// The sweep variant of a configuration: storage, cells per lane, layer
-// kind, FP32 zone (its own variants, so that the other variants carry none of
-// its registers) and a folded plane wave along x (never with the zone).
-template <bool TF>
-static void update_h_go(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                        const Region* regs, int nreg, const float* fold, hipStream_t st) {
-  const bool xz = store == 1 && sc.xz.on;
-  const bool pairs = pair_cells(store, g, nullptr) && even_k(regs, nreg);
-  if (wide_grid(g)) {  // 64-bit cell indices (no split layer or zone there: dtm_create refuses them)
-    if (store == 0) upd_h<0, 1, false, false, TF, true>(g, fields, sc, pm, regs, nreg, fold, st);
-    else if (pairs) upd_h<1, 2, false, false, TF, true>(g, fields, sc, pm, regs, nreg, fold, st);
-    else upd_h<1, 1, false, false, TF, true>(g, fields, sc, pm, regs, nreg, fold, st);
-    return;
-  }
-  if (pm.split) {  // split-field layer: one cell per lane
-    if (store == 0) upd_h<0, 1, true, false, TF>(g, fields, sc, pm, regs, nreg, fold, st);
-    else if (xz) upd_h<1, 1, true, true, false>(g, fields, sc, pm, regs, nreg, fold, st);
-    else upd_h<1, 1, true, false, TF>(g, fields, sc, pm, regs, nreg, fold, st);
-  } else if (store == 0) {
-    upd_h<0, 1, false, false, TF>(g, fields, sc, pm, regs, nreg, fold, st);
-  } else if (xz) {
-    if (pairs) upd_h<1, 2, false, true, false>(g, fields, sc, pm, regs, nreg, fold, st);
-    else upd_h<1, 1, false, true, false>(g, fields, sc, pm, regs, nreg, fold, st);
-  } else if (pairs) {
-    upd_h<1, 2, false, false, TF>(g, fields, sc, pm, regs, nreg, fold, st);
-  } else {
-    upd_h<1, 1, false, false, TF>(g, fields, sc, pm, regs, nreg, fold, st);
-  }
-}
-
-template <bool TF>
-static void update_e_go(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                        const Materials& mt, const Ade& ade, const Region* regs, int nreg, const float* fold,
-                        hipStream_t st) {
-  const bool xz = store == 1 && sc.xz.on;
-  const bool pairs = pair_cells(store, g, &mt) && even_k(regs, nreg);
-  const bool mat = ade.on || mt.d_on;  // else the variants without the dispersive / design branches
-  if (wide_grid(g)) {  // 64-bit cell indices, the material branches kept
-    if (store == 0) upd_e<0, 1, false, false, TF, true, true>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else if (pairs) upd_e<1, 2, false, false, TF, true, true>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<1, 1, false, false, TF, true, true>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    return;
-  }
-  if (pm.split) {
-    if (store == 0) upd_e<0, 1, true, false, TF>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else if (xz) upd_e<1, 1, true, true, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<1, 1, true, false, TF>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  } else if (store == 0) {
-    if (mat) upd_e<0, 1, false, false, TF>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<0, 1, false, false, TF, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  } else if (xz) {
-    if (pairs) upd_e<1, 2, false, true, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<1, 1, false, true, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  } else if (pairs) {
-    if (mat) upd_e<1, 2, false, false, TF>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<1, 2, false, false, TF, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  } else {
-    if (mat) upd_e<1, 1, false, false, TF>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-    else upd_e<1, 1, false, false, TF, false>(g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  }
-}
-
-// With an FP32 zone only a column of cells (the zone's y and z range plus
-// the 3 cells its stencils reach, widened to the tile grid, every x plane)
-// runs the zone variants; the rest of the grid runs the plain ones as up to
-// four boxes around it (y slabs, then z slabs inside the column's y range),
-// all of full x extent, so every launch keeps the long x segments of the
-// whole grid.  Both launches of a sweep write disjoint cells and read only
-// the other family of fields, so their order does not matter and they may
-// run concurrently.  A periodic axis keeps the column at its full extent on
-// that axis.
-static bool zone_split(const Grid& g, const Exact& x, const Region* regs, int nreg, Region* outer, int& nouter,
-                       Region& mid) {
-  if (nreg != 1) return false;
-  const Region& R = regs[0];
-  int j0 = g.per[1] ? R.j0 : max(R.j0, x.j0 - 3), j1 = g.per[1] ? R.j1 : min(R.j1, x.j1 + 3);
-  int k0 = g.per[2] ? R.k0 : max(R.k0, x.k0 - 3), k1 = g.per[2] ? R.k1 : min(R.k1, x.k1 + 3);
-  if (j0 >= j1 || k0 >= k1) return false;
-  // the column on the region's tile grid (rows in 16s, z in 128s from its
-  // origin: every tile shape of the plain launch), so the outer boxes hold
-  // whole tiles of the one-box tiling and add no partial tiles; z bounds are
-  // then even, as the paired FP16 sweeps need (two z cells per lane from an
-  // even k)
-  j0 = R.j0 + (j0 - R.j0) / 16 * 16;
-  j1 = min(R.j1, R.j0 + (j1 - R.j0 + 15) / 16 * 16);
-  k0 = R.k0 + (k0 - R.k0) / 128 * 128;
-  k1 = min(R.k1, R.k0 + (k1 - R.k0 + 127) / 128 * 128);
-  k0 &= ~1;
-  k1 = min(R.k1, (k1 + 1) & ~1);
-  nouter = 0;
-  auto add = [&](int a0, int a1, int b0, int b1) {
-    if (a0 < a1 && b0 < b1) outer[nouter++] = Region{R.i0, R.i1, a0, a1, b0, b1};
-  };
-  add(R.j0, j0, R.k0, R.k1);
-  add(j1, R.j1, R.k0, R.k1);
-  add(j0, j1, R.k0, k0);
-  add(j0, j1, k1, R.k1);
-  mid = Region{R.i0, R.i1, j0, j1, k0, k1};
-  return true;
-}
-
-// The zone's column and the outer boxes write disjoint cells and read only
-// the other family of fields: with a side stream they run concurrently.
-static void side_fork(const SideStream* side, hipStream_t st) {
-  if (!side) return;
-  hipError_t e = hipEventRecord(side->fork, st);
-  if (e == hipSuccess) e = hipStreamWaitEvent(side->st, side->fork, 0);
-  if (e != hipSuccess) fail_launch("side stream fork", hipGetErrorString(e));
-}
-static void side_join(const SideStream* side, hipStream_t st) {
-  if (!side) return;
-  hipError_t e = hipEventRecord(side->join, side->st);
-  if (e == hipSuccess) e = hipStreamWaitEvent(st, side->join, 0);
-  if (e != hipSuccess) fail_launch("side stream join", hipGetErrorString(e));
-}
-
-void launch_update_h(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                     const Region* regs, int nreg, hipStream_t st, const float* fold, const SideStream* side) {
-  Region outer[4], mid;
-  int nouter = 0;
-  if (store == 1 && sc.xz.on && zone_split(g, sc.xz, regs, nreg, outer, nouter, mid)) {
-    Scales plain = sc;
-    plain.xz.on = 0;
-    side_fork(side, st);
-    update_h_go<false>(store, g, fields, sc, pm, &mid, 1, nullptr, side ? side->st : st);
-    if (nouter) update_h_go<false>(store, g, fields, plain, pm, outer, nouter, nullptr, st);
-    side_join(side, st);
-    return;
-  }
-  if (fold && !(store == 1 && sc.xz.on))
-    update_h_go<true>(store, g, fields, sc, pm, regs, nreg, fold, st);
-  else
-    update_h_go<false>(store, g, fields, sc, pm, regs, nreg, nullptr, st);
-}
-
-void launch_update_e(int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
-                     const Materials& mt, const Ade& ade, const Region* regs, int nreg, hipStream_t st,
-                     const float* fold, const SideStream* side) {
-  Region outer[4], mid;
-  int nouter = 0;
-  if (store == 1 && sc.xz.on && zone_split(g, sc.xz, regs, nreg, outer, nouter, mid)) {
-    Scales plain = sc;
-    plain.xz.on = 0;
-    side_fork(side, st);
-    update_e_go<false>(store, g, fields, sc, pm, mt, ade, &mid, 1, nullptr, side ? side->st : st);
-    if (nouter) update_e_go<false>(store, g, fields, plain, pm, mt, ade, outer, nouter, nullptr, st);
-    side_join(side, st);
-    return;
-  }
-  if (fold && !(store == 1 && sc.xz.on))
-    update_e_go<true>(store, g, fields, sc, pm, mt, ade, regs, nreg, fold, st);
-  else
-    update_e_go<false>(store, g, fields, sc, pm, mt, ade, regs, nreg, nullptr, st);
-}
 
 // One launch over the union of the face bands (k_tfsf gives each cell one
 // writer); the host fills each band's first thread index and its overlap
@@ -1947,7 +731,7 @@ void launch_from_float(int store, const float* src, float s, void* dst, long lon
 }
 
 const char* kernel_variant_name(int store) {
-  return store == 0 ? "k_update_{h,e}<fp32>" : "k_update_{h,e}<fp16>";
+  return store == 0 ? "k_sweep<fp32>" : "k_sweep<fp16>";
 }
 
 }  // namespace dtm

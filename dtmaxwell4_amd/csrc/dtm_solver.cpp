@@ -51,7 +51,6 @@ struct dtm_solver {
   dtm_config cfg;
   int dev = 0;
   hipStream_t stream = nullptr;
-  SideStream side{};  // the FP32 zone's column runs on side.st (set with the zone)
   Grid g{};
   Scales sc{};
   int store = 0;
@@ -66,6 +65,7 @@ struct dtm_solver {
   bool torre = false; // fused single-pass step; false: two sweeps per step
   bool no_fold = false; // tabulated plane-wave TF/SF through k_tfsf instead of the sweeps
   float* fold_base = nullptr; // per-plane factors of a folded plane wave, kTableSteps x 2 half-steps
+  int2* fold_w = nullptr;     // the sweeps' weights of that source, one entry per chunk of cells and half-step
   // device copies of the fused step's pointer table, one per buffer parity
   // (the old / new buffers swap every step), and their host images
   TorreCold* cold_dev[2] = {};
@@ -141,10 +141,15 @@ static int dalloc(dtm_solver* s, T** p, size_t bytes) {
   return 0;
 }
 
-// dalloc for buffers that hold time-stepped state.
+// dalloc for buffers that hold time-stepped state.  64 bytes more are
+// allocated on either side: a lane of the sweeps reads whole chunks of cells,
+// the first or last one of an array past its ends where a slab or the z extent
+// is no multiple of a chunk.
 template <typename T>
 static int sdalloc(dtm_solver* s, T** p, size_t bytes) {
-  if (int rc = dalloc(s, p, bytes)) return rc;
+  char* base = nullptr;
+  if (int rc = dalloc(s, &base, bytes + 128)) return rc;
+  *p = reinterpret_cast<T*>(base + 64);
   s->state.emplace_back(static_cast<void*>(*p), bytes == 0 ? 16 : bytes);
   return 0;
 }
@@ -492,8 +497,11 @@ static int setup_tfsf(dtm_solver* s) {
   if (s->tf.kind != DTM_TFSF_NONE && s->tf.tab_axis >= 0) {
     if (int rc = dalloc(s, &s->tab_base, sizeof(double) * 2 * kTableSteps * s->tf.tab_n)) return rc;
     // per-plane factors of a wave along x, for the sweeps (and the fused step) that fold it in
-    if (s->tf.tab_axis == 0)
+    if (s->tf.tab_axis == 0) {
       if (int rc = dalloc(s, &s->fold_base, sizeof(float) * 2 * kTableSteps * fold_floats(s))) return rc;
+      if (int rc = dalloc(s, &s->fold_w, sizeof(int2) * (size_t)fold_weights_size(s->g))) return rc;
+      launch_fold_weights(s->tf, s->fold_w, s->g, s->stream);
+    }
   }
   return 0;
 }
@@ -963,11 +971,7 @@ void dtm_destroy(dtm_solver* s) {
     (void)hipEventDestroy(e[0]);
     (void)hipEventDestroy(e[1]);
   }
-  if (s->side.st) (void)hipStreamSynchronize(s->side.st);
   for (void* p : s->allocs) (void)hipFree(p);
-  if (s->side.fork) (void)hipEventDestroy(s->side.fork);
-  if (s->side.join) (void)hipEventDestroy(s->side.join);
-  if (s->side.st) (void)hipStreamDestroy(s->side.st);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -1182,9 +1186,8 @@ static int one_step(dtm_solver* s) {
     Tfsf tfh{};
     if (s->tf.active) tfh = tfsf_for(s, n, 0);
     ev_begin(s, 0);
-    const SideStream* side = s->sc.xz.on && s->side.st ? &s->side : nullptr;
-    launch_update_h(s->store, s->g, F, s->sc, s->pm, &s->whole, 1, s->stream, fold ? fold_for(s, n, 0) : nullptr,
-                    side);
+    launch_sweep(0, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 0) : nullptr,
+                 s->fold_w, s->stream);
     ev_end(s);
     if (s->tf.active && !fold) {
       ev_begin(s, 4);
@@ -1195,8 +1198,8 @@ static int one_step(dtm_solver* s) {
     Tfsf tfe{};
     if (s->tf.active) tfe = tfsf_for(s, n, 1);
     ev_begin(s, 2);
-    launch_update_e(s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, &s->whole, 1, s->stream,
-                    fold ? fold_for(s, n, 1) : nullptr, side);
+    launch_sweep(1, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 1) : nullptr,
+                 s->fold_w, s->stream);
     ev_end(s);
     ev_begin(s, 4);
     launch_ade(s->store, s->g, F, F, s->sc, s->mt, s->ade, s->stream);
@@ -1871,11 +1874,6 @@ int dtm_set_fp32_zone(dtm_solver* s, int i0, int i1, int j0, int j1, int k0, int
   Exact x{};
   for (int c = 0; c < 6; c++)
     if (int rc = sdalloc(s, &x.f[c], sizeof(float) * (size_t)cells)) return rc;
-  if (!s->side.st) {  // a second stream (default priority) for the zone's column
-    HIPCHK(hipStreamCreate(&s->side.st));
-    HIPCHK(hipEventCreateWithFlags(&s->side.fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&s->side.join, hipEventDisableTiming));
-  }
   x.i0 = i0;
   x.i1 = i1;
   x.j0 = j0;
