@@ -29,8 +29,8 @@ GROUPS_TWOPASS = ("H sweep", "-", "E sweep", "-", "TF/SF+ADE+sources+probes")
 GROUPS_FUSED = ("fused step", "-", "-", "-", "TF/SF+ADE+sources+probes")
 # Algorithmic bytes per cell, the roofline basis: two-pass half-step sweep:
 # read 3E+3H, write 3 components (+1 class byte for E): 36 / 37 B in FP32.
-# Fused step (H and E in one pass): read 3E+3H, write 3E+3H, read the class
-# byte: 49 B.  The CPML psi (two FP32 values read and written per half-step
+# Fused step of FP16 storage (H and E in one pass): read 3E+3H, write 3E+3H,
+# read the class byte: 25 B; in FP32 the fused schedule runs the two sweeps.  The CPML psi (two FP32 values read and written per half-step
 # for each slab a cell lies in: 16 B; 32 B per fused step) is region-local
 # and reported beside it (psi_bytes, roofline.extra_bytes), not in it.
 WORDS_PER_HALF = 9
@@ -99,7 +99,8 @@ def gpu_run(storage, sweep, steps, warmup, nx, ny, nz):
     if not np.isfinite(ez).all():
         raise RuntimeError("non-finite field after timed run")
     esz = 2 if storage else 4
-    fused = s.kernel_name.startswith("k_torre")
+    fused = bool(sweep)
+    bpc = (WORDS_FUSED * esz if s.kernel_name.startswith("k_torre") else 2 * WORDS_PER_HALF * esz) + 1
     names = GROUPS_FUSED if fused else GROUPS_TWOPASS
     pfrac = psi_cells(w.cfg) / cells  # slab memberships per cell
     groups = {}
@@ -110,7 +111,7 @@ def gpu_run(storage, sweep, steps, warmup, nx, ny, nz):
         gc = s.group_cells(g)
         # Yee bytes (the roofline basis) and the CPML psi bytes, reported apart
         if fused:
-            byts = gc * (WORDS_FUSED * esz + 1)
+            byts = gc * bpc
             psib = gc * 2 * PSI_BYTES_HALF * pfrac
         else:
             byts = gc * (WORDS_PER_HALF * esz + (1 if g in (2, 3) else 0))
@@ -120,7 +121,6 @@ def gpu_run(storage, sweep, steps, warmup, nx, ny, nz):
                                 gbs=(byts / (avg * 1e-3) / 1e9) if (gc and avg > 0) else None,
                                 gbs_with_psi=((byts + psib) / (avg * 1e-3) / 1e9) if (gc and avg > 0) else None)
     dom = max((g for g in groups if groups[g]["cells"]), key=lambda g: groups[g]["avg_ms"] * groups[g]["launches"])
-    bpc = (WORDS_FUSED * esz + 1) if fused else (2 * WORDS_PER_HALF * esz + 1)
     res = dict(gcells=val, ms=ms, wall_s=wall, groups=groups, dominant=dom, kernel=s.kernel_name,
                bytes_per_cell_update=bpc, fused=fused)
     s.close()

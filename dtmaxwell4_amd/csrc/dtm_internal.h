@@ -369,9 +369,9 @@ void launch_ade(int store, const Grid& g, const void* fields_src, const void* fi
 // fold non-null: a plane-wave TF/SF source along x added inside the step,
 // from the step's factor tables (the H half-step's, the E half-step's
 // following it at +(nx + 1) * kFoldStride).
-void launch_torre(int store, const Grid& g, const Scales& sc, const Materials& mt, const TorreCold* cold,
+void launch_torre(const Grid& g, const Scales& sc, const Materials& mt, const TorreCold* cold,
                   const Region* regs, int nreg, hipStream_t st, const float* fold = nullptr);
-TorreCold make_torre_cold(const void* fields_old, const void* fields_new, int store, const Cpml& pm_old,
+TorreCold make_torre_cold(const void* fields_old, const void* fields_new, const Cpml& pm_old,
                           const Cpml& pm_new, const Materials& mt, const Ade& ade);
 void launch_soft(int store, const Grid& g, const void* fields, const Scales& sc, const Soft& so,
                  hipStream_t st);

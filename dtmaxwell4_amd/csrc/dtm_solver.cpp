@@ -62,7 +62,12 @@ struct dtm_solver {
   Fields<1> f16{}, f16n{};
   Cpml pm{};         // current psi
   Cpml pmn{};        // second psi buffers (torre step)
-  bool torre = false; // fused single-pass step; false: two sweeps per step
+  // One kernel a step (dtm_torre.hip): the fused schedule in FP16 storage, where
+  // its E update reads H before that is rounded.  In FP32 the two in-place
+  // sweeps give the same update in less time and half the memory, so the
+  // schedule runs them (200^3: 131 us a step, that kernel's 228; 512x256x256:
+  // 572 and 614; 64^3: 17 and 29).
+  bool torre = false;
   bool no_fold = false; // tabulated plane-wave TF/SF through k_tfsf instead of the sweeps
   float* fold_base = nullptr; // per-plane factors of a folded plane wave, kTableSteps x 2 half-steps
   int2* fold_w = nullptr;     // the sweeps' weights of that source, one entry per chunk of cells and half-step
@@ -880,7 +885,7 @@ int dtm_create(const dtm_config* cfg, dtm_solver** out) {
   dtm_solver* s = new dtm_solver();
   s->cfg = c;
   s->store = c.storage;
-  s->torre = c.sweep == DTM_SWEEP_FUSED;
+  s->torre = c.sweep == DTM_SWEEP_FUSED && c.storage == DTM_STORE_FP16;
   hipError_t e = hipGetDevice(&s->dev);
   if (e != hipSuccess) {
     delete s;
@@ -1126,7 +1131,7 @@ static void ev_end(dtm_solver* s) {
 // pointer changes (materials, design box); the stream is drained first, as
 // a queued step may still read the slot.
 static const TorreCold* torre_cold(dtm_solver* s) {
-  const TorreCold h = make_torre_cold(fields_ptr(s), fields_next_ptr(s), s->store, s->pm, s->pmn, s->mt, s->ade);
+  const TorreCold h = make_torre_cold(fields_ptr(s), fields_next_ptr(s), s->pm, s->pmn, s->mt, s->ade);
   for (int k = 0; k < 2; k++)
     if (s->cold_ok[k] && memcmp(&h, &s->cold_host[k], sizeof(TorreCold)) == 0) {
       s->cold_last = k;
@@ -1169,7 +1174,7 @@ static int one_step(dtm_solver* s) {
     const TorreCold* cold = torre_cold(s);
     if (!cold) return DTM_ERR_DEVICE;
     ev_begin(s, 0);
-    launch_torre(s->store, s->g, s->sc, s->mt, cold, &s->whole, 1, s->stream, fold ? fold_for(s, n, 0) : nullptr);
+    launch_torre(s->g, s->sc, s->mt, cold, &s->whole, 1, s->stream, fold ? fold_for(s, n, 0) : nullptr);
     ev_end(s);
     ev_begin(s, 4);
     launch_ade(s->store, s->g, F, fields_next_ptr(s), s->sc, s->mt, s->ade, s->stream);
@@ -1865,7 +1870,7 @@ int dtm_set_fp32_zone(dtm_solver* s, int i0, int i1, int j0, int j1, int k0, int
   if (!s) return fail(DTM_ERR_ARG, "null solver");
   if (s->started) return fail(DTM_ERR_STATE, "the FP32 zone must be set before the first step");
   if (s->store != DTM_STORE_FP16) return fail(DTM_ERR_ARG, "the FP32 zone applies to FP16 storage only");
-  if (s->torre) return fail(DTM_ERR_ARG, "the FP32 zone runs with the two-pass sweeps only");
+  if (s->cfg.sweep == DTM_SWEEP_FUSED) return fail(DTM_ERR_ARG, "the FP32 zone runs with the two-pass sweeps only");
   if (s->sc.xz.on) return fail(DTM_ERR_STATE, "the FP32 zone is already set");
   if (wide_grid(s->g)) return fail(DTM_ERR_LIMIT, "the FP32 zone is limited to grids below 2^32 cells");
   if (!box_ok(s, i0, i1, j0, j1, k0, k1)) return fail(DTM_ERR_ARG, "FP32 zone outside the grid or empty");
@@ -1929,7 +1934,7 @@ int dtm_time_steps(dtm_solver* s, int nsteps, double* ms) {
 }
 
 const char* dtm_kernel_name(const dtm_solver* s) {
-  if (s && s->torre) return s->store == 0 ? "k_torre2<fp32>" : "k_torre2<fp16>";
+  if (s && s->torre) return "k_torre2<fp16>";
   return kernel_variant_name(s ? s->store : 0);
 }
 
@@ -1949,6 +1954,11 @@ int dtm_kernel_times(dtm_solver* s, double* ms, long long* count) {
     s->grp_cnt[s->ev_group[q]] += 1;
   }
   s->ev_used = 0;
+  if (s->cfg.sweep == DTM_SWEEP_FUSED) {  // the step is one group
+    s->grp_ms[0] += s->grp_ms[2];
+    s->grp_ms[2] = 0;
+    s->grp_cnt[2] = 0;
+  }
   for (int g = 0; g < 5; g++) {
     ms[g] = s->grp_ms[g];
     count[g] = s->grp_cnt[g];
@@ -1964,7 +1974,7 @@ long long dtm_group_cells(const dtm_solver* s, int g) {
     return (long long)std::max(0, r.i1 - r.i0) * std::max(0, r.j1 - r.j0) * std::max(0, r.k1 - r.k0);
   };
   if (g < 0 || g > 3) return 0;
-  if (s->torre) return g == 0 ? cells(s->whole) : 0;
+  if (s->cfg.sweep == DTM_SWEEP_FUSED) return g == 0 ? cells(s->whole) : 0;
   return (g == 0 || g == 2) ? cells(s->whole) : 0;
 }
 

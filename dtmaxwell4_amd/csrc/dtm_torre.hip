@@ -1,8 +1,10 @@
 // dtm_torre.hip — fused single-pass time step ("torre" kernel) for gfx950.
 //
 // One launch advances H^{n-1/2} -> H^{n+1/2} and E^n -> E^{n+1} for a set of
-// regions, reading the old fields once and writing the new ones once
-// (48 B per cell-update in FP32 instead of the 72 B of two separate sweeps).
+// regions, reading the old fields once and writing the new ones once.  It runs
+// the fused schedule in FP16 storage, where E is advanced from H^{n+1/2}
+// before that is rounded; in FP32 the two in-place sweeps give the same
+// update in less time (dtm_sweep.hip).
 // This is the temporal fusion of the reference's DiamondTorre, where a torre
 // advances its body diamond (H) and then its nose diamond (E) while sliding
 // one rag along x per step (genAlg.py:385-499, diamond.cu:72-262); here a
@@ -44,7 +46,6 @@ constexpr int NXCD = 8;
 constexpr int kFoldPlanes = 264;  // planes of a block's fold table: segments of at most kFoldPlanes - 3
 
 template <typename T> __device__ __forceinline__ float cv(T v, float inv);
-template <> __device__ __forceinline__ float cv<float>(float v, float) { return v; }
 template <> __device__ __forceinline__ float cv<__half>(__half v, float inv) { return __half2float(v) * inv; }
 // Pointers read from the per-plane table are generic; casting them to the
 // global address space keeps global_load/store (flat accesses would also
@@ -53,7 +54,6 @@ template <typename T> using GlobalT = __attribute__((address_space(1))) T;
 template <typename T> __device__ __forceinline__ GlobalT<T>* gl(T* p) { return (GlobalT<T>*)p; }
 // the table itself lives in the constant address space: scalar loads
 using ColdK = __attribute__((address_space(4))) const TorreCold;
-__device__ __forceinline__ void st(float* F, long long q, float v, float) { gl(F)[q] = v; }
 __device__ __forceinline__ void st(__half* F, long long q, float v, float s) {
   gl(reinterpret_cast<unsigned short*>(F))[q] = __half_as_ushort(__float2half_rn(v * s));
 }
@@ -173,10 +173,10 @@ template <typename T> struct PreT2 {
 // every H evaluation (own and halo columns) adds its weights times the H
 // half-step's factors of plane p, every E update those of the E half-step at
 // plane m.  fold: the H half-step's factor table, the E half-step's after it.
-template <int STORE, int GEN, bool TF>
+template <int GEN, bool TF>
 __global__ __launch_bounds__(TZ* TR) void k_torre2(Grid g, Scales sc, const uint8_t* clsg, const TorreCold* cold,
                                                    TorreSet ts, const float* fold) {
-  using T = typename std::conditional<STORE == 0, float, __half>::type;
+  using T = __half;
   constexpr bool GX = GEN & 1, GY = GEN & 2;
   __shared__ ClassEntry tbl[kMaxClasses];
   __shared__ float sE[2][3][ETILE];   // E^n tile of plane p, buffer (p - p0) & 1
@@ -640,25 +640,23 @@ static int torre_slots(K kernel) {
   return per * cus;
 }
 
-template <int STORE>
-static void torre_go(const Grid& g, const Scales& sc, const Materials& mt, const TorreCold* cold,
-                     const Region* regs, int nreg, hipStream_t st, const float* fold) {
+void launch_torre(const Grid& g, const Scales& sc, const Materials& mt, const TorreCold* cold, const Region* regs,
+                  int nreg, hipStream_t st, const float* fold) {
   const dim3 blk(TZ, TR, 1);
-  static const int slots = torre_slots(k_torre2<STORE, 3, false>);
+  static const int slots = torre_slots(k_torre2<3, false>);
   // a folded source keeps each block's factor table within kFoldPlanes
   TorreSet te = make_torre_set(regs, nreg, torre_seg(regs, nreg, slots, fold ? kFoldPlanes - 3 : 1 << 30));
   if (te.total <= 0) return;
   if (fold)
-    hipLaunchKernelGGL((k_torre2<STORE, 3, true>), dim3(te.per * NXCD), blk, 0, st, g, sc, mt.cls, cold, te, fold);
+    hipLaunchKernelGGL((k_torre2<3, true>), dim3(te.per * NXCD), blk, 0, st, g, sc, mt.cls, cold, te, fold);
   else
-    hipLaunchKernelGGL((k_torre2<STORE, 3, false>), dim3(te.per * NXCD), blk, 0, st, g, sc, mt.cls, cold, te, fold);
+    hipLaunchKernelGGL((k_torre2<3, false>), dim3(te.per * NXCD), blk, 0, st, g, sc, mt.cls, cold, te, fold);
   check_launch("k_torre2");
 }
 
-template <int STORE>
 static void cold_fields(TorreCold& c, const void* fo, const void* fn) {
-  const Fields<STORE>& Fo = *static_cast<const Fields<STORE>*>(fo);
-  const Fields<STORE>& Fn = *static_cast<const Fields<STORE>*>(fn);
+  const Fields<1>& Fo = *static_cast<const Fields<1>*>(fo);
+  const Fields<1>& Fn = *static_cast<const Fields<1>*>(fn);
   for (int q = 0; q < 3; q++) {
     c.fo[q] = Fo.E[q];
     c.fo[3 + q] = Fo.H[q];
@@ -671,12 +669,11 @@ static void cold_fields(TorreCold& c, const void* fo, const void* fn) {
   c.cbytes = (unsigned)(reinterpret_cast<const char*>(Fo.E[1]) - reinterpret_cast<const char*>(Fo.E[0]));
 }
 
-TorreCold make_torre_cold(const void* fields_old, const void* fields_new, int store, const Cpml& pm_old,
+TorreCold make_torre_cold(const void* fields_old, const void* fields_new, const Cpml& pm_old,
                           const Cpml& pm_new, const Materials& mt, const Ade& ade) {
   TorreCold c;
   memset(&c, 0, sizeof(c));  // padding too: callers compare tables bytewise
-  if (store == 0) cold_fields<0>(c, fields_old, fields_new);
-  else cold_fields<1>(c, fields_old, fields_new);
+  cold_fields(c, fields_old, fields_new);
   c.zp.on = pm_old.on;
   for (int a = 0; a < 3; a++) {
     c.zp.plo[a] = pm_old.plo[a];
@@ -693,12 +690,6 @@ TorreCold make_torre_cold(const void* fields_old, const void* fields_new, int st
   memcpy(&c.mt, &mt, sizeof(Materials));
   memcpy(&c.ade, &ade, sizeof(Ade));
   return c;
-}
-
-void launch_torre(int store, const Grid& g, const Scales& sc, const Materials& mt, const TorreCold* cold,
-                  const Region* regs, int nreg, hipStream_t st, const float* fold) {
-  if (store == 0) torre_go<0>(g, sc, mt, cold, regs, nreg, st, fold);
-  else torre_go<1>(g, sc, mt, cold, regs, nreg, st, fold);
 }
 
 }  // namespace dtm

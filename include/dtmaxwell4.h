@@ -166,9 +166,11 @@ typedef struct dtm_soft_source {
 } dtm_soft_source;
 
 /* Time-step schedule.  TWOPASS: one sweep for H, one for E (72 B per
- * cell-update in FP32).  FUSED: H and E of one step in a single x-marching
- * sweep over double-buffered fields (48 B per cell-update plus halo
- * recompute); needs a second copy of the fields. */
+ * cell-update in FP32).  FUSED: one step as a unit.  In FP16 storage H and E
+ * of a step in a single x-marching sweep over double-buffered fields (half
+ * the words of two sweeps plus halo recompute; E is advanced from H before
+ * that is rounded), which needs a second copy of the fields; in FP32 the two
+ * in-place sweeps, which compute the same update in less time. */
 enum { DTM_SWEEP_TWOPASS = 0, DTM_SWEEP_FUSED = 1 };
 
 typedef struct dtm_config {
