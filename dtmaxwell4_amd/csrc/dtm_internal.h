@@ -85,6 +85,8 @@ struct Ade {
   int on;
   int i0, j0, k0, ni, nj, nk;  // bounding box
   long long bsx, bsy;
+  int npoles;                  // the most poles of a material
+  unsigned special[kMaxClasses / 32];  // bit per class: its cells are in the ADE state
   float* Em[3];
   float* Jp[3][kMaxPoles];
   float* Jm[3][kMaxPoles];

@@ -787,6 +787,9 @@ static int build_classes_into(dtm_solver* s, const uint8_t* const m[3]) {
   Ade& A = s->ade;
   A.on = any_special ? 1 : 0;
   A.gyro_on = any_gyro ? 1 : 0;
+  memset(A.special, 0, sizeof(A.special));
+  for (int id = 0; id < ncls; id++)
+    if (s->classes[id].special) A.special[id >> 5] |= 1u << (id & 31);
   if (any_special) {
     A.i0 = bb[0];
     A.j0 = bb[2];
@@ -805,6 +808,7 @@ static int build_classes_into(dtm_solver* s, const uint8_t* const m[3]) {
       maxp = std::max(maxp, am[mm].np);
       if (c.mat[mm].gyro) gyro_coeffs(c.mat[mm], c.dt, gm[mm]);
     }
+    A.npoles = maxp;
     for (int q = 0; q < 3; q++) {
       if (int rc = dalloc(s, &A.curl[q], sizeof(float) * nb)) return rc;
       if (int rc = sdalloc(s, &A.Em[q], sizeof(float) * nb)) return rc;
