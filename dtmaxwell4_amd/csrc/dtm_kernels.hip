@@ -160,9 +160,7 @@ __device__ __forceinline__ int comp_at(int hx, int hy, int hz) {
 // The neighbours differ from the point only along a, so no face is crossed
 // unless the point lies inside the box on the other two axes; then a
 // neighbour crosses when its a-coordinate is on the other side of [hlo, hhi].
-template <int TAB>
-__device__ __forceinline__ float tfsf_dcorr(const Tfsf& s, int hx, int hy, int hz, int a, double t,
-                                           const double* table) {
+__device__ __forceinline__ float tfsf_dcorr(const Tfsf& s, int hx, int hy, int hz, int a, double t) {
   const int hp[3] = {hx, hy, hz};
   const int b1 = (a + 1) % 3, b2 = (a + 2) % 3;
   if (hp[b1] < s.hlo[b1] || hp[b1] > s.hhi[b1] || hp[b2] < s.hlo[b2] || hp[b2] > s.hhi[b2]) return 0.f;
@@ -180,18 +178,7 @@ __device__ __forceinline__ float tfsf_dcorr(const Tfsf& s, int hx, int hy, int h
     const bool qin = hq >= lo && hq <= hi;
     if (qin == pin) continue;
     const bool qsf = s.sf_inside ? qin : !qin;  // the neighbour is in the scattered-field region
-    double v;
-    if constexpr (TAB == 1) {
-      const int ha = s.tab_axis == a ? hq : hp[s.tab_axis];
-      v = s.P[cq] * table[min(max(ha - s.tab_h0, 0), s.tab_n - 1)];
-    } else if constexpr (TAB == 2) {  // the launch's point table; clamped reads stay in it
-      const int px = min(max((a == 0 ? hq : hx) - s.ptab_h0[0], 0), s.ptab_n[0] - 1);
-      const int py = min(max((a == 1 ? hq : hy) - s.ptab_h0[1], 0), s.ptab_n[1] - 1);
-      const int pz = min(max((a == 2 ? hq : hz) - s.ptab_h0[2], 0), s.ptab_n[2] - 1);
-      v = s.ptab[(((long long)cq * s.ptab_n[0] + px) * s.ptab_n[1] + py) * s.ptab_n[2] + pz];
-    } else {
-      v = incident(s, cq, a == 0 ? hq : hx, a == 1 ? hq : hy, a == 2 ? hq : hz, t);
-    }
+    const double v = incident(s, cq, a == 0 ? hq : hx, a == 1 ? hq : hy, a == 2 ? hq : hz, t);
     acc += wt[q] * (qsf ? v : -v);
   }
   return (float)acc;
@@ -378,89 +365,87 @@ __global__ __launch_bounds__(256) void k_ade(AdeArgs<STORE> A) {
 // the first band that contains it, and that thread applies the terms of
 // every axis whose band holds the cell, so cells where bands of different
 // axes overlap (box edges and corners) are written by one thread only.
-template <int STORE, int MODE, int TAB>
-__global__ __launch_bounds__(256) void k_tfsf(Grid g, Fields<STORE> f, Scales sc, Cpml pm, Materials mt, Ade ade,
-                                              Tfsf tf, TfsfBands bands, double tinc) {
-  constexpr int HALF = MODE == 1 ? 1 : 0;
-  // band and position from the thread index: 32-bit arithmetic (band cells
-  // number far fewer than 2^31; 64-bit division would dominate the kernel).
-  // Each band starts at a multiple of 64 threads, so a wavefront lies in one
-  // band: the band index is found from the wavefront's first thread and the
-  // band tables are read with scalar loads.
+// Cell and band of a thread: 32-bit arithmetic (band cells number far fewer
+// than 2^31; 64-bit division would dominate the kernel).  Each band starts at
+// a multiple of 64 threads, so a wavefront lies in one band: the band index is
+// found from the wavefront's first thread and the band tables are read with
+// scalar loads.  False: padding of a band, or the cell of an earlier band.
+__device__ __forceinline__ bool band_has(const TfsfBands& bands, int r, int q, int i, int j, int k) {
+  const Region& Q = bands.r[q];  // (only bands that overlap band r can hold a cell of it)
+  return ((bands.ovl[r] >> q) & 1u) && i >= Q.i0 && i < Q.i1 && j >= Q.j0 && j < Q.j1 && k >= Q.k0 && k < Q.k1;
+}
+__device__ __forceinline__ bool band_cell(const TfsfBands& bands, int& r, int& i, int& j, int& k) {
   const unsigned gid = blockIdx.x * blockDim.x + threadIdx.x;
   const unsigned g0 = __builtin_amdgcn_readfirstlane(gid);
-  int r = 0;
+  r = 0;
   while (r < bands.n && g0 >= bands.start[r + 1]) r++;
-  if (r >= bands.n) return;
+  if (r >= bands.n) return false;
   const Region& R = bands.r[r];
   const unsigned nk = (unsigned)(R.k1 - R.k0), nj = (unsigned)(R.j1 - R.j0);
   unsigned loc = gid - bands.start[r];
-  if (loc >= nk * nj * (unsigned)(R.i1 - R.i0)) return;  // the band's padding
+  if (loc >= nk * nj * (unsigned)(R.i1 - R.i0)) return false;
   const unsigned lk = loc % nk;
   loc /= nk;
-  const int k = R.k0 + (int)lk;
-  const int j = R.j0 + (int)(loc % nj);
-  const int i = R.i0 + (int)(loc / nj);
-  auto holds = [&](int q) {  // cell in band q (only bands that overlap band r can hold it)
-    const Region& Q = bands.r[q];
-    return ((bands.ovl[r] >> q) & 1u) && i >= Q.i0 && i < Q.i1 && j >= Q.j0 && j < Q.j1 && k >= Q.k0 &&
-           k < Q.k1;
-  };
+  k = R.k0 + (int)lk;
+  j = R.j0 + (int)(loc % nj);
+  i = R.i0 + (int)(loc / nj);
   for (int r2 = 0; r2 < r; r2++)
-    if (holds(r2)) return;  // owned by an earlier band
-  const long long q = i * g.sx + j * g.sy + k;
+    if (band_has(bands, r, r2, i, j, k)) return false;
+  return true;
+}
+
+// The correction D of the derivative along axis a in curl component c (t 0:
+// its first term, 1: its second), through the layer: into dc, the curl
+// correction per component, and dc2, its part on the stored split-field part.
+template <int MODE>
+__device__ __forceinline__ void tfsf_term(const Grid& g, const Cpml& pm, int a, int c, int t, float D, int i, int j,
+                                          int k, float* dc, float* dc2) {
+  constexpr int HALF = MODE == 1 ? 1 : 0;
   const int vpos[3] = {i, j, k};
-  static constexpr int off[6][3] = {{0, 1, 1}, {1, 0, 1}, {1, 1, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
-  float dc[3] = {0.f, 0.f, 0.f};  // curl correction per component, all axes
-  float dc2[3] = {0.f, 0.f, 0.f}; // its part on the stored split-field part (second curl axis)
-  for (int rb = r; rb < bands.n; rb++) {
-    if (rb != r && !holds(rb)) continue;
-    const int a = bands.axis[rb];
-    // components with a derivative along a: c1 = (a+2)%3 (first curl term),
-    // c2 = (a+1)%3 (second curl term); psi slots 1 and 0 of axis a.
-    for (int t = 0; t < 2; t++) {
-      const int c = t == 0 ? (a + 2) % 3 : (a + 1) % 3;
-      const float sgn = t == 0 ? 1.0f : -1.0f;
-      const int slot = t == 0 ? 1 : 0;
-      const int comp = HALF == 0 ? 3 + c : c;
-      const int hx = 2 * i + off[comp][0], hy = 2 * j + off[comp][1], hz = 2 * k + off[comp][2];
-      const float D = g.rd[a] * tfsf_dcorr<TAB>(tf, hx, hy, hz, a, tinc, tf.table);
-      if (D == 0.0f) continue;
-      float cp = 0.0f;
-      if (pm.on && pm.split) {  // split-field layer: the part of axis a gets k2 * D
-        auto k2_of = [&](int ax) {  // 1 off the slab of axis ax
-          const int n = ax == 0 ? g.nx : (ax == 1 ? g.ny : g.nz);
-          if (slab_index(vpos[ax], n, pm.plo[ax], pm.phi[ax]) < 0) return 1.0f;
-          return HALF == 0 ? pm.cH[ax][vpos[ax]] : pm.cE[ax][vpos[ax]];
-        };
-        const float k2 = k2_of(a);
-        // the cell keeps split parts when either curl axis has k2 != 1; the
-        // second curl axis (t = 1) owns the stored part
-        if (k2 != 1.0f || k2_of(t == 0 ? (c + 2) % 3 : (c + 1) % 3) != 1.0f) {
-          dc[c] += sgn * k2 * D;
-          if (t == 1) dc2[c] += sgn * k2 * D;
-          continue;
-        }
-      } else if (pm.on) {
-        const int n = a == 0 ? g.nx : (a == 1 ? g.ny : g.nz);
-        const int si = slab_index(vpos[a], n, pm.plo[a], pm.phi[a]);
-        if (si >= 0) {
-          cp = HALF == 0 ? pm.cH[a][vpos[a]] : pm.cE[a][vpos[a]];
-          float* psi = HALF == 0 ? pm.psiH[a][slot] : pm.psiE[a][slot];
-          const long long pq = psi_index(g, pm, a, si, i, j, k);
-          if (MODE == 2) {
-            psi[pq] += cp * D / pm.bH[a][vpos[a]];
-            cp = 0.0f;
-          } else {
-            psi[pq] += cp * D;
-          }
-        }
+  const float sgn = t == 0 ? 1.0f : -1.0f;
+  const int slot = t == 0 ? 1 : 0;  // psi slots 1 and 0 of axis a
+  float cp = 0.0f;
+  if (pm.on && pm.split) {  // split-field layer: the part of axis a gets k2 * D
+    auto k2_of = [&](int ax) {  // 1 off the slab of axis ax
+      const int n = ax == 0 ? g.nx : (ax == 1 ? g.ny : g.nz);
+      if (slab_index(vpos[ax], n, pm.plo[ax], pm.phi[ax]) < 0) return 1.0f;
+      return HALF == 0 ? pm.cH[ax][vpos[ax]] : pm.cE[ax][vpos[ax]];
+    };
+    const float k2 = k2_of(a);
+    // the cell keeps split parts when either curl axis has k2 != 1; the
+    // second curl axis (t = 1) owns the stored part
+    if (k2 != 1.0f || k2_of(t == 0 ? (c + 2) % 3 : (c + 1) % 3) != 1.0f) {
+      dc[c] += sgn * k2 * D;
+      if (t == 1) dc2[c] += sgn * k2 * D;
+      return;
+    }
+  } else if (pm.on) {
+    const int n = a == 0 ? g.nx : (a == 1 ? g.ny : g.nz);
+    const int si = slab_index(vpos[a], n, pm.plo[a], pm.phi[a]);
+    if (si >= 0) {
+      cp = HALF == 0 ? pm.cH[a][vpos[a]] : pm.cE[a][vpos[a]];
+      float* psi = HALF == 0 ? pm.psiH[a][slot] : pm.psiE[a][slot];
+      const long long pq = psi_index(g, pm, a, si, i, j, k);
+      if (MODE == 2) {
+        psi[pq] += cp * D / pm.bH[a][vpos[a]];
+        cp = 0.0f;
+      } else {
+        psi[pq] += cp * D;
       }
-      dc[c] += sgn * (1.0f + cp) * D;
     }
   }
+  dc[c] += sgn * (1.0f + cp) * D;
+}
+
+// Adds the corrections of a cell to its fields.
+template <int STORE, int MODE>
+__device__ __forceinline__ void tfsf_apply(const Grid& g, const Fields<STORE>& f, const Scales& sc, const Cpml& pm,
+                                           const Materials& mt, const Ade& ade, int i, int j, int k, const float* dc,
+                                           const float* dc2) {
+  const long long q = i * g.sx + j * g.sy + k;
   const int xq = STORE == 1 ? exact_idx(sc.xz, i, j, k) : -1;
-  if (HALF == 0) {
+  if (MODE != 1) {
+#pragma unroll
     for (int c = 0; c < 3; c++) {
       if (dc[c] != 0.0f)
         stx(f.H[c], q, ldx(f.H[c], q, sc.ih[c], sc.xz, 3 + c, xq) - g.dt * dc[c], sc.sh[c], sc.xz, 3 + c, xq);
@@ -478,6 +463,7 @@ __global__ __launch_bounds__(256) void k_tfsf(Grid g, Fields<STORE> f, Scales sc
       over = true;
     }
   }
+#pragma unroll
   for (int c = 0; c < 3; c++) {
     if (dc[c] == 0.0f) continue;
     if (!over && (ce.special & (1 << c)) && ade.on) {
@@ -492,6 +478,125 @@ __global__ __launch_bounds__(256) void k_tfsf(Grid g, Fields<STORE> f, Scales sc
       if (dc2[c] != 0.0f) pm.p2E[c][q] += g.dt * ie * dc2[c];
     }
   }
+}
+
+constexpr int kOff[6][3] = {{0, 1, 1}, {1, 0, 1}, {1, 1, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
+
+// Incident field evaluated at every point.
+template <int STORE, int MODE>
+__global__ __launch_bounds__(256) void k_tfsf(Grid g, Fields<STORE> f, Scales sc, Cpml pm, Materials mt, Ade ade,
+                                              Tfsf tf, TfsfBands bands, double tinc) {
+  int r, i, j, k;
+  if (!band_cell(bands, r, i, j, k)) return;
+  float dc[3] = {0.f, 0.f, 0.f}, dc2[3] = {0.f, 0.f, 0.f};
+  for (int rb = r; rb < bands.n; rb++) {
+    if (rb != r && !band_has(bands, r, rb, i, j, k)) continue;
+    const int a = bands.axis[rb];
+    // components with a derivative along a: (a+2)%3 (first curl term), (a+1)%3 (second)
+    for (int t = 0; t < 2; t++) {
+      const int c = t == 0 ? (a + 2) % 3 : (a + 1) % 3;
+      const int comp = MODE == 1 ? c : 3 + c;
+      const float D = g.rd[a] * tfsf_dcorr(tf, 2 * i + kOff[comp][0], 2 * j + kOff[comp][1], 2 * k + kOff[comp][2], a, tinc);
+      if (D == 0.0f) continue;
+      tfsf_term<MODE>(g, pm, a, c, t, D, i, j, k, dc, dc2);
+    }
+  }
+  tfsf_apply<STORE, MODE>(g, f, sc, pm, mt, ade, i, j, k, dc, dc2);
+}
+
+// One point of a dipole's table (Tfsf::ptab) at time t.
+__device__ __forceinline__ void tfsf_point(const Tfsf& tf, double* out, long long q, double t) {
+  const long long n = 6LL * tf.ptab_n[0] * tf.ptab_n[1] * tf.ptab_n[2];
+  if (q >= n) return;  // n < 2^31 (kMaxPointTable)
+  const unsigned n1 = tf.ptab_n[1], n2 = tf.ptab_n[2], u = (unsigned)q;
+  const int p2 = (int)(u % n2);
+  const unsigned r = u / n2;
+  const int p1 = (int)(r % n1);
+  const int p0 = (int)((r / n1) % (unsigned)tf.ptab_n[0]);
+  const int c = (int)(r / n1 / (unsigned)tf.ptab_n[0]);
+  out[q] = incident(tf, c, tf.ptab_h0[0] + p0, tf.ptab_h0[1] + p1, tf.ptab_h0[2] + p2, t);
+}
+
+// Incident field from a table: TAB 1 of a plane wave along an axis, per
+// half-coordinate; TAB 2 of a small dipole box, per point.  The axes and
+// components are unrolled: which component a stencil reads, and all its
+// indices, are then known, and the table values of a cell are loaded together.
+// A dipole's launch takes every cell around its box (bands.r[0]) instead of
+// the face bands, and its blocks from nblk on fill the table of the next
+// half-step.  Bound by its chain of loads: the table, the cell's fields, the
+// store.  A dipole box of 4^3 cells: 5.8 us (H) and 6.7 us (E), against 18.4,
+// 18.8 and 4.6 for each table's own launch with axis, component and neighbour
+// in nested loops.  Plane wave along z, 128x128 cells on two faces: 5.8 and
+// 6.8 us against 7.1 and 7.7.
+template <int STORE, int MODE, int TAB>
+__global__ __launch_bounds__(256) void k_tfsf_tab(Grid g, Fields<STORE> f, Scales sc, Cpml pm, Materials mt, Ade ade,
+                                                  Tfsf tf, TfsfBands bands, unsigned nblk) {
+  if (TAB == 2 && blockIdx.x >= nblk) {
+    tfsf_point(tf, tf.pnext, (blockIdx.x - nblk) * 256LL + threadIdx.x, tf.tnext);
+    return;
+  }
+  int i, j, k;
+  if constexpr (TAB == 2) {
+    const Region& R = bands.r[0];
+    const unsigned nk = (unsigned)(R.k1 - R.k0), nj = (unsigned)(R.j1 - R.j0);
+    const unsigned loc = blockIdx.x * 256 + threadIdx.x, row = loc / nk;
+    if (loc >= nk * nj * (unsigned)(R.i1 - R.i0)) return;
+    k = R.k0 + (int)(loc - row * nk);
+    j = R.j0 + (int)(row % nj);
+    i = R.i0 + (int)(row / nj);
+  } else {
+    int r;
+    if (!band_cell(bands, r, i, j, k)) return;
+  }
+  const int v[3] = {i, j, k};
+  const int ho[4] = {-3, -1, 1, 3};
+  const double wt[4] = {1.0, -27.0, 27.0, -1.0};
+  float dc[3] = {0.f, 0.f, 0.f}, dc2[3] = {0.f, 0.f, 0.f}, D[3][2];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const int b1 = (a + 1) % 3, b2 = (a + 2) % 3;
+    const bool face = (v[a] >= tf.fl0[a] && v[a] <= tf.fl1[a]) || (v[a] >= tf.fh0[a] && v[a] <= tf.fh1[a]);
+    D[a][0] = D[a][1] = 0.f;
+    // (a wave of one band has two axes without a face)
+    if (TAB == 1 && __builtin_amdgcn_ballot_w64(face) == 0) continue;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int c = t == 0 ? b2 : b1;
+      const int comp = MODE == 1 ? c : 3 + c;                       // updated
+      const int cq = (MODE == 1 ? 3 : 0) + (t == 0 ? b1 : b2);      // read across the face
+      const int h[3] = {2 * i + kOff[comp][0], 2 * j + kOff[comp][1], 2 * k + kOff[comp][2]};
+      const bool in = h[b1] >= tf.hlo[b1] && h[b1] <= tf.hhi[b1] && h[b2] >= tf.hlo[b2] && h[b2] <= tf.hhi[b2];
+      const bool pin = h[a] >= tf.hlo[a] && h[a] <= tf.hhi[a];
+      double acc = 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int hq = h[a] + ho[q];
+        const bool qin = hq >= tf.hlo[a] && hq <= tf.hhi[a];
+        const bool need = in && qin != pin;
+        double x;
+        if constexpr (TAB == 1) {
+          const int ha = tf.tab_axis == a ? hq : h[tf.tab_axis == b1 ? b1 : b2];
+          x = tf.P[cq] * tf.table[min(max(ha - tf.tab_h0, 0), tf.tab_n - 1)];
+        } else {
+          int p[3];
+#pragma unroll
+          for (int e = 0; e < 3; e++) p[e] = (e == a ? hq : h[e]) - tf.ptab_h0[e];
+          const int at = ((cq * tf.ptab_n[0] + p[0]) * tf.ptab_n[1] + p[1]) * tf.ptab_n[2] + p[2];
+          x = tf.ptab[need ? at : 0];  // a needed point lies in the table
+        }
+        const bool qsf = tf.sf_inside ? qin : !qin;  // the neighbour is in the scattered-field region
+        acc += wt[q] * (need ? (qsf ? x : -x) : 0.0);
+      }
+      D[a][t] = g.rd[a] * (float)acc;
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      if (D[a][t] != 0.0f)
+        tfsf_term<MODE>(g, pm, a, t == 0 ? (a + 2) % 3 : (a + 1) % 3, t, D[a][t], i, j, k, dc, dc2);
+  tfsf_apply<STORE, MODE>(g, f, sc, pm, mt, ade, i, j, k, dc, dc2);
 }
 
 // Plane-wave waveform along the propagation axis, one value per
@@ -617,10 +722,33 @@ static void check_launch(const char* what) { note_launch(what); }
 // One launch over the union of the face bands (k_tfsf gives each cell one
 // writer); the host fills each band's first thread index and its overlap
 // mask.
+static unsigned point_blocks(const Tfsf& tf) {
+  return (unsigned)((6LL * tf.ptab_n[0] * tf.ptab_n[1] * tf.ptab_n[2] + 255) / 256);
+}
 template <int STORE, int MODE>
 static void tfsf_go(const Grid& g, const void* fields, const Scales& sc, const Cpml& pm, const Materials& mt,
                     const Ade& ade, const Tfsf& tf, const TfsfBands& bands, double tinc, hipStream_t st) {
   const Fields<STORE>& f = *static_cast<const Fields<STORE>*>(fields);
+  if (tf.ptab) {  // a dipole with a table: the cells around its box
+    TfsfBands b{};
+    const int dim[3] = {g.nx, g.ny, g.nz};
+    int lo[3], hi[3];
+    long long n = 1;
+    for (int a = 0; a < 3; a++) {
+      lo[a] = std::max(tf.fl0[a], 0);
+      hi[a] = std::min(tf.fh1[a] + 1, dim[a]);
+      n *= std::max(hi[a] - lo[a], 0);
+    }
+    if (n == 0 || bands.n == 0) return;
+    b.n = 1;
+    b.r[0] = Region{lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]};
+    const unsigned nblk = (unsigned)((n + 255) / 256);
+    const unsigned more = tf.pnext ? point_blocks(tf) : 0;
+    hipLaunchKernelGGL((k_tfsf_tab<STORE, MODE, 2>), dim3(nblk + more), dim3(256), 0, st, g, f, sc, pm, mt, ade, tf,
+                       b, nblk);
+    check_launch("k_tfsf_tab");
+    return;
+  }
   TfsfBands b = bands;
   long long n = 0;
   b.start[0] = 0;
@@ -640,13 +768,11 @@ static void tfsf_go(const Grid& g, const void* fields, const Scales& sc, const C
     fail_launch("k_tfsf", "TF/SF face bands hold 2^31 cells or more");
     return;
   }
-  const dim3 grid((unsigned)((n + 255) / 256));
+  const unsigned nblk = (unsigned)((n + 255) / 256);
   if (tf.tab_axis >= 0)
-    hipLaunchKernelGGL((k_tfsf<STORE, MODE, 1>), grid, dim3(256), 0, st, g, f, sc, pm, mt, ade, tf, b, tinc);
-  else if (tf.ptab)
-    hipLaunchKernelGGL((k_tfsf<STORE, MODE, 2>), grid, dim3(256), 0, st, g, f, sc, pm, mt, ade, tf, b, tinc);
+    hipLaunchKernelGGL((k_tfsf_tab<STORE, MODE, 1>), dim3(nblk), dim3(256), 0, st, g, f, sc, pm, mt, ade, tf, b, nblk);
   else
-    hipLaunchKernelGGL((k_tfsf<STORE, MODE, 0>), grid, dim3(256), 0, st, g, f, sc, pm, mt, ade, tf, b, tinc);
+    hipLaunchKernelGGL((k_tfsf<STORE, MODE>), dim3(nblk), dim3(256), 0, st, g, f, sc, pm, mt, ade, tf, b, tinc);
   check_launch("k_tfsf");
 }
 
@@ -736,23 +862,14 @@ void launch_tfsf_fold(const Tfsf& tf, const double* tables, float* out, int nste
 // one thread per value, so the FP64 transcendentals of a dipole run across
 // the chip instead of in the band threads one after another.
 __global__ __launch_bounds__(256) void k_tfsf_points(Tfsf tf, double t) {
-  const long long n = 6LL * tf.ptab_n[0] * tf.ptab_n[1] * tf.ptab_n[2];
-  const long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const int p2 = (int)(q % tf.ptab_n[2]);
-  const long long r = q / tf.ptab_n[2];
-  const int p1 = (int)(r % tf.ptab_n[1]);
-  const int p0 = (int)((r / tf.ptab_n[1]) % tf.ptab_n[0]);
-  const int c = (int)(r / tf.ptab_n[1] / tf.ptab_n[0]);
-  tf.ptab[q] = incident(tf, c, tf.ptab_h0[0] + p0, tf.ptab_h0[1] + p1, tf.ptab_h0[2] + p2, t);
+  tfsf_point(tf, tf.ptab, blockIdx.x * 256LL + threadIdx.x, t);
 }
 
 void launch_tfsf(int store, int half, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                  const Materials& mt, const Ade& ade, const Tfsf& tf, const TfsfBands& bands, double t_inc,
                  hipStream_t st) {
-  if (tf.ptab && tf.tab_axis < 0) {
-    const long long n = 6LL * tf.ptab_n[0] * tf.ptab_n[1] * tf.ptab_n[2];
-    hipLaunchKernelGGL(k_tfsf_points, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, tf, t_inc);
+  if (tf.ptab && !tf.pfull) {
+    hipLaunchKernelGGL(k_tfsf_points, dim3(point_blocks(tf)), dim3(256), 0, st, tf, t_inc);
     check_launch("k_tfsf_points");
   }
   if (store == 0 && half == 0) tfsf_go<0, 0>(g, fields, sc, pm, mt, ade, tf, bands, t_inc, st);

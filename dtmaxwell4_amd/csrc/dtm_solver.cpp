@@ -70,6 +70,9 @@ struct dtm_solver {
   bool torre = false;
   bool no_fold = false; // tabulated plane-wave TF/SF through k_tfsf instead of the sweeps
   float* fold_base = nullptr; // per-plane factors of a folded plane wave, kTableSteps x 2 half-steps
+  double* points[2] = {};          // a dipole's tables of incident values, by the parity of the half-step
+  long long points_for[2] = {-1, -1};  // 2 n + half that each holds, within a call
+  bool more = false;               // another forward step follows in this call
   int2* fold_w = nullptr;     // the sweeps' weights of that source, one entry per chunk of cells and half-step
   // device copies of the fused step's pointer table, one per buffer parity
   // (the old / new buffers swap every step), and their host images
@@ -497,7 +500,9 @@ static int setup_tfsf(dtm_solver* s) {
       s->tf.ptab_n[a] = (int)std::max(0LL, std::min(n, kMaxPointTable));
     }
     if (tot <= kMaxPointTable)
-      if (int rc = dalloc(s, &s->tf.ptab, sizeof(double) * (size_t)tot)) return rc;
+      for (double*& p : s->points)
+        if (int rc = dalloc(s, &p, sizeof(double) * (size_t)tot)) return rc;
+    s->tf.ptab = s->points[0];
   }
   if (s->tf.kind != DTM_TFSF_NONE && s->tf.tab_axis >= 0) {
     if (int rc = dalloc(s, &s->tab_base, sizeof(double) * 2 * kTableSteps * s->tf.tab_n)) return rc;
@@ -511,11 +516,31 @@ static int setup_tfsf(dtm_solver* s) {
   return 0;
 }
 
+static bool tfsf_gate(const dtm_solver* s, long long n) {
+  const dtm_config& c = s->cfg;
+  if (c.tfsf.kind == DTM_TFSF_NONE) return false;
+  const int nt = c.ntime > 0 ? c.ntime : 1;
+  const long long istep = n / nt;
+  return (double)((istep + 1) * nt) * c.dt < c.tfsf.tStop;  // window.hpp:125
+}
+
 // Tfsf of one TF/SF launch: for a tabulated plane wave, points the table
 // at step n, half (0: H half-step, 1: E half-step), filling the next batch
 // of tables first when step n is not in the current one.
 static Tfsf tfsf_for(dtm_solver* s, long long n, int half) {
   Tfsf t = s->tf;
+  if (t.ptab) {
+    // a dipole's point tables: the launch of a half-step also fills the other
+    // table for the next one, if that runs in this call
+    const long long key = 2 * n + half;
+    t.ptab = s->points[key & 1];
+    t.pfull = s->points_for[key & 1] == key;
+    const bool next = half == 0 || (s->more && tfsf_gate(s, n + 1));
+    t.pnext = next ? s->points[~key & 1] : nullptr;
+    t.tnext = half == 0 ? ((double)n + 0.5) * s->cfg.dt : ((double)n + 1.0) * s->cfg.dt;
+    s->points_for[~key & 1] = next ? key + 1 : -1;
+    return t;
+  }
   if (t.tab_axis < 0) return t;
   if (s->tab_n0 < 0 || n < s->tab_n0 || n >= s->tab_n0 + kTableSteps) {
     s->tab_n0 = n;
@@ -529,14 +554,6 @@ static Tfsf tfsf_for(dtm_solver* s, long long n, int half) {
 // The fold factor table of step n, half (after tfsf_for filled its batch).
 static const float* fold_for(const dtm_solver* s, long long n, int half) {
   return s->fold_base + ((n - s->tab_n0) * 2 + half) * (long long)fold_floats(s);
-}
-
-static bool tfsf_gate(const dtm_solver* s, long long n) {
-  const dtm_config& c = s->cfg;
-  if (c.tfsf.kind == DTM_TFSF_NONE) return false;
-  const int nt = c.ntime > 0 ? c.ntime : 1;
-  const long long istep = n / nt;
-  return (double)((istep + 1) * nt) * c.dt < c.tfsf.tStop;  // window.hpp:125
 }
 
 static int setup_cpml(dtm_solver* s) {
@@ -1266,11 +1283,20 @@ static int one_step(dtm_solver* s) {
   return 0;
 }
 
+static int run_steps(dtm_solver* s, int nsteps) {
+  s->points_for[0] = s->points_for[1] = -1;
+  for (int t = 0; t < nsteps; t++) {
+    s->more = t + 1 < nsteps;
+    if (int rc = one_step(s)) return rc;
+  }
+  s->points_for[0] = s->points_for[1] = -1;
+  return 0;
+}
+
 int dtm_step(dtm_solver* s, int nsteps) {
   if (!s || nsteps < 0) return fail(DTM_ERR_ARG, "bad step arguments");
   if (int rc = start(s)) return rc;
-  for (int t = 0; t < nsteps; t++)
-    if (int rc = one_step(s)) return rc;
+  if (int rc = run_steps(s, nsteps)) return rc;
   return launch_result();
 }
 
@@ -1925,8 +1951,7 @@ int dtm_time_steps(dtm_solver* s, int nsteps, double* ms) {
   HIPCHK(hipEventCreate(&a));
   HIPCHK(hipEventCreate(&b));
   HIPCHK(hipEventRecord(a, s->stream));
-  for (int t = 0; t < nsteps; t++)
-    if (int rc = one_step(s)) return rc;
+  if (int rc = run_steps(s, nsteps)) return rc;
   HIPCHK(hipEventRecord(b, s->stream));
   HIPCHK(hipEventSynchronize(b));
   float f = 0;
