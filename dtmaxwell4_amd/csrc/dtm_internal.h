@@ -335,9 +335,11 @@ int take_launch_error(char* msg, int cap);
 // fold non-null: add a plane-wave TF/SF source along x inside the sweep, from
 // this half-step's per-plane factors (launch_tfsf_fold) and the weights of
 // every chunk of cells (launch_fold_weights); none with an FP32 zone.
+// pr non-null: the launch also records the probes of the field that it only
+// reads (up 0: E as it is before the step, up 1: the new H).
 void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                   const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
-                  hipStream_t st);
+                  const Probes* pr, hipStream_t st);
 // entries of the weights, both half-steps
 long long fold_weights_size(const Grid& g);
 void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t st);
@@ -380,7 +382,8 @@ TorreCold make_torre_cold(const void* fields_old, const void* fields_new, const 
                           const Cpml& pm_new, const Materials& mt, const Ade& ade);
 void launch_soft(int store, const Grid& g, const void* fields, const Scales& sc, const Soft& so,
                  hipStream_t st);
-void launch_record(int store, const Grid& g, const void* fields, const Scales& sc, const Probes& pr,
+// which: bit 0: probes of E components, bit 1: of H components
+void launch_record(int store, const Grid& g, const void* fields, const Scales& sc, const Probes& pr, int which,
                    hipStream_t st);
 // Flux of the step n -> n+1: launch_flux_snap before it, launch_flux after it
 // (dtm_flux.hip).

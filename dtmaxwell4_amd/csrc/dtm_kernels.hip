@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "dtm_internal.h"
+#include "dtm_probe.h"
 
 namespace dtm {
 
@@ -631,57 +632,15 @@ __global__ void k_soft(Fields<STORE> f, Scales sc, Soft so) {
 }
 
 template <int STORE>
-__device__ float fval(const Grid& g, const Fields<STORE>& f, const Scales& sc, int comp, int i, int j, int k) {
-  const int ii = nbr(i, 0, g.nx, g.per[0]), jj = nbr(j, 0, g.ny, g.per[1]), kk = nbr(k, 0, g.nz, g.per[2]);
-  if (ii < 0 || jj < 0 || kk < 0) return 0.f;
-  const long long q = ii * g.sx + jj * g.sy + kk;
-  const int xq = STORE == 1 ? exact_idx(sc.xz, ii, jj, kk) : -1;
-  return comp < 3 ? ldx(f.E[comp], q, sc.ie[comp], sc.xz, comp, xq)
-                  : ldx(f.H[comp - 3], q, sc.ih[comp - 3], sc.xz, comp, xq);
-}
-
-// Reference sensor interpolation (sensor.h:64-71) on the cell lattice.
-template <int STORE>
-__device__ float sensor_val(const Grid& g, const Fields<STORE>& f, const Scales& sc, int comp, int x, int y,
-                            int z) {
-  const int zM = (z == 0) ? z + 1 : z - 1;
-  switch (comp) {
-    case 0:
-      return 0.25f * (fval(g, f, sc, 0, x, y - 1, zM) + fval(g, f, sc, 0, x, y - 1, z) +
-                      fval(g, f, sc, 0, x, y, zM) + fval(g, f, sc, 0, x, y, z));
-    case 1:
-      return 0.25f * (fval(g, f, sc, 1, x - 1, y, zM) + fval(g, f, sc, 1, x - 1, y, z) +
-                      fval(g, f, sc, 1, x, y, zM) + fval(g, f, sc, 1, x, y, z));
-    case 2:
-      return 0.25f * (fval(g, f, sc, 2, x - 1, y - 1, z) + fval(g, f, sc, 2, x - 1, y, z) +
-                      fval(g, f, sc, 2, x, y - 1, z) + fval(g, f, sc, 2, x, y, z));
-    case 3: return 0.5f * (fval(g, f, sc, 3, x - 1, y, z) + fval(g, f, sc, 3, x, y, z));
-    case 4: return 0.5f * (fval(g, f, sc, 4, x, y - 1, z) + fval(g, f, sc, 4, x, y, z));
-    default: return 0.5f * (fval(g, f, sc, 5, x, y, zM) + fval(g, f, sc, 5, x, y, z));
-  }
-}
-
-template <int STORE>
-// One thread per (probe, DFT bin): every thread of a probe reads its value
-// (a few cached loads), the bin-0 thread stores it to the series, and each
-// thread advances its own FP64 accumulator, so the sincos of the bins run in
-// parallel rather than one after another (64 bins: 26 -> 5 us per step).
-__global__ void k_record(Grid g, Fields<STORE> f, Scales sc, Probes pr) {
-  const int nb = pr.nfreq > 0 ? pr.nfreq : 1;
-  const long long tid = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (tid >= (long long)pr.n * nb) return;
-  const int p = (int)(tid / nb), fq = (int)(tid % nb);
-  const ProbeDesc d = pr.desc[p];
-  const float v = d.kind == 0 ? fval(g, f, sc, d.comp, d.i, d.j, d.k) : sensor_val(g, f, sc, d.comp, d.i, d.j, d.k);
-  if (fq == 0) pr.series[(long long)pr.row * pr.n + p] = v;
-  if (pr.nfreq > 0) {
-    const double t = d.comp < 3 ? (double)(pr.step + 1) * pr.dt : ((double)pr.step + 0.5) * pr.dt;
-    double* acc = pr.dft + ((long long)p * pr.nfreq + fq) * 2;
-    double s, c;
-    sincos(pr.omega[fq] * t, &s, &c);
-    acc[0] += (double)v * c * pr.dt;
-    acc[1] += (double)v * s * pr.dt;
-  }
+__global__ void k_record(Grid g, Fields<STORE> f, Scales sc, Probes pr, int fields) {
+  record_thread(pr, blockIdx.x * (long long)blockDim.x + threadIdx.x, fields, [&](int comp, int i, int j, int k) {
+    const int ii = nbr(i, 0, g.nx, g.per[0]), jj = nbr(j, 0, g.ny, g.per[1]), kk = nbr(k, 0, g.nz, g.per[2]);
+    if (ii < 0 || jj < 0 || kk < 0) return 0.f;
+    const long long q = ii * g.sx + jj * g.sy + kk;
+    const int xq = STORE == 1 ? exact_idx(sc.xz, ii, jj, kk) : -1;
+    return comp < 3 ? ldx(f.E[comp], q, sc.ie[comp], sc.xz, comp, xq)
+                    : ldx(f.H[comp - 3], q, sc.ih[comp - 3], sc.xz, comp, xq);
+  });
 }
 
 __global__ void k_to_float_h(const __half* src, float inv, float* dst, long long n) {
@@ -954,14 +913,14 @@ void launch_soft(int store, const Grid&, const void* fields, const Scales& sc, c
   check_launch("k_soft");
 }
 
-void launch_record(int store, const Grid& g, const void* fields, const Scales& sc, const Probes& pr, hipStream_t st) {
+void launch_record(int store, const Grid& g, const void* fields, const Scales& sc, const Probes& pr, int which,
+                   hipStream_t st) {
   if (pr.n <= 0) return;
-  const long long threads = (long long)pr.n * (pr.nfreq > 0 ? pr.nfreq : 1);
-  const int nb = (int)((threads + 63) / 64);
+  const unsigned nb = (unsigned)((record_threads(pr) + 63) / 64);
   if (store == 0)
-    hipLaunchKernelGGL(k_record<0>, dim3(nb), dim3(64), 0, st, g, *static_cast<const Fields<0>*>(fields), sc, pr);
+    hipLaunchKernelGGL(k_record<0>, dim3(nb), dim3(64), 0, st, g, *static_cast<const Fields<0>*>(fields), sc, pr, which);
   else
-    hipLaunchKernelGGL(k_record<1>, dim3(nb), dim3(64), 0, st, g, *static_cast<const Fields<1>*>(fields), sc, pr);
+    hipLaunchKernelGGL(k_record<1>, dim3(nb), dim3(64), 0, st, g, *static_cast<const Fields<1>*>(fields), sc, pr, which);
   check_launch("k_record");
 }
 

@@ -78,6 +78,8 @@ struct dtm_solver {
   double* points[2] = {};          // a dipole's tables of incident values, by the parity of the half-step
   long long points_for[2] = {-1, -1};  // 2 n + half that each holds, within a call
   bool more = false;               // another forward step follows in this call
+  bool probes_e = false, probes_h = false;  // there are probes of E, of H components
+  Probes late{};                   // E probes of the last step, which the next H sweep records (n 0: none)
   int2* fold_w = nullptr;     // the sweeps' weights of that source, one entry per chunk of cells and half-step
   // device copies of the fused step's pointer table, one per buffer parity
   // (the old / new buffers swap every step), and their host images
@@ -1098,6 +1100,7 @@ static int start(dtm_solver* s) {
   if (np > 0) {
     if (int rc = dalloc(s, &s->probes_dev, sizeof(ProbeDesc) * np)) return rc;
     HIPCHK(hipMemcpy(s->probes_dev, s->probes.data(), sizeof(ProbeDesc) * np, hipMemcpyHostToDevice));
+    for (const ProbeDesc& d : s->probes) (d.comp < 3 ? s->probes_e : s->probes_h) = true;
     if (int rc = dalloc(s, &s->series_dev, sizeof(float) * (size_t)s->series_cap * np)) return rc;
     if (s->nfreq > 0)
       if (int rc = dalloc(s, &s->dft_dev, sizeof(double) * 2 * (size_t)np * s->nfreq)) return rc;
@@ -1185,7 +1188,25 @@ static int one_step(dtm_solver* s) {
   s->tf.active = (!s->adjoint && tfsf_gate(s, n)) ? 1 : 0;
   const void* F = fields_ptr(s);
   const bool rec = !s->adjoint && !s->replay;  // probes and flux record forward steps only
-  if (rec && s->fs.nface > 0) launch_flux_snap(s->store, s->g, F, s->sc, s->fs, s->stream);
+  const int np = rec ? (int)s->probes.size() : 0;
+  const int nf = rec ? s->fs.nface : 0;
+  // Probes ride with the two sweeps: the H probes of a step with its E sweep,
+  // its E probes with the next step's H sweep, or, at the end of a call or of
+  // a block of the series, with a launch of their own.
+  const bool ride = !s->torre && !s->timing && (long long)np * std::max(s->nfreq, 1) < (1 << 30);
+  Probes pr{};
+  if (np > 0) {
+    pr.n = np;
+    pr.desc = s->probes_dev;
+    pr.series = s->series_dev;
+    pr.row = s->series_row;
+    pr.nfreq = s->nfreq;
+    pr.omega = s->omega_dev;
+    pr.dft = s->dft_dev;
+    pr.dt = c.dt;
+    pr.step = n;
+  }
+  if (nf > 0) launch_flux_snap(s->store, s->g, F, s->sc, s->fs, s->stream);
   const double th = (double)n * c.dt, te = ((double)n + 0.5) * c.dt;
   if (s->torre) {
     // A plane wave along x is folded into the fused step (both half-steps'
@@ -1221,7 +1242,8 @@ static int one_step(dtm_solver* s) {
     if (s->tf.active) tfh = tfsf_for(s, n, 0);
     ev_begin(s, 0);
     launch_sweep(0, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 0) : nullptr,
-                 s->fold_w, s->stream);
+                 s->fold_w, s->late.n > 0 ? &s->late : nullptr, s->stream);
+    s->late.n = 0;
     ev_end(s);
     if (s->tf.active && !fold) {
       ev_begin(s, 4);
@@ -1233,7 +1255,7 @@ static int one_step(dtm_solver* s) {
     if (s->tf.active) tfe = tfsf_for(s, n, 1);
     ev_begin(s, 2);
     launch_sweep(1, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 1) : nullptr,
-                 s->fold_w, s->stream);
+                 s->fold_w, ride && s->probes_h ? &pr : nullptr, s->stream);
     ev_end(s);
     ev_begin(s, 4);
     launch_ade(s->store, s->g, F, F, s->sc, s->mt, s->ade, s->stream);
@@ -1264,21 +1286,12 @@ static int one_step(dtm_solver* s) {
     }
     launch_soft(s->store, s->g, F, s->sc, so, s->stream);
   }
-  const int np = rec ? (int)s->probes.size() : 0;
-  const int nf = rec ? s->fs.nface : 0;
   if (nf > 0) launch_flux(s->store, s->g, F, s->sc, s->fs, s->series_row, c.dt, s->stream);
   if (np > 0) {
-    Probes pr{};
-    pr.n = np;
-    pr.desc = s->probes_dev;
-    pr.series = s->series_dev;
-    pr.row = s->series_row;
-    pr.nfreq = s->nfreq;
-    pr.omega = s->omega_dev;
-    pr.dft = s->dft_dev;
-    pr.dt = c.dt;
-    pr.step = n;
-    launch_record(s->store, s->g, F, s->sc, pr, s->stream);
+    const bool later = ride && s->more && s->series_row + 1 < s->series_cap;
+    if (later) s->late = s->probes_e ? pr : Probes{};
+    const int which = (s->probes_e && !later ? 1 : 0) | (s->probes_h && !ride ? 2 : 0);
+    if (which) launch_record(s->store, s->g, F, s->sc, pr, which, s->stream);
   }
   ev_end(s);
   if (int rc = launch_result()) return rc;
@@ -1293,6 +1306,7 @@ static int one_step(dtm_solver* s) {
 
 static int run_steps(dtm_solver* s, int nsteps) {
   s->points_for[0] = s->points_for[1] = -1;
+  s->late.n = 0;
   for (int t = 0; t < nsteps; t++) {
     s->more = t + 1 < nsteps;
     if (int rc = one_step(s)) return rc;

@@ -43,6 +43,7 @@
 #include <type_traits>
 
 #include "dtm_internal.h"
+#include "dtm_probe.h"
 
 namespace dtm {
 
@@ -94,6 +95,7 @@ struct SweepArgs {
     float* curl[3];
   } ade;
   Exact xz;
+  Probes pr;  // probes of src, recorded by the blocks after the sweep's
 };
 using ArgsK = __attribute__((address_space(4))) const SweepArgs;
 // The kernel's own argument block, behind a pointer the compiler cannot see
@@ -269,6 +271,22 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
   constexpr bool HALF = STORE == 1 && !XZ;     // differences in stored units
   constexpr int CS = UP ? 3 : 0, CD = UP ? 0 : 3;  // first source and destination component (Ex .. Hz)
   const int blk = blockIdx.x;
+  // Probes of the field that this launch only reads: blocks of their own beside
+  // the sweep's (a launch of their own took 3 us of a 48x40x40 step's 18, and
+  // 4.6 us where 64 bins are summed).
+  if (blk >= A.sw.per * NXCD) {
+    record_thread(A.pr, (blk - A.sw.per * NXCD) * 64LL + threadIdx.x, 1 << UP,
+                  [&](int comp, int i, int j, int k) -> float {
+                    const int ii = nbr(i, A.nx, A.per[0]), jj = nbr(j, A.ny, A.per[1]), kk = nbr(k, A.nz, A.per[2]);
+                    if (ii < 0 || jj < 0 || kk < 0) return 0.f;
+                    const int xq = STORE == 1 ? exact_idx(A.xz, ii, jj, kk) : -1;
+                    if (xq >= 0) return A.xz.f[comp][xq];
+                    const char* p = A.set + A.comp * comp + (ii * A.sx + (long long)jj * A.nz + kk) * (STORE ? 2 : 4);
+                    if constexpr (STORE == 0) return *reinterpret_cast<const float*>(p);
+                    else return (float)*reinterpret_cast<const _Float16*>(p) * A.isrc[UP ? comp - 3 : comp];
+                  });
+    return;
+  }
   int lid = (blk % NXCD) * A.sw.per + blk / NXCD;  // XCD-contiguous
   if (lid >= A.sw.total[2]) return;
   int nlb = A.sw.lb1 - A.sw.lb0, lo = A.sw.i0, hi = A.sw.h0;
@@ -884,8 +902,9 @@ void go(SweepArgs& A, hipStream_t st) {
   w.total[1] = (int)(n[0] + n[1]);
   w.total[2] = (int)blocks;
   w.per = (w.total[2] + NXCD - 1) / NXCD;
-  if (blocks == 0) return;
-  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD>), dim3(w.per * NXCD), dim3(64), 0, st, A);
+  const int more = (int)((record_threads(A.pr) + 63) / 64);
+  if (blocks == 0 && more == 0) return;
+  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD>), dim3(w.per * NXCD + more), dim3(64), 0, st, A);
   note_launch(UP ? "k_sweep E" : "k_sweep H");
 }
 
@@ -989,8 +1008,9 @@ void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t s
 
 void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                   const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
-                  hipStream_t st) {
+                  const Probes* pr, hipStream_t st) {
   SweepArgs A{};
+  if (pr) A.pr = *pr;
   A.fold = fold;
   A.foldw = foldw ? foldw + (up ? fold_weights_size(g) / 2 : 0) : nullptr;
   A.mt = mt;
@@ -1031,6 +1051,7 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
     w.hb0 = g.per[1] ? 0 : (int)((long long)std::max(x.j0 - 3, 0) * w.nzv / 64);
     w.hb1 = g.per[1] ? nlb : (int)(((long long)std::min(x.j1 + 3, g.ny) * w.nzv + 63) / 64);
     part(i0, i1, 0, nlb, false);
+    A.pr.n = 0;
     const int a = w.h0, b = w.h1, b0 = w.hb0, b1 = w.hb1;
     w.h0 = w.h1 = b;
     w.hb0 = w.hb1 = b1;
