@@ -598,7 +598,7 @@ static int setup_cpml(dtm_solver* s) {
     }
     float* t[4];
     for (int q = 0; q < 4; q++)
-      if (int rc = dalloc(s, &t[q], sizeof(float) * n[a])) return rc;
+      if (int rc = dalloc(s, &t[q], sizeof(float) * (n[a] + 4))) return rc;  // the sweeps read four at once
     HIPCHK(hipMemcpy(t[0], bE.data(), sizeof(float) * n[a], hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(t[1], cE.data(), sizeof(float) * n[a], hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(t[2], bH.data(), sizeof(float) * n[a], hipMemcpyHostToDevice));

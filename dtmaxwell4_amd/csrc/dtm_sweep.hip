@@ -30,11 +30,11 @@
 // Bounds and figures (us a step of both sweeps, plane wave on a sphere, CPML;
 // in brackets the sweeps before these: 64 x 8 or 16 column tiles in LDS with a
 // barrier per plane, one cell per lane):
-//   512x256x256 FP32  572 (591)  HBM: 73 B/cell and psi at 4.6 TB/s, a copy 4.7-5.3
-//               FP16  370 (477)  HBM and issue: 37 B/cell and psi at 3.7 TB/s
-//   200^3       FP32  131 (161)  FP16  91 (152)  fields partly, or all, in the Infinity Cache
-//   128^3       FP32   43  (57)  FP16  36  (53)  one or two rounds of waves: latency and issue
-//    64^3       FP32   17  (33)  FP16  18  (35)  two launches of one plane per wave: latency
+//   512x256x256 FP32  565 (591)  HBM: 73 B/cell and psi at 4.8 TB/s, a copy 4.7-5.3
+//               FP16  356 (477)  HBM and issue: 37 B/cell and psi at 4.2 TB/s
+//   200^3       FP32  122 (161)  FP16  82 (152)  fields partly, or all, in the Infinity Cache
+//   128^3       FP32   38  (57)  FP16  31  (53)  one or two rounds of waves: latency and issue
+//    64^3       FP32   13  (33)  FP16  14  (35)  two launches of one plane per wave: latency
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -313,6 +313,65 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
   const int nz = A.nz, perz = A.per[2];
   const O cell = (O)j * (O)nz + (O)k;
   const O own = act ? cell * ES : OUT;
+  const int nx = A.nx, perx = A.per[0];
+  auto plane = [&](int p) -> int { return nbr(p, nx, perx); };
+  // plane p of component c (Ex .. Hz); outside the grid: empty.  A lane reads
+  // whole chunks: the last one of an array reaches into its pad (kPad).
+  auto at = [&](int p, int c) -> Plane<AD> {
+    const long long o = (long long)max(p, 0) * A.sx * (long long)ES;
+    if constexpr (AD == kNear) return span<AD>(A.set, o, p < 0 ? 0 : kBytes, (unsigned)A.comp * (unsigned)c);
+    else return span<AD>(A.set, o + (long long)A.comp * c, p < 0 ? 0 : (unsigned long long)(A.sx + NV) * ES);
+  };
+
+  // A wave's first loads (fold weights, layer coefficients, the queues) go out
+  // before the rest of its start is worked out, without a branch, in the order
+  // of their use: waiting for one after the other took 1.3 of 13.9 us a step at
+  // 64^3 and 1.6 of 39 at 128^3.
+  // packed TF/SF weights of the cells (k_fold_weights)
+  int fz = 0, fi = 0;
+  if constexpr (TF) {
+    const u2 w = ldt<u2>(span<AD>(A.foldw, 0, A.fold ? (unsigned long long)A.sw.NL * 8 : 0), act ? (O)L * 8u : OUT);
+    fz = (int)w[0];
+    fi = (int)w[1];
+  }
+  // Cells of the chunk in a z slab (bit q).
+  const int zl = A.plo[2], zh = A.phi[2], yl = A.plo[1], yh = A.phi[1];
+  const int Pz = zl + zh;
+  const int zin = min(max(zl - k, 0), NV), zout = min(max(nz - zh - k, 0), NV);
+  unsigned zm = (((1u << zin) - 1u) | ~((1u << zout) - 1u)) & ((1u << min(NV, nz - k)) - 1u);
+  zm = act ? zm : 0u;
+  const bool zwave = __builtin_amdgcn_ballot_w64(zm != 0) != 0;
+  // (a chunk that reaches into both slabs over a gap has no place in psi)
+  const bool zboth = !SP && A.sw.zgap > 0 && A.sw.zgap < 3;
+  const bool zslab = !SP && zwave && !zboth;
+  const int yup = j - (A.ny - yh);
+  int yslab = j < yl ? j : yup >= 0 ? yl + yup : -1;  // the row's place in the y slabs
+  yslab = act ? yslab : -1;
+  const int ysl = SP ? -1 : yslab;
+  const bool sy = SP && yslab >= 0;
+  const bool ywave = __builtin_amdgcn_ballot_w64(yslab >= 0) != 0;
+  F zb = {}, zc = {};
+  float by = 0.f, cy = 0.f;
+  if constexpr (!SP) {
+    if (zslab) {  // (NV floats follow the coefficients: setup_cpml)
+      const O o = zm != 0 ? (O)k * 4u : OUT;
+      zb = ldt<F>(span<AD>(A.b[2], 0, (unsigned long long)(nz + NV) * 4), o);
+      zc = ldt<F>(span<AD>(A.c[2], 0, (unsigned long long)(nz + NV) * 4), o);
+    }
+    if (ywave) {
+      const O o = ysl >= 0 ? (O)j * 4u : OUT;
+      by = ldt<float>(span<AD>(A.b[1], 0, (unsigned long long)A.ny * 4), o);
+      cy = ldt<float>(span<AD>(A.c[1], 0, (unsigned long long)A.ny * 4), o);
+    }
+  }
+  // queues of the source's y and z components: sample q of plane i is plane i-OWN+q
+  V qy[4], qz[4];
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    const int p = plane(p0 - OWN + q);
+    qy[q] = ldw<STORE, XZ>(at(p, CS + 1), own, A.isrc[1]);
+    qz[q] = ldw<STORE, XZ>(at(p, CS + 2), own, A.isrc[2]);
+  }
   auto row = [&](int dj) -> O {
     const int jj = nbr(j + dj, A.ny, A.per[1]);
     return (act && jj >= 0) ? ((O)jj * (O)nz + (O)k) * ES : OUT;
@@ -335,16 +394,6 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
 #pragma unroll
     for (int t = 0; t < 2; t++) oh[t] = zhi ? zoff(ke + t) : OUT;
   }
-  const int nx = A.nx, perx = A.per[0];
-  auto plane = [&](int p) -> int { return nbr(p, nx, perx); };
-  // plane p of component c (Ex .. Hz); outside the grid: empty.  A lane reads
-  // whole chunks: the last one of an array reaches into its pad (kPad).
-  auto at = [&](int p, int c) -> Plane<AD> {
-    const long long o = (long long)max(p, 0) * A.sx * (long long)ES;
-    if constexpr (AD == kNear) return span<AD>(A.set, o, p < 0 ? 0 : kBytes, (unsigned)A.comp * (unsigned)c);
-    else return span<AD>(A.set, o + (long long)A.comp * c, p < 0 ? 0 : (unsigned long long)(A.sx + NV) * ES);
-  };
-
   // FP32 zone: values of zone cells come from their FP32 copies
   bool xwave = false;  // the rows and columns that the wave reads meet the zone
   if constexpr (XZ) {
@@ -389,47 +438,21 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
     }
   };
 
-  // absorbing layer, this lane's part
-  const int ysl = (!SP && A.pml && act) ? slab_index(j, A.ny, A.plo[1], A.phi[1]) : -1;
-  const bool sy = SP && A.pml && act && slab_index(j, A.ny, A.plo[1], A.phi[1]) >= 0;
-  const bool ywave = __builtin_amdgcn_ballot_w64(ysl >= 0 || sy) != 0;
+  // places in psi: of the row, and of the chunk's first cell, where it is or
+  // would be: the cells of a slab are contiguous there
   const O oy = ysl >= 0 ? ((O)ysl * (O)nz + (O)k) * 4u : OUT;
-  const float by = ysl >= 0 ? A.b[1][j] : 0.f, cy = ysl >= 0 ? A.c[1][j] : 0.f;
-  // cells of the chunk in a z slab (bit q), and where psi of the chunk's first
-  // cell is or would be: the cells of a slab are contiguous there
-  unsigned zm = 0;
-#pragma unroll
-  for (int q = 0; q < NV; q++)
-    if (A.pml && act && q < nv && slab_index(k + q, nz, A.plo[2], A.phi[2]) >= 0) zm |= 1u << q;
-  const bool zwave = __builtin_amdgcn_ballot_w64(zm != 0) != 0;
-  // (a chunk that reaches into both slabs over a gap has no such place)
-  const bool zboth = !SP && A.sw.zgap > 0 && A.sw.zgap < 3;
-  const bool zslab = !SP && zwave && !zboth;
-  const int Pz = A.plo[2] + A.phi[2];
-  const O oz = zm != 0 ? (O)((long long)j * Pz + (k < A.plo[2] ? k : k - A.sw.zgap) + (int)kFront) * 4u : OUT;
+  const O oz = zm != 0 ? (O)((long long)j * Pz + (k < zl ? k : k - A.sw.zgap) + (int)kFront) * 4u : OUT;
   // z coefficients of the layer wait in the lane's own LDS slot (nothing is shared)
   __shared__ F lcoef[SP ? 1 : 2][SP ? 1 : 64];
   if constexpr (!SP) {
     if (zslab && zm != 0) {
-      F b, c;
-#pragma unroll
-      for (int q = 0; q < NV; q++) {
-        b[q] = A.b[2][min(k + q, nz - 1)];
-        c[q] = A.c[2][min(k + q, nz - 1)];
-      }
-      lcoef[0][lane] = b;
-      lcoef[SP ? 0 : 1][lane] = c;
+      lcoef[0][lane] = zb;
+      lcoef[SP ? 0 : 1][lane] = zc;
     }
   }
-  // TF/SF fold: packed weights of the cells (k_fold_weights), and which kinds occur in the wave
-  int fz = 0, fi = 0;
+  // which kinds of TF/SF weights occur in the wave
   bool twy = false, twz = false, twx = false;
   if constexpr (TF) {
-    if (act && A.fold) {
-      const int2 w = A.foldw[(long long)j * A.sw.nzv + kc];
-      fz = w.x;
-      fi = w.y;
-    }
     twy = __builtin_amdgcn_ballot_w64((fz & 0x3f000000) != 0) != 0;
     twz = __builtin_amdgcn_ballot_w64((fz & 0x00ffffff) != 0) != 0;
     twx = __builtin_amdgcn_ballot_w64((fi & 0x3fc00) != 0) != 0;
@@ -444,16 +467,11 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
 
   float one = 1.0f;
   if constexpr (HALF) asm volatile("" : "+s"(one));
-  // queues of the source's y and z components: sample q of plane i is plane i-OWN+q
-  V qy[4], qz[4];
+  if (XZ && xwave) {
 #pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const int p = plane(p0 - OWN + q);
-    qy[q] = ldw<STORE, XZ>(at(p, CS + 1), own, A.isrc[1]);
-    qz[q] = ldw<STORE, XZ>(at(p, CS + 2), own, A.isrc[2]);
-    if (XZ && xwave) {
-      zone(qy[q], CS + 1, p, 0);
-      zone(qz[q], CS + 2, p, 0);
+    for (int q = 0; q < 3; q++) {
+      zone(qy[q], CS + 1, plane(p0 - OWN + q), 0);
+      zone(qz[q], CS + 2, plane(p0 - OWN + q), 0);
     }
   }
 
@@ -920,7 +938,8 @@ void pick(SweepArgs& A, bool split, hipStream_t st) {
   if (w.i1 <= w.i0) return;
   // (offsets in a plane, of fields and of psi, as the descriptors can span them)
   const bool huge = (unsigned long long)(A.sx + 64) * 4 >= kBytes ||
-                    ((unsigned long long)A.ny * (A.plo[2] + A.phi[2]) + 64) * 4 >= kBytes;
+                    ((unsigned long long)A.ny * (A.plo[2] + A.phi[2]) + 64) * 4 >= kBytes ||
+                    (unsigned long long)w.NL * sizeof(int2) >= kBytes;
   const bool far = 6 * A.comp >= kBytes;
   const bool plain = w.rag == 0 && !A.per[2] && 64 % w.nzv == 0;
   if (huge || (XZ && far)) {
