@@ -274,13 +274,17 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
   // Probes of the field that this launch only reads: blocks of their own beside
   // the sweep's (a launch of their own took 3 us of a 48x40x40 step's 18, and
   // 4.6 us where 64 bins are summed).
-  if (blk >= A.sw.per * NXCD) {
+  // (The zone's variants have none, the plain launch before them does: with the
+  // recorder in it the compiler kept the arguments of one in scratch memory and
+  // spilled 54 registers, 38 us for 13.)
+  if (!XZ && blk >= A.sw.per * NXCD) {
+    const ArgsK* C = again();
     record_thread(A.pr, (blk - A.sw.per * NXCD) * 64LL + threadIdx.x, 1 << UP,
                   [&](int comp, int i, int j, int k) -> float {
                     const int ii = nbr(i, A.nx, A.per[0]), jj = nbr(j, A.ny, A.per[1]), kk = nbr(k, A.nz, A.per[2]);
                     if (ii < 0 || jj < 0 || kk < 0) return 0.f;
                     const int xq = STORE == 1 ? exact_idx(A.xz, ii, jj, kk) : -1;
-                    if (xq >= 0) return A.xz.f[comp][xq];
+                    if (xq >= 0) return C->xz.f[comp][xq];
                     const char* p = A.set + A.comp * comp + (ii * A.sx + (long long)jj * A.nz + kk) * (STORE ? 2 : 4);
                     if constexpr (STORE == 0) return *reinterpret_cast<const float*>(p);
                     else return (float)*reinterpret_cast<const _Float16*>(p) * A.isrc[UP ? comp - 3 : comp];
