@@ -312,6 +312,7 @@ struct FluxSet {
   double* total;   // [face], running sum of flux * dt
 };
 
+constexpr int kSweepSoft = 4;
 struct Soft {
   int n;
   int comp[16];
@@ -335,11 +336,12 @@ int take_launch_error(char* msg, int cap);
 // fold non-null: add a plane-wave TF/SF source along x inside the sweep, from
 // this half-step's per-plane factors (launch_tfsf_fold) and the weights of
 // every chunk of cells (launch_fold_weights); none with an FP32 zone.
+// soft non-null (up 1): at most kSweepSoft sources, subtracted from the new E.
 // pr non-null: the launch also records the probes of the field that it only
 // reads (up 0: E as it is before the step, up 1: the new H).
 void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                   const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
-                  const Probes* pr, hipStream_t st);
+                  const Probes* pr, const Soft* soft, hipStream_t st);
 // entries of the weights, both half-steps
 long long fold_weights_size(const Grid& g);
 void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t st);

@@ -1182,6 +1182,31 @@ static const TorreCold* torre_cold(dtm_solver* s) {
   return s->cold_dev[k];
 }
 
+// The soft sources' contributions to E of step n.
+static void soft_values(const dtm_solver* s, long long n, Soft& so) {
+  const dtm_config& c = s->cfg;
+  so.n = c.nsoft;
+  const double th = ((double)n + 0.5) * c.dt;
+  for (int q = 0; q < c.nsoft; q++) {
+    const dtm_soft_source& ss = c.soft[q];
+    const size_t idx = ((size_t)ss.i * c.ny + ss.j) * c.nz + ss.k;
+    const ClassEntry& ce = s->classes[cls_of(s, idx)];
+    double ie = ce.inv_eps[ss.comp];
+    if (s->mt.d_on) {
+      const int di = ss.i - s->mt.d_i0, dj = ss.j - s->mt.d_j0, dk = ss.k - s->mt.d_k0;
+      if (di >= 0 && di < s->mt.d_ni && dj >= 0 && dj < s->mt.d_nj && dk >= 0 && dk < s->mt.d_nk)
+        ie = s->design_host[((size_t)di * s->mt.d_nj + dj) * s->mt.d_nk + dk];
+    }
+    const double J = ss.amp * wave_value(ss.waveform, ss.w, ss.kEnv, ss.t0, ss.tw, th);
+    so.comp[q] = ss.comp;
+    so.q[q] = (long long)idx;
+    so.ijk[q][0] = ss.i;
+    so.ijk[q][1] = ss.j;
+    so.ijk[q][2] = ss.k;
+    so.val[q] = (float)(c.dt * ie * J);
+  }
+}
+
 static int one_step(dtm_solver* s) {
   const dtm_config& c = s->cfg;
   const long long n = s->step;
@@ -1206,6 +1231,11 @@ static int one_step(dtm_solver* s) {
     pr.dt = c.dt;
     pr.step = n;
   }
+  // Soft sources go into the E sweep, unless it does not run or k_tfsf adds to
+  // the new E first.
+  Soft so{};
+  bool so_in = false;
+  if (c.nsoft > 0 && !s->adjoint) soft_values(s, n, so);
   if (nf > 0) launch_flux_snap(s->store, s->g, F, s->sc, s->fs, s->stream);
   const double th = (double)n * c.dt, te = ((double)n + 0.5) * c.dt;
   if (s->torre) {
@@ -1242,7 +1272,7 @@ static int one_step(dtm_solver* s) {
     if (s->tf.active) tfh = tfsf_for(s, n, 0);
     ev_begin(s, 0);
     launch_sweep(0, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 0) : nullptr,
-                 s->fold_w, s->late.n > 0 ? &s->late : nullptr, s->stream);
+                 s->fold_w, s->late.n > 0 ? &s->late : nullptr, nullptr, s->stream);
     s->late.n = 0;
     ev_end(s);
     if (s->tf.active && !fold) {
@@ -1253,39 +1283,17 @@ static int one_step(dtm_solver* s) {
     // E half-step: incident H at t = (n+1/2) dt (genAlg.py:499)
     Tfsf tfe{};
     if (s->tf.active) tfe = tfsf_for(s, n, 1);
+    so_in = so.n > 0 && so.n <= kSweepSoft && (fold || !s->tf.active);
     ev_begin(s, 2);
     launch_sweep(1, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, 0, c.nx, fold ? fold_for(s, n, 1) : nullptr,
-                 s->fold_w, ride && s->probes_h ? &pr : nullptr, s->stream);
+                 s->fold_w, ride && s->probes_h ? &pr : nullptr, so_in ? &so : nullptr, s->stream);
     ev_end(s);
     ev_begin(s, 4);
     launch_ade(s->store, s->g, F, F, s->sc, s->mt, s->ade, s->stream);
     if (s->tf.active && !fold)
       launch_tfsf(s->store, 1, s->g, F, s->sc, s->pm, s->mt, s->ade, tfe, s->bands, te, s->stream);
   }
-  if (c.nsoft > 0 && !s->adjoint) {
-    Soft so{};
-    so.n = c.nsoft;
-    const double th = ((double)n + 0.5) * c.dt;
-    for (int q = 0; q < c.nsoft; q++) {
-      const dtm_soft_source& ss = c.soft[q];
-      const size_t idx = ((size_t)ss.i * c.ny + ss.j) * c.nz + ss.k;
-      const ClassEntry& ce = s->classes[cls_of(s, idx)];
-      double ie = ce.inv_eps[ss.comp];
-      if (s->mt.d_on) {
-        const int di = ss.i - s->mt.d_i0, dj = ss.j - s->mt.d_j0, dk = ss.k - s->mt.d_k0;
-        if (di >= 0 && di < s->mt.d_ni && dj >= 0 && dj < s->mt.d_nj && dk >= 0 && dk < s->mt.d_nk)
-          ie = s->design_host[((size_t)di * s->mt.d_nj + dj) * s->mt.d_nk + dk];
-      }
-      const double J = ss.amp * wave_value(ss.waveform, ss.w, ss.kEnv, ss.t0, ss.tw, th);
-      so.comp[q] = ss.comp;
-      so.q[q] = (long long)idx;
-      so.ijk[q][0] = ss.i;
-      so.ijk[q][1] = ss.j;
-      so.ijk[q][2] = ss.k;
-      so.val[q] = (float)(c.dt * ie * J);
-    }
-    launch_soft(s->store, s->g, F, s->sc, so, s->stream);
-  }
+  if (so.n > 0 && !so_in) launch_soft(s->store, s->g, F, s->sc, so, s->stream);
   if (nf > 0) launch_flux(s->store, s->g, F, s->sc, s->fs, s->series_row, c.dt, s->stream);
   if (np > 0) {
     const bool later = ride && s->more && s->series_row + 1 < s->series_cap;

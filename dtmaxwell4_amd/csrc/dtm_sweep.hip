@@ -70,6 +70,14 @@ struct Sweep {
   int per, total[3];    // blocks per XCD, and in all
   int zgap;             // cells between the two z slabs
 };
+// Soft sources that the E sweep subtracts from its new values.
+struct SweepSoft {
+  int lo, hi;  // their x planes lie in [lo, hi)
+  int n;
+  int i[kSweepSoft], q[kSweepSoft], comp[kSweepSoft];  // plane, cell of its chunk, component
+  long long cell[kSweepSoft];                            // the chunk's first cell in the plane
+  float val[kSweepSoft];
+};
 // The arguments of one half-step: the scales of the three components the curl
 // is taken of (src) and of the three it updates (dst), and of the absorbing
 // layer the parts that belong to dst.
@@ -95,6 +103,7 @@ struct SweepArgs {
     float* curl[3];
   } ade;
   Exact xz;
+  SweepSoft soft;
   Probes pr;  // probes of src, recorded by the blocks after the sweep's
 };
 using ArgsK = __attribute__((address_space(4))) const SweepArgs;
@@ -857,6 +866,24 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
         if (sany && ((in >> q) & 1u)) split(q, k0, k1, k2);
       }
     }
+    if constexpr (UP && STORE == 0 && !TF) {  // launch_sweep: soft_in
+      if (i >= A.soft.lo && i < A.soft.hi) {
+        const ArgsK* C = again();
+        for (int t = 0; t < C->soft.n; t++) {
+          if (C->soft.i[t] != i || own != (O)C->soft.cell[t] * ES) continue;
+          const int at = C->soft.q[t], comp = C->soft.comp[t];
+          const float val = C->soft.val[t];
+          auto take = [&](F& v, int c) {
+#pragma unroll
+            for (int q = 0; q < NV; q++)
+              if (comp == c && at == q) v[q] -= val;
+          };
+          take(n0, 0);
+          take(n1, 1);
+          take(n2, 2);
+        }
+      }
+    }
     if constexpr (XZ) {
       if (xwave && i >= A.xz.i0 && i < A.xz.i1) {  // new values of zone cells to the FP32 copy too
 #pragma unroll
@@ -946,6 +973,15 @@ void go(SweepArgs& A, hipStream_t st) {
   note_launch(UP ? "k_sweep E" : "k_sweep H");
 }
 
+// What the descriptors can span of a plane, of its psi and weights, and of the field set.
+int addressing(const SweepArgs& A) {
+  if ((unsigned long long)(A.sx + 64) * 4 >= kBytes ||
+      ((unsigned long long)A.ny * (A.plo[2] + A.phi[2]) + 64) * 4 >= kBytes ||
+      (unsigned long long)A.sw.NL * sizeof(int2) >= kBytes)
+    return kHuge;
+  return 6 * A.comp >= kBytes ? kFar : kNear;
+}
+
 // The variant of a configuration.  The plain ones (no GEN) need rows that fill
 // a wave or a whole fraction of it and a z axis without wrap-around; the far
 // and huge ones and those of the split layer and the zone are built for the
@@ -956,11 +992,8 @@ void pick(SweepArgs& A, bool split, hipStream_t st) {
   w.rag = A.nz % NV;
   w.zgap = A.nz - A.phi[2] - A.plo[2];
   if (w.i1 <= w.i0) return;
-  // (offsets in a plane, of fields and of psi, as the descriptors can span them)
-  const bool huge = (unsigned long long)(A.sx + 64) * 4 >= kBytes ||
-                    ((unsigned long long)A.ny * (A.plo[2] + A.phi[2]) + 64) * 4 >= kBytes ||
-                    (unsigned long long)w.NL * sizeof(int2) >= kBytes;
-  const bool far = 6 * A.comp >= kBytes;
+  const int ad = addressing(A);
+  const bool huge = ad == kHuge, far = ad == kFar;
   const bool plain = w.rag == 0 && !A.per[2] && 64 % w.nzv == 0;
   if (huge || (XZ && far)) {
     if (split) go<UP, STORE, true, true, !XZ, XZ, kHuge>(A, st);
@@ -1047,7 +1080,7 @@ void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t s
 
 void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                   const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
-                  const Probes* pr, hipStream_t st) {
+                  const Probes* pr, const Soft* soft, hipStream_t st) {
   SweepArgs A{};
   if (pr) A.pr = *pr;
   A.fold = fold;
@@ -1064,14 +1097,33 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   w.nzv = (g.nz + NV - 1) / NV;
   w.NL = (long long)w.nzv * g.ny;
   const int nlb = (int)((w.NL + 63) / 64);
+  if (store) fill<1>(A, up, false, g, fields, sc, pm);
+  else fill<0>(A, up, false, g, fields, sc, pm);
+  // Soft sources are subtracted where E is new in the plain FP32 variants:
+  // k_soft's launch took 1.8 of 36 us a step at 128^3.  In the variants with the
+  // fold or in half storage the few registers this takes made spills that cost
+  // every step 2 to 4%: there k_soft follows.
+  const bool soft_in = soft && soft->n <= kSweepSoft && store == 0 && !fold && !split && addressing(A) == kNear;
+  if (soft_in) {
+    A.soft.lo = g.nx;
+    A.soft.n = soft->n;
+    for (int t = 0; t < soft->n; t++) {
+      A.soft.i[t] = soft->ijk[t][0];
+      A.soft.q[t] = soft->ijk[t][2] % NV;
+      A.soft.cell[t] = (long long)soft->ijk[t][1] * g.nz + soft->ijk[t][2] / NV * NV;
+      A.soft.comp[t] = soft->comp[t];
+      A.soft.val[t] = soft->val[t];
+      A.soft.lo = std::min(A.soft.lo, soft->ijk[t][0]);
+      A.soft.hi = std::max(A.soft.hi, soft->ijk[t][0] + 1);
+    }
+  }
   // blocks [b0, b1) of the planes [a, b), without the hole set in w
   auto part = [&](int a, int b, int b0, int b1, bool zone) {
     w.i0 = a;
     w.i1 = b;
     w.lb0 = b0;
     w.lb1 = b1;
-    if (store) fill<1>(A, up, zone, g, fields, sc, pm);
-    else fill<0>(A, up, false, g, fields, sc, pm);
+    if (zone) fill<1>(A, up, true, g, fields, sc, pm);
     if (zone) up ? pick<1, 1, true>(A, split, st) : pick<0, 1, true>(A, split, st);
     else if (store) up ? pick<1, 1, false>(A, split, st) : pick<0, 1, false>(A, split, st);
     else up ? pick<1, 0, false>(A, split, st) : pick<0, 0, false>(A, split, st);
@@ -1098,6 +1150,7 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   } else {
     part(i0, i1, 0, nlb, false);
   }
+  if (soft && !soft_in) launch_soft(store, g, fields, sc, *soft, st);
 }
 
 }  // namespace dtm
