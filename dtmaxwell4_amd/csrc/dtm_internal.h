@@ -292,6 +292,7 @@ struct Probes {
   double* dft;  // [n][nfreq][2]
   double dt;
   long long step;
+  int i0, i1;  // the probes of these x planes
 };
 
 // Poynting-flux faces (dtm_flux.hip).  Face normal to axis a on the H plane
@@ -336,7 +337,7 @@ int take_launch_error(char* msg, int cap);
 // fold non-null: add a plane-wave TF/SF source along x inside the sweep, from
 // this half-step's per-plane factors (launch_tfsf_fold) and the weights of
 // every chunk of cells (launch_fold_weights); none with an FP32 zone.
-// soft non-null (up 1): at most kSweepSoft sources, subtracted from the new E.
+// soft non-null (up 1): sources, those of the planes subtracted from the new E.
 // pr non-null: the launch also records the probes of the field that it only
 // reads (up 0: E as it is before the step, up 1: the new H).
 void launch_sweep(int up, int store, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,

@@ -37,7 +37,7 @@ __device__ __forceinline__ void record_thread(const Probes& pr, long long tid, i
     fq = (int)((unsigned)tid % (unsigned)nb);
   }
   const ProbeDesc d = pr.desc[p];
-  if (!(fields & (d.comp < 3 ? 1 : 2))) return;
+  if (!(fields & (d.comp < 3 ? 1 : 2)) || d.i < pr.i0 || d.i >= pr.i1) return;
   const float v = d.kind == 0 ? get(d.comp, d.i, d.j, d.k) : sensor_val(get, d.comp, d.i, d.j, d.k);
   if (fq == 0) pr.series[(long long)pr.row * pr.n + p] = v;
   if (pr.nfreq > 0) {

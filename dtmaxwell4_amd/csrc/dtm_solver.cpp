@@ -28,6 +28,15 @@
 using namespace dtm;
 
 static thread_local std::string g_err;
+// Time skewing (skewed_steps): a state up to kCacheResident bytes stays in the
+// Infinity Cache (256 MB) by itself; kCacheSlab is what a slab may take of it.
+// Measured, us a step, one step at a time and skewed: FP32 200^3 (238 MB) 127
+// and 127, 207^3 (263 MB) 166 and 155, 256^3 301 and 272; 512x256x256 FP32 567,
+// and 544 / 532 / 541 / 593 in slabs of 48 / 80 / 96 / 128 planes (85, 142, 170
+// and 226 MB), FP16 353, and 361 / 340 / 325 / 328 / 378 in slabs of 64 / 96 /
+// 128 / 192 / 256 (63, 94, 126, 189 and 252 MB): smaller ones leave the chip's
+// last round of waves emptier, larger ones leave the cache.
+static constexpr double kCacheResident = 245e6, kCacheSlab = 170e6;
 static constexpr int kTableSteps = 32;  // plane-wave waveform tables per batch
 
 static int fail(int code, const std::string& msg) {
@@ -1207,6 +1216,25 @@ static void soft_values(const dtm_solver* s, long long n, Soft& so) {
   }
 }
 
+// The probes on the x planes [i0, i1), for step n into row `row` of the series
+// (n = 0: none there).
+static Probes probes_of(const dtm_solver* s, long long n, int row, int i0, int i1) {
+  Probes pr{};
+  for (const ProbeDesc& d : s->probes)
+    if (d.i >= i0 && d.i < i1) pr.n = (int)s->probes.size();
+  pr.desc = s->probes_dev;
+  pr.series = s->series_dev;
+  pr.row = row;
+  pr.nfreq = s->nfreq;
+  pr.omega = s->omega_dev;
+  pr.dft = s->dft_dev;
+  pr.dt = s->cfg.dt;
+  pr.step = n;
+  pr.i0 = i0;
+  pr.i1 = i1;
+  return pr;
+}
+
 static int one_step(dtm_solver* s) {
   const dtm_config& c = s->cfg;
   const long long n = s->step;
@@ -1219,18 +1247,7 @@ static int one_step(dtm_solver* s) {
   // its E probes with the next step's H sweep, or, at the end of a call or of
   // a block of the series, with a launch of their own.
   const bool ride = !s->torre && !s->timing && (long long)np * std::max(s->nfreq, 1) < (1 << 30);
-  Probes pr{};
-  if (np > 0) {
-    pr.n = np;
-    pr.desc = s->probes_dev;
-    pr.series = s->series_dev;
-    pr.row = s->series_row;
-    pr.nfreq = s->nfreq;
-    pr.omega = s->omega_dev;
-    pr.dft = s->dft_dev;
-    pr.dt = c.dt;
-    pr.step = n;
-  }
+  const Probes pr = rec ? probes_of(s, n, s->series_row, 0, c.nx) : Probes{};
   // Soft sources go into the E sweep, unless it does not run or k_tfsf adds to
   // the new E first.
   Soft so{};
@@ -1312,11 +1329,98 @@ static int one_step(dtm_solver* s) {
   return 0;
 }
 
+// Several steps of the two-pass schedule at once, slab by slab along x (time
+// skewing): the state of a grid larger than the Infinity Cache comes from HBM
+// twice a step, but a slab of it stays in that cache while it is advanced by
+// `group` steps.  A slab's bounds move down from step to step, so that every
+// plane a stencil reads is at the right time: H of step t goes up to X - 3t and
+// E to X - 3t - 2 (E reads H on i-1 .. i+2, the next H reads E on i-2 .. i+1),
+// and where a slab ends the next one begins.  In place, without recomputation,
+// and with the same operations on every cell as one step at a time.  Needs an
+// x axis without wrap-around and steps that are the two sweeps alone: no flux
+// boxes (their sums span the grid), no cells or sources finished by kernels of
+// their own but soft ones.
+struct SkewPlan {
+  int slab = 0, group = 0;  // x planes and steps; slab 0: one step at a time
+};
+static SkewPlan skew_plan(const dtm_solver* s) {
+  SkewPlan p;
+  const dtm_config& c = s->cfg;
+  const bool folds = s->fold_base && !s->no_fold;
+  if (s->torre || c.bc[0] == DTM_BC_PERIODIC || s->fs.nface > 0 || s->timing || s->sc.xz.on || s->ade.on ||
+      (c.tfsf.kind != DTM_TFSF_NONE && !folds))
+    return p;
+  const double yz = (double)c.ny * c.nz;
+  const double plane = yz * (s->store ? 12 : 24) +
+                       (s->pm.split ? 24.0 * yz : 16.0 * ((double)(c.npml[2] + c.npml[3]) * c.nz +
+                                                          (double)(c.npml[4] + c.npml[5]) * c.ny));
+  const double total = plane * c.nx + (s->pm.split ? 0.0 : 16.0 * yz * (c.npml[0] + c.npml[1]));
+  if (total <= kCacheResident) return p;
+  const int most = (int)(kCacheSlab / plane);
+  if (most < 24) return p;
+  const int ns = (c.nx + most - 1) / most;
+  p.slab = (c.nx + ns - 1) / ns;
+  p.group = std::min(16, p.slab / 6);
+  return p;
+}
+
+static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps) {
+  const dtm_config& c = s->cfg;
+  const long long n0 = s->step;
+  const void* F = fields_ptr(s);
+  const int np = (int)s->probes.size();
+  if (s->fold_base && tfsf_gate(s, n0) && (s->tab_n0 < 0 || n0 < s->tab_n0 || n0 + steps > s->tab_n0 + kTableSteps))
+    s->tab_n0 = -1;  // the slabs share one batch of tables
+  const int ns = (c.nx + p.slab - 1) / p.slab;
+  auto bound = [&](int x, int back) { return x <= 0 ? 0 : (x >= c.nx ? c.nx : std::max(0, x - back)); };
+  for (int q = 0; q < ns; q++) {
+    const int lo = q * p.slab, hi = (q + 1) * p.slab;
+    for (int t = 0; t < steps; t++) {
+      const long long n = n0 + t;
+      const int h0 = bound(lo, 3 * t), h1 = bound(hi, 3 * t), e0 = bound(lo, 3 * t + 2), e1 = bound(hi, 3 * t + 2);
+      const bool wave = tfsf_gate(s, n);
+      if (wave) (void)tfsf_for(s, n, 0);
+      if (h0 < h1) {
+        launch_sweep(0, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, h0, h1, wave ? fold_for(s, n, 0) : nullptr,
+                     s->fold_w, s->late.n > 0 ? &s->late : nullptr, nullptr, s->stream);
+        s->late.n = 0;
+      }
+      if (e0 >= e1) continue;
+      if (s->late.n > 0) launch_record(s->store, s->g, F, s->sc, s->late, 1, s->stream);
+      s->late.n = 0;
+      Probes pr = probes_of(s, n, s->series_row + t, e0, e1);
+      Soft so{};
+      if (c.nsoft > 0) soft_values(s, n, so);
+      launch_sweep(1, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, e0, e1, wave ? fold_for(s, n, 1) : nullptr,
+                   s->fold_w, s->probes_h && pr.n > 0 ? &pr : nullptr, so.n > 0 ? &so : nullptr, s->stream);
+      if (s->probes_e) s->late = pr;
+    }
+  }
+  if (s->late.n > 0) launch_record(s->store, s->g, F, s->sc, s->late, 1, s->stream);
+  s->late.n = 0;
+  if (int rc = launch_result()) return rc;
+  s->step += steps;
+  if (np > 0) {
+    s->series_row += steps;
+    if (s->series_row == s->series_cap) return flush_series(s);
+  }
+  return 0;
+}
+
 static int run_steps(dtm_solver* s, int nsteps) {
   s->points_for[0] = s->points_for[1] = -1;
   s->late.n = 0;
-  for (int t = 0; t < nsteps; t++) {
-    s->more = t + 1 < nsteps;
+  const SkewPlan p = skew_plan(s);
+  for (int t = 0; t < nsteps;) {
+    int m = std::min(nsteps - t, p.group);
+    if (!s->probes.empty()) m = std::min(m, s->series_cap - s->series_row);
+    if (p.slab > 0 && m >= 2) {
+      if (int rc = skewed_steps(s, p, m)) return rc;
+      t += m;
+      continue;
+    }
+    t++;
+    s->more = t < nsteps && p.slab == 0;
     if (int rc = one_step(s)) return rc;
   }
   s->points_for[0] = s->points_for[1] = -1;

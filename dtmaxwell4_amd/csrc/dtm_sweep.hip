@@ -1082,6 +1082,15 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
                   const Materials& mt, const Ade& ade, int i0, int i1, const float* fold, const int2* foldw,
                   const Probes* pr, const Soft* soft, hipStream_t st) {
   SweepArgs A{};
+  Soft here{};  // the sources of these planes
+  for (int t = 0; soft && t < soft->n; t++) {
+    if (soft->ijk[t][0] < i0 || soft->ijk[t][0] >= i1) continue;
+    here.comp[here.n] = soft->comp[t];
+    here.q[here.n] = soft->q[t];
+    here.val[here.n] = soft->val[t];
+    for (int a = 0; a < 3; a++) here.ijk[here.n][a] = soft->ijk[t][a];
+    here.n++;
+  }
   if (pr) A.pr = *pr;
   A.fold = fold;
   A.foldw = foldw ? foldw + (up ? fold_weights_size(g) / 2 : 0) : nullptr;
@@ -1103,18 +1112,18 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   // k_soft's launch took 1.8 of 36 us a step at 128^3.  In the variants with the
   // fold or in half storage the few registers this takes made spills that cost
   // every step 2 to 4%: there k_soft follows.
-  const bool soft_in = soft && soft->n <= kSweepSoft && store == 0 && !fold && !split && addressing(A) == kNear;
+  const bool soft_in = here.n > 0 && here.n <= kSweepSoft && store == 0 && !fold && !split && addressing(A) == kNear;
   if (soft_in) {
     A.soft.lo = g.nx;
-    A.soft.n = soft->n;
-    for (int t = 0; t < soft->n; t++) {
-      A.soft.i[t] = soft->ijk[t][0];
-      A.soft.q[t] = soft->ijk[t][2] % NV;
-      A.soft.cell[t] = (long long)soft->ijk[t][1] * g.nz + soft->ijk[t][2] / NV * NV;
-      A.soft.comp[t] = soft->comp[t];
-      A.soft.val[t] = soft->val[t];
-      A.soft.lo = std::min(A.soft.lo, soft->ijk[t][0]);
-      A.soft.hi = std::max(A.soft.hi, soft->ijk[t][0] + 1);
+    A.soft.n = here.n;
+    for (int t = 0; t < here.n; t++) {
+      A.soft.i[t] = here.ijk[t][0];
+      A.soft.q[t] = here.ijk[t][2] % NV;
+      A.soft.cell[t] = (long long)here.ijk[t][1] * g.nz + here.ijk[t][2] / NV * NV;
+      A.soft.comp[t] = here.comp[t];
+      A.soft.val[t] = here.val[t];
+      A.soft.lo = std::min(A.soft.lo, here.ijk[t][0]);
+      A.soft.hi = std::max(A.soft.hi, here.ijk[t][0] + 1);
     }
   }
   // blocks [b0, b1) of the planes [a, b), without the hole set in w
@@ -1150,7 +1159,7 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   } else {
     part(i0, i1, 0, nlb, false);
   }
-  if (soft && !soft_in) launch_soft(store, g, fields, sc, *soft, st);
+  if (here.n > 0 && !soft_in) launch_soft(store, g, fields, sc, here, st);
 }
 
 }  // namespace dtm
