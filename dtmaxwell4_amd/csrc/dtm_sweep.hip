@@ -381,14 +381,14 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
   const bool ywave = __builtin_amdgcn_ballot_w64(yslab >= 0) != 0;
   F zb = {}, zc = {};
   float by = 0.f, cy = 0.f;
-  if constexpr (!SP) {
-    if (zslab) {  // (NV floats follow the coefficients: setup_cpml)
+  {
+    if (SP ? zwave : zslab) {  // (NV floats follow the coefficients: setup_cpml)
       const O o = zm != 0 ? (O)k * 4u : OUT;
       zb = ldt<F>(span<AD>(A.b[2], 0, (unsigned long long)(nz + NV) * 4), o);
       zc = ldt<F>(span<AD>(A.c[2], 0, (unsigned long long)(nz + NV) * 4), o);
     }
     if (ywave) {
-      const O o = ysl >= 0 ? (O)j * 4u : OUT;
+      const O o = yslab >= 0 ? (O)j * 4u : OUT;
       by = ldt<float>(span<AD>(A.b[1], 0, (unsigned long long)A.ny * 4), o);
       cy = ldt<float>(span<AD>(A.c[1], 0, (unsigned long long)A.ny * 4), o);
     }
@@ -569,10 +569,27 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
       pz1 = ldt<F>(psiz(1), oz);
     }
     float bx_ = 0.f, cx_ = 0.f;
-    if (!SP && xsl >= 0) {
+    if (xsl >= 0) {
       using CoefK = __attribute__((address_space(4))) const float;
       bx_ = ((const CoefK*)A.b[0])[i];
       cx_ = ((const CoefK*)A.c[0])[i];
+    }
+    // Split layer: the stored parts of the lane's cells, in a wave that meets a
+    // slab, loaded and stored as whole chunks beside the fields.  (Part by part
+    // and cell by cell, behind a branch each, the 12 loads and the coefficients
+    // were a chain: 40.4 us a step at 117x110x103, 30.3 so.)
+    const bool sany = SP && (zwave || ywave || xsl >= 0);
+    F pn0 = {}, pn1 = {}, pn2 = {};
+    auto stored = [&](int t) {
+      return span<AD>(A.p2[t], (long long)i * A.sx * 4, ((unsigned long long)A.sx + NV) * 4);
+    };
+    const O op = xsl >= 0 || sy || zm != 0 ? ox : OUT;
+    if (sany) {
+      pn0 = ldt<F>(stored(0), op);
+      pn1 = ldt<F>(stored(1), op);
+      pn2 = ldt<F>(stored(2), op);
+    }
+    if (!SP && xsl >= 0) {
       pe0 = ldt<F>(psix(0), ox);
       pe1 = ldt<F>(psix(1), ox);
     } else if (!SP && ywave) {
@@ -794,26 +811,27 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
         n2[q] = __builtin_fmaf(k2, dxy[q] - dyx[q], o2[q]);
       }
     };
-    // split field: x component (y, z), y (z, x), z (x, y)
-    const bool sany = SP && (zwave || ywave || xsl >= 0);
+    // split field: x component (y, z), y (z, x), z (x, y); the stored parts pn
     auto split = [&](int q, float k0, float k1, float k2) {
-      const ArgsK* C = again();
-      const float k1x = xsl >= 0 ? C->b[0][i] : 1.f, k2x = xsl >= 0 ? C->c[0][i] : 1.f;
-      const float k1y = sy ? C->b[1][j] : 1.f, k2y = sy ? C->c[1][j] : 1.f;
-      const bool zin = slab_index(k + q, nz, C->plo[2], C->phi[2]) >= 0;
-      const float k1z = zin ? C->b[2][k + q] : 1.f, k2z = zin ? C->c[2][k + q] : 1.f;
-      const long long b = (long long)i * C->sx + (long long)cell + q;
-      auto part = [&](float* P2, float f0, float k1a, float k2a, float ua, float k1b, float k2b, float ub,
+      const float k1x = xsl >= 0 ? bx_ : 1.f, k2x = xsl >= 0 ? cx_ : 1.f;
+      const float k1y = sy ? by : 1.f, k2y = sy ? cy : 1.f;
+      const bool zin = (zm >> q) & 1u;
+      const float k1z = zin ? zb[q] : 1.f, k2z = zin ? zc[q] : 1.f;
+      auto part = [&](float& stored, float f0, float k1a, float k2a, float ua, float k1b, float k2b, float ub,
                       float n) -> float {
-        if (k2a == 1.0f && k2b == 1.0f) return n;
-        const float p2 = P2[b], p1 = f0 - p2;
+        const float p2 = stored, p1 = f0 - p2;
         const float m1 = __builtin_fmaf(k2a, ua, k1a * p1), m2 = __builtin_fmaf(k2b, ub, k1b * p2);
-        P2[b] = m2;
-        return m1 + m2;
+        const bool out = k2a == 1.0f && k2b == 1.0f;  // outside every slab of the component
+        stored = out ? p2 : m2;
+        return out ? n : m1 + m2;
       };
-      n0[q] = part(C->p2[0], o0[q], k1y, k2y, k0 * dyz[q], k1z, k2z, -k0 * dzy[q], n0[q]);
-      n1[q] = part(C->p2[1], o1[q], k1z, k2z, k1 * dzx[q], k1x, k2x, -k1 * dxz[q], n1[q]);
-      n2[q] = part(C->p2[2], o2[q], k1x, k2x, k2 * dxy[q], k1y, k2y, -k2 * dyx[q], n2[q]);
+      float s0 = pn0[q], s1 = pn1[q], s2 = pn2[q];
+      n0[q] = part(s0, o0[q], k1y, k2y, k0 * dyz[q], k1z, k2z, -k0 * dzy[q], n0[q]);
+      n1[q] = part(s1, o1[q], k1z, k2z, k1 * dzx[q], k1x, k2x, -k1 * dxz[q], n1[q]);
+      n2[q] = part(s2, o2[q], k1x, k2x, k2 * dxy[q], k1y, k2y, -k2 * dyx[q], n2[q]);
+      pn0[q] = s0;
+      pn1[q] = s1;
+      pn2[q] = s2;
     };
     const unsigned in = act ? (1u << nv) - 1u : 0u;
     unsigned put = in;  // cells whose new value this sweep stores
@@ -865,6 +883,11 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
         upd(q, k0, k1, k2);
         if (sany && ((in >> q) & 1u)) split(q, k0, k1, k2);
       }
+    }
+    if (sany && op != OUT) {
+      putf(stored(0), op, pn0);
+      putf(stored(1), op, pn1);
+      putf(stored(2), op, pn2);
     }
     if constexpr (UP && STORE == 0 && !TF) {  // launch_sweep: soft_in
       if (i >= A.soft.lo && i < A.soft.hi) {
