@@ -31,12 +31,13 @@ static thread_local std::string g_err;
 // Time skewing (skewed_steps): a state up to kCacheResident bytes stays in the
 // Infinity Cache (256 MB) by itself; kCacheSlab is what a slab may take of it.
 // Measured, us a step, one step at a time and skewed: FP32 200^3 (238 MB) 127
-// and 127, 207^3 (263 MB) 166 and 155, 256^3 301 and 272; 512x256x256 FP32 567,
-// and 544 / 532 / 541 / 593 in slabs of 48 / 80 / 96 / 128 planes (85, 142, 170
-// and 226 MB), FP16 353, and 361 / 340 / 325 / 328 / 378 in slabs of 64 / 96 /
-// 128 / 192 / 256 (63, 94, 126, 189 and 252 MB): smaller ones leave the chip's
-// last round of waves emptier, larger ones leave the cache.
-static constexpr double kCacheResident = 245e6, kCacheSlab = 170e6;
+// and 127, 207^3 (263 MB) 166 and 155, 256^3 301 and 280.  Smaller slabs leave
+// the last round of waves emptier, larger ones leave the cache: 512x256x256 FP32
+// 567, and 540 / 538 / 532 / 536 / 593 in slabs of 110 / 130 / 150 / 170 / 226 MB,
+// FP16 353, and 340 / 328 / 328 / 338 / 378 at 110 / 130 / 150 / 170 / 252 MB;
+// 256^3 FP32 290 / 282 / 282 / 277 and FP16 (195) 179 / 165 / 165 / 165 at 110 /
+// 130 / 150 / 170 MB.
+static constexpr double kCacheResident = 245e6, kCacheSlab = 150e6;
 static constexpr int kTableSteps = 32;  // plane-wave waveform tables per batch
 
 static int fail(int code, const std::string& msg) {
