@@ -98,7 +98,7 @@ struct SweepArgs {
   float* p2[3];
   Materials mt;
   struct {
-    int i0, j0, k0;
+    int on, i0, j0, k0;
     long long bsx, bsy;
     float* curl[3];
   } ade;
@@ -840,32 +840,52 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
       const bool dpl = dwave && i >= A.mt.d_i0 && i < A.mt.d_i0 + A.mt.d_ni;
       mixed = __builtin_amdgcn_ballot_w64(cls != 0) != 0 || special0 || dpl;
       if (mixed) {
-        const ArgsK* C = again();  // cells of another class than 0, of the design box, or finished by k_ade
+        // Cells of another class than 0, of the design box, or finished by k_ade.
+        // The entries of several cells are loaded together: cell by cell, behind
+        // a branch each, the E sweep with a sphere of radius 40 took 72 us at
+        // 200^3, 65 so (four at a time; half storage has registers for two:
+        // 512x256x256 190 and 183).
+        const ArgsK* C = again();
+        using Entry = unsigned __attribute__((ext_vector_type(4)));  // ClassEntry: inv_eps, then mat and special bytes
+        constexpr int AT = STORE == 1 ? 2 : NV;  // entries in registers at a time
 #pragma unroll
-        for (int q = 0; q < NV; q++) {
-          n0[q] = n1[q] = n2[q] = 0.f;
-          if (!((in >> q) & 1u)) continue;
-          const ClassEntry ce = C->mt.table[(cls >> (8 * q)) & 0xffu];
-          float i0 = ce.inv_eps[0], i1 = ce.inv_eps[1], i2 = ce.inv_eps[2];
-          bool over = false;
+        for (int q0 = 0; q0 < NV; q0 += AT) {
+          Entry ce[AT];
+#pragma unroll
+          for (int t = 0; t < AT; t++)
+            ce[t] = *reinterpret_cast<const Entry*>(C->mt.table + ((cls >> (8 * (q0 + t))) & 0xffu));
+          unsigned over = 0;
           if (dpl) {
-            const int dj = j - C->mt.d_j0, dk = k + q - C->mt.d_k0;
-            if (dj >= 0 && dj < C->mt.d_nj && dk >= 0 && dk < C->mt.d_nk) {
-              i0 = i1 = i2 = C->mt.d_inv_eps[((long long)(i - C->mt.d_i0) * C->mt.d_nj + dj) * C->mt.d_nk + dk];
-              over = true;
+#pragma unroll
+            for (int t = 0; t < AT; t++) {
+              const int dj = j - C->mt.d_j0, dk = k + q0 + t - C->mt.d_k0;
+              if (((in >> (q0 + t)) & 1u) && dj >= 0 && dj < C->mt.d_nj && dk >= 0 && dk < C->mt.d_nk) {
+                ce[t][0] = ce[t][1] = ce[t][2] = __float_as_uint(
+                    C->mt.d_inv_eps[((long long)(i - C->mt.d_i0) * C->mt.d_nj + dj) * C->mt.d_nk + dk]);
+                over |= 1u << t;
+              }
             }
           }
-          const float k0 = C->dt * i0, k1 = C->dt * i1, k2 = C->dt * i2;
-          if (ce.special && !over) {  // its curl, for k_ade
-            const long long bq = (long long)(i - C->ade.i0) * C->ade.bsx + (long long)(j - C->ade.j0) * C->ade.bsy +
-                                 (k + q - C->ade.k0);
-            C->ade.curl[0][bq] = dyz[q] - dzy[q];
-            C->ade.curl[1][bq] = dzx[q] - dxz[q];
-            C->ade.curl[2][bq] = dxy[q] - dyx[q];
-            put &= ~(1u << q);
-          } else {
+#pragma unroll
+          for (int t = 0; t < AT; t++) {
+            const int q = q0 + t;
+            const float k0 = C->dt * __uint_as_float(ce[t][0]), k1 = C->dt * __uint_as_float(ce[t][1]),
+                        k2 = C->dt * __uint_as_float(ce[t][2]);
             upd(q, k0, k1, k2);
-            if (sany) split(q, k0, k1, k2);
+            if (sany && ((in >> q) & 1u)) split(q, k0, k1, k2);
+          }
+          if (C->ade.on) {
+#pragma unroll
+            for (int t = 0; t < AT; t++) {
+              const int q = q0 + t;
+              if (!((in >> q) & 1u) || (ce[t][3] >> 24) == 0 || ((over >> t) & 1u)) continue;
+              const long long bq = (long long)(i - C->ade.i0) * C->ade.bsx + (long long)(j - C->ade.j0) * C->ade.bsy +
+                                   (k + q - C->ade.k0);  // its curl, for k_ade
+              C->ade.curl[0][bq] = dyz[q] - dzy[q];
+              C->ade.curl[1][bq] = dzx[q] - dxz[q];
+              C->ade.curl[2][bq] = dxy[q] - dyx[q];
+              put &= ~(1u << q);
+            }
           }
         }
       }
@@ -1118,6 +1138,7 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   A.fold = fold;
   A.foldw = foldw ? foldw + (up ? fold_weights_size(g) / 2 : 0) : nullptr;
   A.mt = mt;
+  A.ade.on = ade.on;
   A.ade.i0 = ade.i0;
   A.ade.j0 = ade.j0;
   A.ade.k0 = ade.k0;
