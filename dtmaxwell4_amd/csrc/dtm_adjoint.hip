@@ -20,80 +20,61 @@
 #include <math.h>
 #include <stdio.h>
 
+#include <algorithm>
+
 #include "dtm_internal.h"
 
 namespace dtm {
 
 namespace {
 
-// E of the design box, three components, into out[c * nd + cell].
-__global__ __launch_bounds__(256) void k_adj_snap(Grid g, Fields<0> f, Materials mt, float* out) {
-  const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-  const long long b = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (b >= nd) return;
+// The design cells and the monitors of some x planes: cells [b0, b1) of the
+// box, monitors whose cell index lies in [q0, q1).
+struct Part {
+  long long b0, b1, q0, q1;
+};
+__device__ __forceinline__ long long design_cell(const Grid& g, const Materials& mt, long long b) {
   const int k = mt.d_k0 + (int)(b % mt.d_nk);
   const int j = mt.d_j0 + (int)((b / mt.d_nk) % mt.d_nj);
   const int i = mt.d_i0 + (int)(b / ((long long)mt.d_nk * mt.d_nj));
-  const long long q = i * g.sx + j * g.sy + k;
-  for (int c = 0; c < 3; c++) out[c * nd + b] = f.E[c][q];
+  return i * g.sx + j * g.sy + k;
 }
 
-// series[m] = Ez at the monitor cells.
-__global__ __launch_bounds__(256) void k_adj_monitor(Fields<0> f, const long long* q, int nmon, float* series) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < nmon) series[m] = f.E[2][q[m]];
+// The first nbs blocks: E of the design box, three components, into
+// out[c * nd + cell]; the rest: series[m] = Ez at the monitor cells.
+__global__ __launch_bounds__(256) void k_adj_record(Grid g, Fields<0> f, Materials mt, Part pt, float* out, unsigned nbs,
+                                                    const long long* q, int nmon, float* series) {
+  if (blockIdx.x < nbs) {
+    const long long b = pt.b0 + blockIdx.x * 256LL + threadIdx.x;
+    if (b >= pt.b1) return;
+    const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk, cell = design_cell(g, mt, b);
+    for (int c = 0; c < 3; c++) out[c * nd + b] = f.E[c][cell];
+    return;
+  }
+  const int m = (blockIdx.x - nbs) * 256 + threadIdx.x;
+  if (m < nmon && q[m] >= pt.q0 && q[m] < pt.q1) series[m] = f.E[2][q[m]];
 }
 
-// acc[cell] += sum_c eps^2 zeta_c (E1_c - E0_c)  (design inverse permittivity is isotropic)
-__global__ __launch_bounds__(256) void k_adj_grad(Grid g, Fields<0> f, Materials mt, const float* e0, const float* e1,
-                                                  double* acc) {
-  const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-  const long long b = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (b >= nd) return;
-  const int k = mt.d_k0 + (int)(b % mt.d_nk);
-  const int j = mt.d_j0 + (int)((b / mt.d_nk) % mt.d_nj);
-  const int i = mt.d_i0 + (int)(b / ((long long)mt.d_nk * mt.d_nj));
-  const long long q = i * g.sx + j * g.sy + k;
-  const double eps = 1.0 / (double)mt.d_inv_eps[b];
-  double s = 0.0;
-  for (int c = 0; c < 3; c++) s += (double)f.E[c][q] * ((double)e1[c * nd + b] - (double)e0[c * nd + b]);
-  acc[b] += eps * eps * s;
-}
-
-// zeta_z += M dJ/dEz^n at the monitors: dJ/dEz_m^n = 2 dt Re(conj(F_m) e^{i w n dt}).
-__global__ __launch_bounds__(256) void k_adj_inject(Fields<0> f, const long long* q, const float* inv_eps,
-                                                    const double* F, int nmon, double w, double dt, long long n) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= nmon) return;
-  double sn, cn;
-  sincos(w * (double)n * dt, &sn, &cn);
-  const double gJ = 2.0 * dt * (F[2 * m] * cn + F[2 * m + 1] * sn);
-  f.E[2][q[m]] += (float)(gJ * inv_eps[m]);
-}
-
-// k_adj_inject at step n and k_adj_grad of step n-1 in one launch: the
-// first nbg blocks accumulate the gradient, the rest inject.  Only used when
+// The first nbg blocks: acc[cell] += sum_c eps^2 zeta_c (E1_c - E0_c) (design
+// inverse permittivity is isotropic); the rest: zeta_z += M dJ/dEz^n at the
+// monitors, dJ/dEz_m^n = 2 dt Re(conj(F_m) e^{i w n dt}).  Both at once only when
 // no monitor lies in the design box, so the two touch disjoint cells.
-__global__ __launch_bounds__(256) void k_adj_inject_grad(Grid g, Fields<0> f, Materials mt, const float* e0,
+__global__ __launch_bounds__(256) void k_adj_inject_grad(Grid g, Fields<0> f, Materials mt, Part pt, const float* e0,
                                                          const float* e1, double* acc, unsigned nbg,
                                                          const long long* q, const float* inv_eps, const double* F,
                                                          int nmon, double w, double dt, long long n) {
   if (blockIdx.x < nbg) {
-    const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-    const long long b = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (b >= nd) return;
-    const int k = mt.d_k0 + (int)(b % mt.d_nk);
-    const int j = mt.d_j0 + (int)((b / mt.d_nk) % mt.d_nj);
-    const int i = mt.d_i0 + (int)(b / ((long long)mt.d_nk * mt.d_nj));
-    const long long qq = i * g.sx + j * g.sy + k;
+    const long long b = pt.b0 + blockIdx.x * 256LL + threadIdx.x;
+    if (b >= pt.b1) return;
+    const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk, qq = design_cell(g, mt, b);
     const double eps = 1.0 / (double)mt.d_inv_eps[b];
     double sum = 0.0;
     for (int c = 0; c < 3; c++) sum += (double)f.E[c][qq] * ((double)e1[c * nd + b] - (double)e0[c * nd + b]);
     acc[b] += eps * eps * sum;
     return;
   }
-  const int m = (blockIdx.x - nbg) * blockDim.x + threadIdx.x;
-  if (m >= nmon) return;
+  const int m = (blockIdx.x - nbg) * 256 + threadIdx.x;
+  if (m >= nmon || q[m] < pt.q0 || q[m] >= pt.q1) return;
   double sn, cn;
   sincos(w * (double)n * dt, &sn, &cn);
   const double gJ = 2.0 * dt * (F[2 * m] * cn + F[2 * m + 1] * sn);
@@ -102,46 +83,35 @@ __global__ __launch_bounds__(256) void k_adj_inject_grad(Grid g, Fields<0> f, Ma
 
 void check(const char* what) { note_launch(what); }
 
-unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
+unsigned blocks_for(long long n) { return n > 0 ? (unsigned)((n + 255) / 256) : 0u; }
+
+Part part(const Grid& g, const Materials& mt, int i0, int i1) {
+  const long long pl = (long long)mt.d_nj * mt.d_nk;
+  return Part{pl * std::min(std::max(0, i0 - mt.d_i0), mt.d_ni), pl * std::max(0, std::min(mt.d_ni, i1 - mt.d_i0)),
+              g.sx * i0, g.sx * i1};
+}
 
 }  // namespace
 
-void launch_adj_snap(const Grid& g, const void* fields, const Materials& mt, float* out, hipStream_t st) {
-  const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-  hipLaunchKernelGGL(k_adj_snap, dim3(blocks_for(nd)), dim3(256), 0, st, g, *static_cast<const Fields<0>*>(fields), mt,
-                     out);
-  check("k_adj_snap");
+void launch_adj_record(const Grid& g, const void* fields, const Materials& mt, int i0, int i1, float* snap,
+                       const long long* q, int nmon, float* series, hipStream_t st) {
+  const Part p = part(g, mt, i0, i1);
+  const unsigned nbs = snap ? blocks_for(p.b1 - p.b0) : 0, nbm = series ? blocks_for(nmon) : 0;
+  if (nbs + nbm == 0) return;
+  hipLaunchKernelGGL(k_adj_record, dim3(nbs + nbm), dim3(256), 0, st, g, *static_cast<const Fields<0>*>(fields), mt, p,
+                     snap, nbs, q, nmon, series);
+  check("k_adj_record");
 }
 
-void launch_adj_monitor(const void* fields, const long long* q, int nmon, float* series, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_monitor, dim3(blocks_for(nmon)), dim3(256), 0, st, *static_cast<const Fields<0>*>(fields),
-                     q, nmon, series);
-  check("k_adj_monitor");
-}
-
-void launch_adj_grad(const Grid& g, const void* fields, const Materials& mt, const float* e0, const float* e1,
-                     double* acc, hipStream_t st) {
-  const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-  hipLaunchKernelGGL(k_adj_grad, dim3(blocks_for(nd)), dim3(256), 0, st, g, *static_cast<const Fields<0>*>(fields), mt,
-                     e0, e1, acc);
-  check("k_adj_grad");
-}
-
-void launch_adj_inject_grad(const Grid& g, const void* fields, const Materials& mt, const float* e0, const float* e1,
-                            double* acc, const long long* q, const float* inv_eps, const double* F, int nmon,
-                            double w, double dt, long long n, hipStream_t st) {
-  const long long nd = (long long)mt.d_ni * mt.d_nj * mt.d_nk;
-  const unsigned nbg = blocks_for(nd);
-  hipLaunchKernelGGL(k_adj_inject_grad, dim3(nbg + blocks_for(nmon)), dim3(256), 0, st, g,
-                     *static_cast<const Fields<0>*>(fields), mt, e0, e1, acc, nbg, q, inv_eps, F, nmon, w, dt, n);
+void launch_adj_inject_grad(const Grid& g, const void* fields, const Materials& mt, int i0, int i1, const float* e0,
+                            const float* e1, double* acc, const long long* q, const float* inv_eps, const double* F,
+                            int nmon, double w, double dt, long long n, hipStream_t st) {
+  const Part p = part(g, mt, i0, i1);
+  const unsigned nbg = e0 ? blocks_for(p.b1 - p.b0) : 0, nbm = q ? blocks_for(nmon) : 0;
+  if (nbg + nbm == 0) return;
+  hipLaunchKernelGGL(k_adj_inject_grad, dim3(nbg + nbm), dim3(256), 0, st, g, *static_cast<const Fields<0>*>(fields),
+                     mt, p, e0, e1, acc, nbg, q, inv_eps, F, nmon, w, dt, n);
   check("k_adj_inject_grad");
-}
-
-void launch_adj_inject(const void* fields, const long long* q, const float* inv_eps, const double* F, int nmon,
-                       double w, double dt, long long n, hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_inject, dim3(blocks_for(nmon)), dim3(256), 0, st, *static_cast<const Fields<0>*>(fields), q,
-                     inv_eps, F, nmon, w, dt, n);
-  check("k_adj_inject");
 }
 
 }  // namespace dtm

@@ -355,17 +355,15 @@ void launch_tfsf_fold(const Tfsf& tf, const double* tables, float* out, int nste
 // mode 0: H post-correction, 1: E post-correction, 2: H pre-correction
 // (applied to H^{n-1/2} and psi before a fused step: psi += c D / b).
 // design-gradient adjoint (FP32 storage)
-void launch_adj_snap(const Grid& g, const void* fields, const Materials& mt, float* out, hipStream_t st);
-void launch_adj_monitor(const void* fields, const long long* q, int nmon, float* series, hipStream_t st);
-void launch_adj_grad(const Grid& g, const void* fields, const Materials& mt, const float* e0, const float* e1,
-                     double* acc, hipStream_t st);
-void launch_adj_inject(const void* fields, const long long* q, const float* inv_eps, const double* F, int nmon,
-                       double w, double dt, long long n, hipStream_t st);
-// launch_adj_inject at step n, then launch_adj_grad (of step n-1), in one
-// launch; only for monitors outside the design box.
-void launch_adj_inject_grad(const Grid& g, const void* fields, const Materials& mt, const float* e0, const float* e1,
-                            double* acc, const long long* q, const float* inv_eps, const double* F, int nmon,
-                            double w, double dt, long long n, hipStream_t st);
+// Both on the x planes [i0, i1).  Record: the design box's E into snap (null:
+// not) and Ez at the monitors into series (null: not).  Inject / grad: dJ/dE at
+// step n (q null: not), and the gradient of step n-1 (e0 null: not); both in one
+// launch only for monitors outside the design box.
+void launch_adj_record(const Grid& g, const void* fields, const Materials& mt, int i0, int i1, float* snap,
+                       const long long* q, int nmon, float* series, hipStream_t st);
+void launch_adj_inject_grad(const Grid& g, const void* fields, const Materials& mt, int i0, int i1, const float* e0,
+                            const float* e1, double* acc, const long long* q, const float* inv_eps, const double* F,
+                            int nmon, double w, double dt, long long n, hipStream_t st);
 void launch_tfsf_tables(const Tfsf& tf, double* out, long long n0, int nsteps, double dt, hipStream_t st);
 void launch_tfsf(int store, int half, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                  const Materials& mt, const Ade& ade, const Tfsf& tf, const TfsfBands& bands, double t_inc,

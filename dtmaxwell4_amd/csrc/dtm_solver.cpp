@@ -184,6 +184,17 @@ static int zero_state(dtm_solver* s) {
   return 0;
 }
 
+// What a caller does when E of its step t (counted from the call) is final on
+// the x planes [i0, i1).
+struct AfterE {
+  const void* f;
+  void (*call)(const void* f, int t, int i0, int i1);
+  template <typename F>
+  explicit AfterE(const F& fn)
+      : f(&fn), call([](const void* p, int t, int i0, int i1) { (*static_cast<const F*>(p))(t, i0, i1); }) {}
+  void operator()(int t, int i0, int i1) const { call(f, t, i0, i1); }
+};
+
 extern "C" {
 
 const char* dtm_last_error(void) { return g_err.c_str(); }
@@ -1365,12 +1376,12 @@ static SkewPlan skew_plan(const dtm_solver* s) {
   return p;
 }
 
-static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps) {
+static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps, int t0, const AfterE* after) {
   const dtm_config& c = s->cfg;
   const long long n0 = s->step;
   const void* F = fields_ptr(s);
-  const int np = (int)s->probes.size();
-  if (s->fold_base && tfsf_gate(s, n0) && (s->tab_n0 < 0 || n0 < s->tab_n0 || n0 + steps > s->tab_n0 + kTableSteps))
+  const int np = !s->adjoint && !s->replay ? (int)s->probes.size() : 0;
+  if (s->fold_base && !s->adjoint && tfsf_gate(s, n0) && (s->tab_n0 < 0 || n0 < s->tab_n0 || n0 + steps > s->tab_n0 + kTableSteps))
     s->tab_n0 = -1;  // the slabs share one batch of tables
   const int ns = (c.nx + p.slab - 1) / p.slab;
   auto bound = [&](int x, int back) { return x <= 0 ? 0 : (x >= c.nx ? c.nx : std::max(0, x - back)); };
@@ -1379,7 +1390,7 @@ static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps) {
     for (int t = 0; t < steps; t++) {
       const long long n = n0 + t;
       const int h0 = bound(lo, 3 * t), h1 = bound(hi, 3 * t), e0 = bound(lo, 3 * t + 2), e1 = bound(hi, 3 * t + 2);
-      const bool wave = tfsf_gate(s, n);
+      const bool wave = !s->adjoint && tfsf_gate(s, n);
       if (wave) (void)tfsf_for(s, n, 0);
       if (h0 < h1) {
         launch_sweep(0, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, h0, h1, wave ? fold_for(s, n, 0) : nullptr,
@@ -1389,12 +1400,13 @@ static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps) {
       if (e0 >= e1) continue;
       if (s->late.n > 0) launch_record(s->store, s->g, F, s->sc, s->late, 1, s->stream);
       s->late.n = 0;
-      Probes pr = probes_of(s, n, s->series_row + t, e0, e1);
+      const Probes pr = np > 0 ? probes_of(s, n, s->series_row + t, e0, e1) : Probes{};
       Soft so{};
-      if (c.nsoft > 0) soft_values(s, n, so);
+      if (c.nsoft > 0 && !s->adjoint) soft_values(s, n, so);
       launch_sweep(1, s->store, s->g, F, s->sc, s->pm, s->mt, s->ade, e0, e1, wave ? fold_for(s, n, 1) : nullptr,
                    s->fold_w, s->probes_h && pr.n > 0 ? &pr : nullptr, so.n > 0 ? &so : nullptr, s->stream);
       if (s->probes_e) s->late = pr;
+      if (after) (*after)(t0 + t, e0, e1);
     }
   }
   if (s->late.n > 0) launch_record(s->store, s->g, F, s->sc, s->late, 1, s->stream);
@@ -1408,21 +1420,22 @@ static int skewed_steps(dtm_solver* s, const SkewPlan& p, int steps) {
   return 0;
 }
 
-static int run_steps(dtm_solver* s, int nsteps) {
+static int run_steps(dtm_solver* s, int nsteps, const AfterE* after = nullptr) {
   s->points_for[0] = s->points_for[1] = -1;
   s->late.n = 0;
   const SkewPlan p = skew_plan(s);
   for (int t = 0; t < nsteps;) {
     int m = std::min(nsteps - t, p.group);
-    if (!s->probes.empty()) m = std::min(m, s->series_cap - s->series_row);
+    if (!s->probes.empty() && !s->adjoint && !s->replay) m = std::min(m, s->series_cap - s->series_row);
     if (p.slab > 0 && m >= 2) {
-      if (int rc = skewed_steps(s, p, m)) return rc;
+      if (int rc = skewed_steps(s, p, m, t, after)) return rc;
       t += m;
       continue;
     }
-    t++;
-    s->more = t < nsteps && p.slab == 0;
+    s->more = t + 1 < nsteps && p.slab == 0;
     if (int rc = one_step(s)) return rc;
+    if (after) (*after)(t, 0, s->cfg.nx);
+    t++;
   }
   s->points_for[0] = s->points_for[1] = -1;
   return 0;
@@ -1623,6 +1636,11 @@ int dtm_adjoint_design_gradient(dtm_solver* s, int nsteps, double omega, int nmo
   auto* stash = static_cast<char*>(d_stash);
   std::vector<StateImage> ck_ptrs(nck);
   const size_t snap = 3 * (size_t)nd;
+  auto monitors_on = [&](int i0, int i1) {
+    for (long long m : q)
+      if (m >= i0 * s->g.sx && m < i1 * s->g.sx) return true;
+    return false;
+  };
   int rc = 0;
   do {
     if (hipMemcpyAsync(hq, q.data(), sizeof(long long) * nmon, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
@@ -1634,15 +1652,22 @@ int dtm_adjoint_design_gradient(dtm_solver* s, int nsteps, double omega, int nmo
     // forward: record Ez at the monitors every step, and the design-box E
     // every step (history) or the whole state every K steps (checkpoints)
     // plus the tail segments' snapshots
-    for (int n = 0; n < nsteps && !rc; n++) {
-      if (n < n_last && n % K == 0) {
-        ck_ptrs[n / K] = state_ptrs(s);
-        if ((rc = save_state(s, ck + (size_t)(n / K) * sbytes))) break;
+    for (int b = 0; b < nsteps && !rc;) {
+      const int e = b < n_last ? std::min(b + K, n_last) : nsteps;
+      if (b < n_last) {
+        ck_ptrs[b / K] = state_ptrs(s);
+        if ((rc = save_state(s, ck + (size_t)(b / K) * sbytes))) break;
+      } else {
+        launch_adj_record(s->g, fields_ptr(s), mt, 0, c.nx, hist, nullptr, 0, nullptr, s->stream);
       }
-      if (n == n_last) launch_adj_snap(s->g, fields_ptr(s), mt, hist, s->stream);
-      rc = one_step(s);
-      launch_adj_monitor(fields_ptr(s), hq, nmon, ser + (size_t)n * nmon, s->stream);
-      if (n >= n_last) launch_adj_snap(s->g, fields_ptr(s), mt, hist + (size_t)(n - n_last + 1) * snap, s->stream);
+      const auto record = [&](int t, int i0, int i1) {
+        const int n = b + t;
+        launch_adj_record(s->g, fields_ptr(s), mt, i0, i1, n >= n_last ? hist + (size_t)(n - n_last + 1) * snap : nullptr,
+                          hq, nmon, monitors_on(i0, i1) ? ser + (size_t)n * nmon : nullptr, s->stream);
+      };
+      const AfterE after(record);
+      rc = run_steps(s, e - b, &after);
+      b = e;
     }
     if (!rc) rc = launch_result();
     if (rc) break;
@@ -1673,7 +1698,8 @@ int dtm_adjoint_design_gradient(dtm_solver* s, int nsteps, double omega, int nmo
     // forward sweeps; zeta^N = M dJ/dE^N
     if ((rc = zero_state(s))) break;
     s->adjoint = true;
-    launch_adj_inject(fields_ptr(s), hq, hie, Fd, nmon, omega, c.dt, nsteps, s->stream);
+    launch_adj_inject_grad(s->g, fields_ptr(s), mt, 0, c.nx, nullptr, nullptr, acc, hq, hie, Fd, nmon, omega, c.dt,
+                           nsteps, s->stream);
     for (int seg = nseg - 1; seg >= 0 && !rc; seg--) {
       const int n0 = seg * K, n1 = std::min(n0 + K, nsteps);
       // this segment's snapshots: kept from the forward pass (tail) or
@@ -1687,11 +1713,13 @@ int dtm_adjoint_design_gradient(dtm_solver* s, int nsteps, double omega, int nmo
         s->replay = true;
         s->step = n0;
         s->tab_n0 = -1;
-        launch_adj_snap(s->g, fields_ptr(s), mt, hist, s->stream);
-        for (int n = n0; n < n1 && !rc; n++) {
-          rc = one_step(s);
-          launch_adj_snap(s->g, fields_ptr(s), mt, hist + (size_t)(n - n0 + 1) * snap, s->stream);
-        }
+        launch_adj_record(s->g, fields_ptr(s), mt, 0, c.nx, hist, nullptr, 0, nullptr, s->stream);
+        const auto record = [&](int t, int i0, int i1) {
+          launch_adj_record(s->g, fields_ptr(s), mt, i0, i1, hist + (size_t)(t + 1) * snap, nullptr, 0, nullptr,
+                            s->stream);
+        };
+        const AfterE after(record);
+        rc = run_steps(s, n1 - n0, &after);
         s->replay = false;
         s->adjoint = true;
         if (rc || (rc = load_state(s, stash, adj))) break;
@@ -1700,21 +1728,21 @@ int dtm_adjoint_design_gradient(dtm_solver* s, int nsteps, double omega, int nmo
       // gradient of step n, one backward step, injection at step n; the
       // injection and the next step's gradient share a launch when they
       // touch disjoint cells
-      launch_adj_grad(s->g, fields_ptr(s), mt, hs0 + (size_t)(n1 - 1 - n0) * snap, hs0 + (size_t)(n1 - n0) * snap,
-                      acc, s->stream);
-      for (int n = n1 - 1; n >= n0 && !rc; n--) {
-        rc = one_step(s);
+      launch_adj_inject_grad(s->g, fields_ptr(s), mt, 0, c.nx, hs0 + (size_t)(n1 - 1 - n0) * snap,
+                             hs0 + (size_t)(n1 - n0) * snap, acc, nullptr, hie, Fd, 0, omega, c.dt, 0, s->stream);
+      const auto inject = [&](int t, int i0, int i1) {
+        const int n = n1 - 1 - t;
         const bool next = n - 1 >= n0;  // the gradient of step n-1 follows in this segment
-        if (n >= 1 && next && !mon_in_design) {
-          launch_adj_inject_grad(s->g, fields_ptr(s), mt, hs0 + (size_t)(n - 1 - n0) * snap,
-                                 hs0 + (size_t)(n - n0) * snap, acc, hq, hie, Fd, nmon, omega, c.dt, n, s->stream);
-          continue;
-        }
-        if (n >= 1) launch_adj_inject(fields_ptr(s), hq, hie, Fd, nmon, omega, c.dt, n, s->stream);
-        if (next)
-          launch_adj_grad(s->g, fields_ptr(s), mt, hs0 + (size_t)(n - 1 - n0) * snap, hs0 + (size_t)(n - n0) * snap,
-                          acc, s->stream);
-      }
+        const float* const e0 = next ? hs0 + (size_t)(n - 1 - n0) * snap : nullptr;
+        const long long* const at = n >= 1 && monitors_on(i0, i1) ? hq : nullptr;
+        if (mon_in_design && at)
+          launch_adj_inject_grad(s->g, fields_ptr(s), mt, i0, i1, nullptr, nullptr, acc, at, hie, Fd, nmon, omega, c.dt,
+                                 n, s->stream);
+        launch_adj_inject_grad(s->g, fields_ptr(s), mt, i0, i1, e0, e0 ? e0 + snap : nullptr, acc,
+                               mon_in_design ? nullptr : at, hie, Fd, nmon, omega, c.dt, n, s->stream);
+      };
+      const AfterE after(inject);
+      if ((rc = run_steps(s, n1 - n0, &after))) break;
     }
     s->adjoint = false;
     s->replay = false;

@@ -63,3 +63,30 @@ def test_one_call_equals_single_steps(n, storage, split, wave, soft, probes):
     assert max(np.abs(x).max() for x in a[:6]) > 1e-4
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("every,inside", [(0, False), (13, False), (13, True)])
+def test_adjoint_slab_by_slab_equals_whole_steps(every, inside):
+    """Both passes of the adjoint on a large grid; with event timing on, every
+    step runs over the whole grid.  Monitors beside and inside the design box,
+    with the history kept and rebuilt from checkpoints."""
+    from dtmaxwell4_amd.solver import Solver
+    n = (300, 190, 207)
+    out = []
+    for timing in (False, True):
+        cfg = abi.default_config(*n, D, D, D, configs.dt_for(D, D, D))
+        cfg.npml[:] = [8] * 6
+        cfg.nsoft = 1
+        so = cfg.soft[0]
+        so.comp, so.i, so.j, so.k = abi.EZ, 130, 95, 103
+        so.waveform, so.amp, so.w, so.tw, so.t0 = abi.WAVE_GAUSS_SINE, 5.0, 2 * math.pi, 0.3, 0.2
+        s = Solver(cfg)
+        s.set_design_eps(144, 90, 98, 1 + 2 * np.random.default_rng(2).random((25, 11, 10)))
+        if every:
+            s.set_adjoint_checkpoints(every)
+        s.set_kernel_timing(timing)
+        mon = [(150, 95, 100), (160, 92, 103)] if inside else [(175, 95, 100), (138, 93, 103), (180, 96, 105)]
+        out.append(s.design_gradient(47, 6.0, mon))
+        s.close()
+    assert out[0][0] > 0 and np.abs(out[0][1]).max() > 0
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
