@@ -1790,30 +1790,37 @@ static int zone_copy(dtm_solver* s, int comp, float* buf, bool to_host) {
 }
 
 // Device to pageable host memory, all of `src` final on s->stream or earlier.
-// A plain copy runs at 10 GB/s here: the runtime stages it through pinned
-// memory, and one thread writes (and first touches) the destination.  From
-// kReadStaged bytes on the device fills a ring of pinned chunks and kReaders
-// threads empty it (134 MB: 12.7 ms plain, 3.6 so; 32 MB: 3.1 and 1.0; 8 MB:
-// 1.2 and 0.5; 1 MB: 0.55 and 0.26; six threads gain nothing more).
-static constexpr size_t kReadStaged = 1 << 20;
+// A plain copy runs at 10 GB/s into fresh pages and at 17 into warm ones: the
+// runtime stages it through pinned memory, and one thread writes (and first
+// touches) the destination.  From kReadStaged bytes on the device fills a ring
+// of pinned chunks and kReaders threads empty it.  Plain and so, ms, fresh | warm:
+// 134 MB 12.8 and 3.6 | 7.4 and 3.6; 32 MB 3.3 and 1.3 | 1.8 and 1.1; 8 MB 0.97 and
+// 0.42 | 0.44 and 0.31; 4 MB 0.90 and 0.44 | 0.23 and 0.19; below, the warm copy
+// is as fast plain (2 MB: 0.11 and 0.12).  Six threads gain nothing more.
+static constexpr size_t kReadStaged = 4 << 20;
 static constexpr int kReaders = 4, kReadSlots = 8;
 static int read_back(dtm_solver* s, void* dst, const void* src, size_t bytes) {
   hipPointerAttribute_t at{};
   const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
   (void)hipGetLastError();  // (an unknown pointer may be an error)
-  if (known || bytes < kReadStaged) {
+  auto plain = [&]() -> int {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
     return 0;
-  }
+  };
+  if (known || bytes < kReadStaged) return plain();
   HIPCHK(hipStreamSynchronize(s->stream));  // the readers spin: not while steps run
-  const size_t chunk = bytes <= (4u << 20) ? 512u << 10 : bytes <= (16u << 20) ? 1u << 20 : 2u << 20;
+  const size_t chunk = bytes <= (32u << 20) ? 1u << 20 : 2u << 20;
   const long n = (long)((bytes + chunk - 1) / chunk);
   if (s->ring_bytes < chunk * kReadSlots) {
     if (s->ring) (void)hipHostFree(s->ring);
     s->ring = nullptr;
     s->ring_bytes = 0;
-    HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&s->ring), chunk * kReadSlots, hipHostMallocDefault));
+    if (hipHostMalloc(reinterpret_cast<void**>(&s->ring), chunk * kReadSlots, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      s->ring = nullptr;
+      return plain();
+    }
     s->ring_bytes = chunk * kReadSlots;
   }
   for (hipEvent_t& e : s->ring_ev)
