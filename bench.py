@@ -52,12 +52,12 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def profiled_traffic(kernel_prefix, sweep):
+def profiled_traffic(kernel_prefix):
     """HBM bytes per launch of a kernel from the committed rocprofv3 summary
     (FETCH_SIZE and WRITE_SIZE passes, scaled by a plain copy; the file names
     its command): read MB + write MB of the first row whose kernel name starts
     with kernel_prefix, or None."""
-    path = os.path.join(ROOT, "profiles", f"k_{'torre_fused' if sweep else 'update_twopass'}_fp32_512x256x256.txt")
+    path = os.path.join(ROOT, "profiles", "k_sweep_fp32_512x256x256.txt")
     try:
         for line in open(path):
             if line.startswith(kernel_prefix):
@@ -324,9 +324,8 @@ def main():
     dom = r32["groups"][r32["dominant"]]
     achieved = dom["gbs"]
     # measured HBM bytes of the dominant kernel, from the committed profile
-    prefix = {"E sweep": "void dtm::k_update_e<0, 3, 1,", "H sweep": "void dtm::k_update_h<0, 3, 1,",
-              "fused step": "void dtm::k_torre2<0, 3>"}.get(r32["dominant"], "")
-    tr = profiled_traffic(prefix, sw) if prefix and (nx, ny, nz) == (512, 256, 256) else None
+    prefix = {"E sweep": "void dtm::k_sweep<1, 0,", "H sweep": "void dtm::k_sweep<0, 0,"}.get(r32["dominant"], "")
+    tr = profiled_traffic(prefix) if prefix and (nx, ny, nz) == (512, 256, 256) else None
     out = {
         "metric": "Gcells/s at 512x256x256 FP32 vs FP16-store; adjoint/forward time ratio",
         "value": round(r32["gcells"], 3),

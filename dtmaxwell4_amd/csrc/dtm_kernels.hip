@@ -38,10 +38,6 @@ __device__ __forceinline__ void stx(__half* F, long long q, float v, float s, co
   if (xq >= 0) xz.f[comp][xq] = v;
   st(F, q, v, s);
 }
-template <typename T>
-__device__ __forceinline__ float ldn(const T* F, long long q, bool ok, float inv) {
-  return ok ? ld(F, q, inv) : 0.0f;
-}
 
 // Neighbour index along one axis with the boundary rule: -1 => zero field.
 __device__ __forceinline__ int nbr(int v, int o, int n, int per) {
@@ -51,11 +47,6 @@ __device__ __forceinline__ int nbr(int v, int o, int n, int per) {
   return w < 0 ? w + n : w - n;
 }
 
-// (2,4) difference with weights (+1, -27, +27, -1) on the samples at
-// half-offsets (-3, -1, +1, +3) (genAlg.py:196-198, sign folded).
-__device__ __forceinline__ float d24(float f0, float f1, float f2, float f3) {
-  return 27.0f * (f2 - f1) - (f3 - f0);
-}
 
 // ------------------------------------------------------- incident fields
 __device__ __forceinline__ void wave3(int waveform, double p, double w, double kEnv, double t0, double tw,
@@ -140,11 +131,6 @@ __device__ __forceinline__ double incident(const Tfsf& s, int comp, int hx, int 
   }
 }
 
-__device__ __forceinline__ bool in_sf(const Tfsf& s, int hx, int hy, int hz) {
-  const bool inside = hx >= s.hlo[0] && hx <= s.hhi[0] && hy >= s.hlo[1] && hy <= s.hhi[1] &&
-                      hz >= s.hlo[2] && hz <= s.hhi[2];
-  return s.sf_inside ? inside : !inside;
-}
 
 // Component living at half-coordinates (genAlg.py:24 typing).
 __device__ __forceinline__ int comp_at(int hx, int hy, int hz) {
@@ -200,12 +186,6 @@ __device__ __forceinline__ long long psi_index(const Grid& g, const Cpml& p, int
   return ((long long)i * g.ny + j) * P + s;
 }
 
-// psi <- b psi + c D ; D <- D + psi   (CPML, kappa=1, alpha=0)
-__device__ __forceinline__ void cpml_apply(float* psi, long long pq, float b, float c, float& D) {
-  float v = b * psi[pq] + c * D;
-  psi[pq] = v;
-  D += v;
-}
 // ============================================================ ADE cells
 // Dispersive / gyrotropic cells: countDisp (dispersion.cpp:85-99) and the
 // magnetised-plasma current, from the curl H the E sweep stored.

@@ -30,11 +30,12 @@
 // Bounds and figures (us a step of both sweeps, plane wave on a sphere, CPML;
 // in brackets the sweeps before these: 64 x 8 or 16 column tiles in LDS with a
 // barrier per plane, one cell per lane):
-//   512x256x256 FP32  565 (591)  HBM: 73 B/cell and psi at 4.8 TB/s, a copy 4.7-5.3
-//               FP16  356 (477)  HBM and issue: 37 B/cell and psi at 4.2 TB/s
-//   200^3       FP32  122 (161)  FP16  82 (152)  fields partly, or all, in the Infinity Cache
-//   128^3       FP32   38  (57)  FP16  31  (53)  one or two rounds of waves: latency and issue
-//    64^3       FP32   13  (33)  FP16  14  (35)  two launches of one plane per wave: latency
+//   512x256x256 FP32  564 (591)  HBM: 73 B/cell and psi at 5.1-5.4 TB/s, a copy 4.7-5.3
+//               FP16  353 (477)  HBM and issue: 37 B/cell and psi at 4.5-4.7 TB/s
+//   200^3       FP32  121 (161)  FP16  80 (152)  fields partly, or all, in the Infinity Cache
+//   128^3       FP32   38  (57)  FP16  30  (53)  one or two rounds of waves: latency and issue
+//    64^3       FP32   12  (33)  FP16  13  (35)  two launches of one plane per wave: latency
+// (whole grid; several steps of a large grid run slab by slab, see skewed_steps).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -992,11 +993,12 @@ void go(SweepArgs& A, hipStream_t st) {
   Sweep& w = A.sw;
   const int len = w.i1 - w.i0, nlb = w.lb1 - w.lb0, nhb = w.hb1 - w.hb0;
   // Segments.  Up to six planes per resident wave: one round of waves, each
-  // marching its share (64^3: one plane, 17 us a step; 16 planes 63 us).
+  // marching its share (us a step: 64^3 in segments of 1 / 2 / 8 planes 12.7 /
+  // 15.4 / 35.4, 128^3 in 1 / 2 / 3 / 5 planes 41.0 / 39.4 / 38.3 / 41.7).
   // Beyond: several rounds of short segments, which balance the planes and
   // rows with a layer against those without; shorter ones load the three
-  // planes of a segment's start too often (512x256x256 FP32: segments of 43
-  // planes 634 us a step, 16: 535, 7: 508, 3: 519).
+  // planes of a segment's start too often (256^3 in 1 / 2 / 3 / 6 / 8 planes
+  // FP32 338 / 311 / 296 / 298 / 310, FP16 251 / 212 / 196 / 192 / 191).
   const double share = (double)nlb * len / slots;
   w.seg = share <= 6 ? std::max(1, (int)ceil(share)) : std::max(STORE == 1 ? 4 : 2, (int)(share / 6 + 0.5));
   auto segs = [&](int a, int b) { return (long long)((b - a + w.seg - 1) / w.seg); };
@@ -1186,9 +1188,9 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   if (store == 1 && sc.xz.on) {
     // The blocks whose stencils reach the FP32 zone run the zone's variants,
     // the others the plain ones, which skip those: the two launches write
-    // disjoint cells and read only the other family of fields.  The dispersive
-    // 256^3 emitter run with a zone of 21^3 cells: 377 us a step, against 471
-    // with zone variants on every block of the zone's planes.
+    // disjoint cells and read only the other family of fields.  (256^3 with a
+    // zone of 21^3 cells: the two zone launches take 26 us a step, 121 with zone
+    // variants on every block of the zone's planes.)
     const Exact& x = sc.xz;
     w.h0 = g.per[0] ? i0 : std::min(std::max(x.i0 - 3, i0), i1);
     w.h1 = g.per[0] ? i1 : std::min(std::max(x.i1 + 3, w.h0), i1);

@@ -54,9 +54,6 @@ template <typename T> using GlobalT = __attribute__((address_space(1))) T;
 template <typename T> __device__ __forceinline__ GlobalT<T>* gl(T* p) { return (GlobalT<T>*)p; }
 // the table itself lives in the constant address space: scalar loads
 using ColdK = __attribute__((address_space(4))) const TorreCold;
-__device__ __forceinline__ void st(__half* F, long long q, float v, float s) {
-  gl(reinterpret_cast<unsigned short*>(F))[q] = __half_as_ushort(__float2half_rn(v * s));
-}
 // word at a position under the boundary rule (off < 0 or plane < 0: zero pad)
 template <typename T>
 __device__ __forceinline__ T ldz(const T* F, long long base, int off, unsigned zidx) {
@@ -86,8 +83,6 @@ __device__ __forceinline__ unsigned psi_index(const Grid& g, unsigned P, int a, 
   if (a == 1) return ((unsigned)i * P + (unsigned)s) * (unsigned)g.nz + (unsigned)k;
   return ((unsigned)i * (unsigned)g.ny + (unsigned)j) * P + (unsigned)s;
 }
-// ring slot of plane p in an R-plane ring (p >= -8)
-template <int R> __device__ __forceinline__ int slot(int p) { return (p + 4 * R) % R; }
 
 struct TorreTile {
   int r, i0, i1, j0, k0;
