@@ -1203,10 +1203,13 @@ static const TorreCold* torre_cold(dtm_solver* s) {
   return s->cold_dev[k];
 }
 
-// The soft sources' contributions to E of step n.
+// The soft sources' contributions to E of step n.  Sources of one component of
+// one cell are one entry, their sum: k_soft's lanes each read, subtract and write
+// a value, so two entries for one would lose all but one of them.
 static void soft_values(const dtm_solver* s, long long n, Soft& so) {
   const dtm_config& c = s->cfg;
-  so.n = c.nsoft;
+  so.n = 0;
+  double val[DTM_MAX_SOFT];
   const double th = ((double)n + 0.5) * c.dt;
   for (int q = 0; q < c.nsoft; q++) {
     const dtm_soft_source& ss = c.soft[q];
@@ -1219,13 +1222,20 @@ static void soft_values(const dtm_solver* s, long long n, Soft& so) {
         ie = s->design_host[((size_t)di * s->mt.d_nj + dj) * s->mt.d_nk + dk];
     }
     const double J = ss.amp * wave_value(ss.waveform, ss.w, ss.kEnv, ss.t0, ss.tw, th);
-    so.comp[q] = ss.comp;
-    so.q[q] = (long long)idx;
-    so.ijk[q][0] = ss.i;
-    so.ijk[q][1] = ss.j;
-    so.ijk[q][2] = ss.k;
-    so.val[q] = (float)(c.dt * ie * J);
+    int at = 0;
+    while (at < so.n && (so.comp[at] != ss.comp || so.q[at] != (long long)idx)) at++;
+    if (at == so.n) {
+      so.n++;
+      so.comp[at] = ss.comp;
+      so.q[at] = (long long)idx;
+      so.ijk[at][0] = ss.i;
+      so.ijk[at][1] = ss.j;
+      so.ijk[at][2] = ss.k;
+      val[at] = 0.0;
+    }
+    val[at] += c.dt * ie * J;
   }
+  for (int q = 0; q < so.n; q++) so.val[q] = (float)val[q];
 }
 
 // The probes on the x planes [i0, i1), for step n into row `row` of the series
