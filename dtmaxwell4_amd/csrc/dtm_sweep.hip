@@ -279,11 +279,13 @@ __device__ __forceinline__ float cpml(float old, float b, float c, float D) { re
 // genAlg.py:219-221 is added to the derivative it belongs to, from this
 // half-step's factor table.
 // XZ: half storage with the FP32 zone.
+// SO: soft sources are subtracted from the new E.  Only launches with sources
+// run it: in the ragged FP32 sweep the block costs 9 spilled registers, 3 without.
 //
 // Registers decide the waves per SIMD: four in half storage (128 VGPRs; at
 // three the 512x256x256 step took 14% longer), three in FP32 (168; at four it
 // spills and takes 25% longer).
-template <int UP, int STORE, bool GEN, bool SP, bool TF, bool XZ, int AD>
+template <int UP, int STORE, bool GEN, bool SP, bool TF, bool XZ, int AD, bool SO>
 __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 : 3)) void k_sweep(SweepArgs A) {
   using S = Word<STORE, XZ>;
   using V = Vec<S, NV>;
@@ -910,7 +912,7 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
       putf(stored(1), op, pn1);
       putf(stored(2), op, pn2);
     }
-    if constexpr (UP && STORE == 0 && !TF) {  // launch_sweep: soft_in
+    if constexpr (SO) {
       if (i >= A.soft.lo && i < A.soft.hi) {
         const ArgsK* C = again();
         for (int t = 0; t < C->soft.n; t++) {
@@ -987,9 +989,9 @@ int resident_waves(K kernel) {  // waves of one launch that fit on the device at
   return per * p.multiProcessorCount;
 }
 
-template <int UP, int STORE, bool GEN, bool SP, bool TF, bool XZ, int AD>
+template <int UP, int STORE, bool GEN, bool SP, bool TF, bool XZ, int AD, bool SO = false>
 void go(SweepArgs& A, hipStream_t st) {
-  static const int slots = resident_waves(k_sweep<UP, STORE, GEN, SP, TF, XZ, AD>);
+  static const int slots = resident_waves(k_sweep<UP, STORE, GEN, SP, TF, XZ, AD, SO>);
   Sweep& w = A.sw;
   const int len = w.i1 - w.i0, nlb = w.lb1 - w.lb0, nhb = w.hb1 - w.hb0;
   // Segments.  Up to six planes per resident wave: one round of waves, each
@@ -1014,7 +1016,7 @@ void go(SweepArgs& A, hipStream_t st) {
   w.per = (w.total[2] + NXCD - 1) / NXCD;
   const int more = (int)((record_threads(A.pr) + 63) / 64);
   if (blocks == 0 && more == 0) return;
-  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD>), dim3(w.per * NXCD + more), dim3(64), 0, st, A);
+  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD, SO>), dim3(w.per * NXCD + more), dim3(64), 0, st, A);
   note_launch(UP ? "k_sweep E" : "k_sweep H");
 }
 
@@ -1051,6 +1053,10 @@ void pick(SweepArgs& A, bool split, hipStream_t st) {
     else go<UP, STORE, true, false, true, false, kFar>(A, st);
   } else if (split) {
     go<UP, STORE, true, true, true, false, kNear>(A, st);
+  } else if (A.soft.n > 0) {  // FP32 E (launch_sweep: soft_in)
+    constexpr bool SO = UP && STORE == 0;
+    if (plain) go<UP, STORE, false, false, false, false, kNear, SO>(A, st);
+    else go<UP, STORE, true, false, false, false, kNear, SO>(A, st);
   } else if (plain) {
     if (A.fold) go<UP, STORE, false, false, true, false, kNear>(A, st);
     else go<UP, STORE, false, false, false, false, kNear>(A, st);
@@ -1154,10 +1160,14 @@ void launch_sweep(int up, int store, const Grid& g, const void* fields, const Sc
   const int nlb = (int)((w.NL + 63) / 64);
   if (store) fill<1>(A, up, false, g, fields, sc, pm);
   else fill<0>(A, up, false, g, fields, sc, pm);
-  // Soft sources are subtracted where E is new in the plain FP32 variants:
-  // k_soft's launch took 1.8 of 36 us a step at 128^3.  In the variants with the
-  // fold or in half storage the few registers this takes made spills that cost
-  // every step 2 to 4%: there k_soft follows.
+  // Soft sources are subtracted where E is new by FP32 variants of their own
+  // (SO), which only launches with sources run: us a step at 44^3, 100^3, 128^3,
+  // 160^3, 198^3 11.2, 23.2, 34.4, 62.5, 101.3 so and 13.1, 24.8, 36, 63.6, 102.2
+  // with k_soft's launch after the sweep; from 206^3 on both take the same.  In
+  // the one ragged variant that all grids ran before, the block cost those
+  // without sources 1% to 4%: 131^3 39.7 and 39.4 without it, 180^3 78.2 and 76.6,
+  // 300^3 453 and 432.  With the fold or in half storage it spills more, and
+  // every step takes 2 to 4% longer: there k_soft follows.
   const bool soft_in = here.n > 0 && here.n <= kSweepSoft && store == 0 && !fold && !split && addressing(A) == kNear;
   if (soft_in) {
     A.soft.lo = g.nx;
