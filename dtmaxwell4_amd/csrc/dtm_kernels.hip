@@ -132,41 +132,27 @@ __device__ __forceinline__ double incident(const Tfsf& s, int comp, int hx, int 
 }
 
 
-// Component living at half-coordinates (genAlg.py:24 typing).
-__device__ __forceinline__ int comp_at(int hx, int hy, int hz) {
-  const int o0 = hx & 1, o1 = hy & 1, o2 = hz & 1;
-  if (o0 + o1 + o2 == 2) return o0 == 0 ? 0 : (o1 == 0 ? 1 : 2);
-  return o0 ? 3 : (o1 ? 4 : 5);
-}
-
-// Sum over the 4 stencil neighbours along axis a of component-at-(hp) of the
-// TF/SF corrections (genAlg.py:219-221) weighted by (+1,-27,+27,-1).
-// TAB 1: plane wave with k along one axis, the incident value is the
-// polarisation factor P[comp] times this half-step's waveform table entry;
-// TAB 2: a dipole's point table (k_tfsf_points); TAB 0: evaluated here.
+// Sum over the 4 stencil neighbours along axis a, which hold component cq, of
+// the TF/SF corrections (genAlg.py:219-221) weighted by (+1,-27,+27,-1).
 // The neighbours differ from the point only along a, so no face is crossed
 // unless the point lies inside the box on the other two axes; then a
 // neighbour crosses when its a-coordinate is on the other side of [hlo, hhi].
-__device__ __forceinline__ float tfsf_dcorr(const Tfsf& s, int hx, int hy, int hz, int a, double t) {
-  const int hp[3] = {hx, hy, hz};
-  const int b1 = (a + 1) % 3, b2 = (a + 2) % 3;
-  if (hp[b1] < s.hlo[b1] || hp[b1] > s.hhi[b1] || hp[b2] < s.hlo[b2] || hp[b2] > s.hhi[b2]) return 0.f;
-  const int h = hp[a], lo = s.hlo[a], hi = s.hhi[a];
-  const bool pin = h >= lo && h <= hi;
-  const int ho[4] = {-3, -1, 1, 3};
-  const double wt[4] = {1.0, -27.0, 27.0, -1.0};
-  // the four neighbours (odd offsets along a) hold one component, the same
-  // for every cell of a band and component (wavefront-uniform)
-  const int cq = __builtin_amdgcn_readfirstlane(comp_at(a == 0 ? hx + 1 : hx, a == 1 ? hy + 1 : hy, a == 2 ? hz + 1 : hz));
+__device__ __forceinline__ float tfsf_dcorr(const Tfsf& s, int hx, int hy, int hz, int a, int cq, double t) {
+  const bool inx = hx >= s.hlo[0] && hx <= s.hhi[0], iny = hy >= s.hlo[1] && hy <= s.hhi[1],
+             inz = hz >= s.hlo[2] && hz <= s.hhi[2];
+  if (!((a == 0 || inx) && (a == 1 || iny) && (a == 2 || inz))) return 0.f;
+  const int h = a == 0 ? hx : (a == 1 ? hy : hz), lo = s.hlo[a], hi = s.hhi[a];
+  const bool pin = a == 0 ? inx : (a == 1 ? iny : inz);
   double acc = 0.0;
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const int hq = h + ho[q];
+    const int hq = h + 2 * q - 3;
     const bool qin = hq >= lo && hq <= hi;
     if (qin == pin) continue;
     const bool qsf = s.sf_inside ? qin : !qin;  // the neighbour is in the scattered-field region
     const double v = incident(s, cq, a == 0 ? hq : hx, a == 1 ? hq : hy, a == 2 ? hq : hz, t);
-    acc += wt[q] * (qsf ? v : -v);
+    const double wt = q == 0 ? 1.0 : (q == 1 ? -27.0 : (q == 2 ? 27.0 : -1.0));
+    acc += wt * (qsf ? v : -v);
   }
   return (float)acc;
 }
@@ -382,40 +368,45 @@ template <int MODE>
 __device__ __forceinline__ void tfsf_term(const Grid& g, const Cpml& pm, int a, int c, int t, float D, int i, int j,
                                           int k, float* dc, float* dc2) {
   constexpr int HALF = MODE == 1 ? 1 : 0;
-  const int vpos[3] = {i, j, k};
+  auto pos = [&](int ax) { return ax == 0 ? i : (ax == 1 ? j : k); };
+  auto add = [&](float* d, float v) {
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+      if (e == c) d[e] += v;
+  };
   const float sgn = t == 0 ? 1.0f : -1.0f;
   const int slot = t == 0 ? 1 : 0;  // psi slots 1 and 0 of axis a
   float cp = 0.0f;
   if (pm.on && pm.split) {  // split-field layer: the part of axis a gets k2 * D
     auto k2_of = [&](int ax) {  // 1 off the slab of axis ax
       const int n = ax == 0 ? g.nx : (ax == 1 ? g.ny : g.nz);
-      if (slab_index(vpos[ax], n, pm.plo[ax], pm.phi[ax]) < 0) return 1.0f;
-      return HALF == 0 ? pm.cH[ax][vpos[ax]] : pm.cE[ax][vpos[ax]];
+      if (slab_index(pos(ax), n, pm.plo[ax], pm.phi[ax]) < 0) return 1.0f;
+      return HALF == 0 ? pm.cH[ax][pos(ax)] : pm.cE[ax][pos(ax)];
     };
     const float k2 = k2_of(a);
     // the cell keeps split parts when either curl axis has k2 != 1; the
     // second curl axis (t = 1) owns the stored part
     if (k2 != 1.0f || k2_of(t == 0 ? (c + 2) % 3 : (c + 1) % 3) != 1.0f) {
-      dc[c] += sgn * k2 * D;
-      if (t == 1) dc2[c] += sgn * k2 * D;
+      add(dc, sgn * k2 * D);
+      if (t == 1) add(dc2, sgn * k2 * D);
       return;
     }
   } else if (pm.on) {
     const int n = a == 0 ? g.nx : (a == 1 ? g.ny : g.nz);
-    const int si = slab_index(vpos[a], n, pm.plo[a], pm.phi[a]);
+    const int si = slab_index(pos(a), n, pm.plo[a], pm.phi[a]);
     if (si >= 0) {
-      cp = HALF == 0 ? pm.cH[a][vpos[a]] : pm.cE[a][vpos[a]];
+      cp = HALF == 0 ? pm.cH[a][pos(a)] : pm.cE[a][pos(a)];
       float* psi = HALF == 0 ? pm.psiH[a][slot] : pm.psiE[a][slot];
       const long long pq = psi_index(g, pm, a, si, i, j, k);
       if (MODE == 2) {
-        psi[pq] += cp * D / pm.bH[a][vpos[a]];
+        psi[pq] += cp * D / pm.bH[a][pos(a)];
         cp = 0.0f;
       } else {
         psi[pq] += cp * D;
       }
     }
   }
-  dc[c] += sgn * (1.0f + cp) * D;
+  add(dc, sgn * (1.0f + cp) * D);
 }
 
 // Adds the corrections of a cell to its fields.
@@ -463,21 +454,30 @@ __device__ __forceinline__ void tfsf_apply(const Grid& g, const Fields<STORE>& f
 
 constexpr int kOff[6][3] = {{0, 1, 1}, {1, 0, 1}, {1, 1, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
 
-// Incident field evaluated at every point.
+// Incident field evaluated at every point.  Bound by its FP64 instructions
+// (sines and exponentials) at three waves a SIMD; the axis is a scalar and no
+// array is indexed by it, or the grid's constants go to scratch memory and
+// registers for two waves are left.  Both launches of a step, oblique wave: 128^3
+// 68.0 us so, 49.6 now; 256^3 215 and 139; dipole box of 40^3 cells 69.7 and 63.5.
+// (One copy of the evaluation for the four neighbours too: 50.8, 143, 66.6.)
 template <int STORE, int MODE>
 __global__ __launch_bounds__(256) void k_tfsf(Grid g, Fields<STORE> f, Scales sc, Cpml pm, Materials mt, Ade ade,
                                               Tfsf tf, TfsfBands bands, double tinc) {
   int r, i, j, k;
   if (!band_cell(bands, r, i, j, k)) return;
+  r = __builtin_amdgcn_readfirstlane(r);
   float dc[3] = {0.f, 0.f, 0.f}, dc2[3] = {0.f, 0.f, 0.f};
+#pragma nounroll
   for (int rb = r; rb < bands.n; rb++) {
     if (rb != r && !band_has(bands, r, rb, i, j, k)) continue;
-    const int a = bands.axis[rb];
-    // components with a derivative along a: (a+2)%3 (first curl term), (a+1)%3 (second)
+    const int a = __builtin_amdgcn_readfirstlane(bands.axis[rb]), b1 = a == 2 ? 0 : a + 1, b2 = a == 0 ? 2 : a - 1;
+    // components with a derivative along a: b2 (first curl term), b1 (second)
+#pragma nounroll
     for (int t = 0; t < 2; t++) {
-      const int c = t == 0 ? (a + 2) % 3 : (a + 1) % 3;
-      const int comp = MODE == 1 ? c : 3 + c;
-      const float D = g.rd[a] * tfsf_dcorr(tf, 2 * i + kOff[comp][0], 2 * j + kOff[comp][1], 2 * k + kOff[comp][2], a, tinc);
+      const int c = t == 0 ? b2 : b1, cq = (MODE == 1 ? 3 : 0) + (t == 0 ? b1 : b2);
+      auto half = [&](int v, int e) { return 2 * v + ((e == c) == (MODE == 1) ? 0 : 1); };
+      const float rd0 = g.rd[0], rd1 = g.rd[1], rd2 = g.rd[2], rd = a == 0 ? rd0 : (a == 1 ? rd1 : rd2);
+      const float D = rd * tfsf_dcorr(tf, half(i, 0), half(j, 1), half(k, 2), a, cq, tinc);
       if (D == 0.0f) continue;
       tfsf_term<MODE>(g, pm, a, c, t, D, i, j, k, dc, dc2);
     }

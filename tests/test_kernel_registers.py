@@ -1,7 +1,9 @@
-"""Vector registers that the FP32 sweeps of the main path keep in scratch memory
-in launches without soft sources, from the kernel descriptors of the built
-library: none in the H sweeps; in the E sweeps none, 3 with a ragged z extent or
-with a folded plane wave, 7 with both."""
+"""Registers of kernels, from their descriptors in the built library.  FP32 sweeps
+of the main path in launches without soft sources: no vector register of the H
+sweeps in scratch memory; of the E sweeps none, 3 with a ragged z extent or with
+a folded plane wave, 7 with both.  The TF/SF correction that evaluates the
+incident field at every point: no scratch memory, and registers for three waves
+a SIMD."""
 import os
 import re
 import shutil
@@ -15,7 +17,7 @@ LLVM = "/opt/rocm/llvm/bin"
 
 
 @pytest.fixture(scope="module")
-def spills(tmp_path_factory):
+def kernels(tmp_path_factory):
     if not os.path.exists(os.path.join(LLVM, "llvm-readelf")) or not os.path.exists(abi.LIB_PATH):
         pytest.skip("needs the built library and ROCm's LLVM tools")
     d = str(tmp_path_factory.mktemp("code"))
@@ -29,7 +31,9 @@ def spills(tmp_path_factory):
         text = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", name], cwd=d, check=True,
                               stdout=subprocess.PIPE, text=True).stdout
         for k in text.split("- .agpr_count:")[1:]:
-            out[re.search(r"\.name:\s+(\S+)", k).group(1)] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", k).group(1))
+            out[re.search(r"\.name:\s+(\S+)", k).group(1)] = {
+                f: int(re.search(rf"\.{f}:\s+(\d+)", k).group(1))
+                for f in ("vgpr_count", "vgpr_spill_count", "private_segment_fixed_size")}
     return out
 
 
@@ -40,6 +44,13 @@ def sweep(up, general, fold, soft=0):
 
 @pytest.mark.parametrize("up,general,fold,most", [
     (0, 0, 0, 0), (0, 1, 0, 0), (0, 0, 1, 0), (0, 1, 1, 0), (1, 0, 0, 0), (1, 1, 0, 3), (1, 0, 1, 3), (1, 1, 1, 7)])
-def test_sweeps_without_soft_sources(spills, up, general, fold, most):
-    got = [n for name, n in spills.items() if sweep(up, general, fold) in name]
+def test_sweeps_without_soft_sources(kernels, up, general, fold, most):
+    got = [k["vgpr_spill_count"] for name, k in kernels.items() if sweep(up, general, fold) in name]
     assert len(got) == 1 and got[0] <= most
+
+
+@pytest.mark.parametrize("store", [0, 1])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_correction_with_the_incident_field(kernels, store, mode):
+    got = [k for name, k in kernels.items() if f"6k_tfsfILi{store}ELi{mode}E" in name]
+    assert len(got) == 1 and got[0]["private_segment_fixed_size"] == 0 and got[0]["vgpr_count"] <= 168
