@@ -8,6 +8,7 @@
 
 #include <algorithm>
 
+#include "dtm_box.h"
 #include "dtm_internal.h"
 #include "dtm_probe.h"
 
@@ -176,7 +177,7 @@ __device__ __forceinline__ long long psi_index(const Grid& g, const Cpml& p, int
 // Dispersive / gyrotropic cells: countDisp (dispersion.cpp:85-99) and the
 // magnetised-plasma current, from the curl H the E sweep stored.
 //
-// One lane per cell of the bounding box, nblk blocks per x plane.  A box of a
+// One lane per cell of the bounding box (dtm_box.h).  A box of a
 // few 10^5 cells is bound by its chain of loads more than by its bytes: the
 // special classes are a mask in the arguments, so a cell's class byte says at
 // once whether its state is needed, all of that is loaded together (NP and
@@ -186,8 +187,8 @@ __device__ __forceinline__ long long psi_index(const Grid& g, const Cpml& p, int
 // FP16 with the FP32 zone 18.9, against 20.7 and 30 with the class entry, the
 // material and each pole fetched in turn by the lane that needs them.
 template <int STORE> struct AdeArgs {
-  unsigned nblk;
-  int nj, nk, i0, j0, k0;  // the box
+  BoxUnits un;
+  int ni, nj, nk, i0, j0, k0;  // the box
   long long sx, sy;
   const uint8_t* cls;
   decltype(Fields<STORE>::E) E, Ed;  // E^n, E^{n+1}
@@ -202,11 +203,11 @@ template <int STORE> struct AdeArgs {
   Exact xz;
 };
 template <int STORE, int NP, bool GYRO, bool XZ>
-__global__ __launch_bounds__(256) void k_ade(AdeArgs<STORE> A) {
-  const unsigned ip = blockIdx.x / A.nblk;
+__global__ __launch_bounds__(kBoxBlock) void k_ade(AdeArgs<STORE> A) {
   const unsigned long long pl = (unsigned long long)(unsigned)A.nj * (unsigned)A.nk;  // cells of a plane of the box
-  const unsigned long long loc = (blockIdx.x - ip * A.nblk) * 256ull + threadIdx.x;
-  const bool live = loc < pl;
+  unsigned ip;
+  unsigned long long loc;
+  const bool live = box_lane(A.un, (unsigned)A.ni, pl, blockIdx.x, threadIdx.x, ip, loc);
   const int jb = pl >> 32 ? (int)(loc / (unsigned)A.nk) : (int)((unsigned)loc / (unsigned)A.nk);
   const int i = A.i0 + (int)ip, j = A.j0 + jb;
   const int k = A.k0 + (int)(loc - (unsigned long long)jb * (unsigned)A.nk);
@@ -824,7 +825,7 @@ template <int STORE, bool XZ>
 static void ade_go(const Grid& g, const Fields<STORE>& f, const Fields<STORE>& fd, const Scales& sc,
                    const Materials& mt, const Ade& ade, hipStream_t st) {
   AdeArgs<STORE> A{};
-  A.nblk = (unsigned)(((long long)ade.nj * ade.nk + 255) / 256);
+  A.ni = ade.ni;
   A.nj = ade.nj;
   A.nk = ade.nk;
   A.i0 = ade.i0;
@@ -858,18 +859,20 @@ static void ade_go(const Grid& g, const Fields<STORE>& f, const Fields<STORE>& f
     A.dn[c] = dn[c];
   }
   A.xz = sc.xz;
-  const dim3 grid(A.nblk * (unsigned)ade.ni), blk(256);
-  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, blk, 0, st, A); };
-  if (ade.gyro_on) {
-    if (ade.npoles > 2) run(k_ade<STORE, 4, true, XZ>);
-    else if (ade.npoles > 0) run(k_ade<STORE, 2, true, XZ>);
-    else run(k_ade<STORE, 0, true, XZ>);
-  } else {
-    if (ade.npoles > 2) run(k_ade<STORE, 4, false, XZ>);
-    else if (ade.npoles > 1) run(k_ade<STORE, 2, false, XZ>);
-    else if (ade.npoles > 0) run(k_ade<STORE, 1, false, XZ>);
-    else run(k_ade<STORE, 0, false, XZ>);
-  }
+  box_launches((unsigned)ade.ni, (unsigned long long)ade.nj * ade.nk, [&](const BoxUnits& un, unsigned blocks) {
+    A.un = un;
+    auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBoxBlock), 0, st, A); };
+    if (ade.gyro_on) {
+      if (ade.npoles > 2) run(k_ade<STORE, 4, true, XZ>);
+      else if (ade.npoles > 0) run(k_ade<STORE, 2, true, XZ>);
+      else run(k_ade<STORE, 0, true, XZ>);
+    } else {
+      if (ade.npoles > 2) run(k_ade<STORE, 4, false, XZ>);
+      else if (ade.npoles > 1) run(k_ade<STORE, 2, false, XZ>);
+      else if (ade.npoles > 0) run(k_ade<STORE, 1, false, XZ>);
+      else run(k_ade<STORE, 0, false, XZ>);
+    }
+  });
   check_launch("k_ade");
 }
 

@@ -1006,17 +1006,18 @@ void go(SweepArgs& A, hipStream_t st) {
   auto segs = [&](int a, int b) { return (long long)((b - a + w.seg - 1) / w.seg); };
   const long long n[3] = {segs(w.i0, w.h0) * nlb, segs(w.h0, w.h1) * (nlb - nhb), segs(w.h1, w.i1) * nlb};
   const long long blocks = n[0] + n[1] + n[2];
-  if (blocks > (1LL << 30)) {
-    fail_launch("k_sweep", "more than 2^30 blocks");
+  const long long more = (record_threads(A.pr) + 63) / 64;
+  // (a launch of 2^32 lanes or more may run only some of its blocks, without an error)
+  if (blocks + NXCD + more >= (1LL << 26)) {
+    fail_launch("k_sweep", "2^26 blocks or more");
     return;
   }
   w.total[0] = (int)n[0];
   w.total[1] = (int)(n[0] + n[1]);
   w.total[2] = (int)blocks;
   w.per = (w.total[2] + NXCD - 1) / NXCD;
-  const int more = (int)((record_threads(A.pr) + 63) / 64);
   if (blocks == 0 && more == 0) return;
-  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD, SO>), dim3(w.per * NXCD + more), dim3(64), 0, st, A);
+  hipLaunchKernelGGL((k_sweep<UP, STORE, GEN, SP, TF, XZ, AD, SO>), dim3(w.per * NXCD + (int)more), dim3(64), 0, st, A);
   note_launch(UP ? "k_sweep E" : "k_sweep H");
 }
 
