@@ -1378,8 +1378,13 @@ static SkewPlan skew_plan(const dtm_solver* s) {
                                                           (double)(c.npml[4] + c.npml[5]) * c.ny));
   const double total = plane * c.nx + (s->pm.split ? 0.0 : 16.0 * yz * (c.npml[0] + c.npml[1]));
   if (total <= kCacheResident) return p;
+  // Slabs of few planes have small groups, and gain little or nothing: one step at
+  // a time and skewed, us a step, FP32 with 46 / 41 / 30 / 25 planes (256x512, 384^2,
+  // 448^2, 490^2) 1070 and 981 / 914 and 865 / 1293 and 1257 / 1764 and 1781, with 18
+  // (600^2) 1661 and 1730; FP16 with 84 / 58 / 52 / 47 / 33 (384^2, 300x700, 480^2, 500^2,
+  // 600^2) 704 and 682 / 986 and 978 / 1032 and 1092 / 959 and 999 / 1307 and 1407.
   const int most = (int)(kCacheSlab / plane);
-  if (most < 24) return p;
+  if (most < (s->store ? 56 : 24)) return p;
   const int ns = (c.nx + most - 1) / most;
   p.slab = (c.nx + ns - 1) / ns;
   p.group = std::min(16, p.slab / 6);

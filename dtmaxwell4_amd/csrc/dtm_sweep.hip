@@ -62,6 +62,8 @@ using rsrc = __amdgpu_buffer_rsrc_t;
 // blocks [hb0, hb1) of the planes [h0, h1) (the hole, whose planes are below
 // h0 = i1 if there is none).  The planes before, of and after the hole are cut
 // into segments of seg planes: total[] are the blocks up to the end of each.
+// Planes of more than SweepArgs::strip blocks are run strip by strip: all segments
+// of the first `strip` blocks of a plane, then those of the next.
 struct Sweep {
   int i0, i1, seg, lb0, lb1;
   int h0, h1, hb0, hb1;
@@ -93,6 +95,7 @@ struct SweepArgs {
   const float* fold;    // this half-step's factor table, and the packed weights of every chunk
   const int2* foldw;
   int pml, plo[3], phi[3];
+  int strip;  // of Sweep
   float* psi[3][2];
   const float* b[3];
   const float* c[3];
@@ -334,12 +337,21 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
     nlb -= A.sw.hb1 - A.sw.hb0;
     hole = true;
   }
+  int lb = A.sw.lb0;
+  if (nlb > A.strip) {
+    const int nseg = (hi - lo + A.sw.seg - 1) / A.sw.seg, sp = lid / (nseg * A.strip);
+    lid -= sp * nseg * A.strip;
+    lb += sp * A.strip;
+    nlb = min(A.strip, nlb - sp * A.strip);
+  }
   const int bs = lid / nlb;
-  int lb = lid - bs * nlb + A.sw.lb0;
+  lb += lid - bs * nlb;
   if (hole && lb >= A.sw.hb0) lb += A.sw.hb1 - A.sw.hb0;
   using LI = typename std::conditional<AD == kHuge, long long, int>::type;
   const LI L = (LI)lb * 64 + (int)threadIdx.x;
-  const int p0 = lo + bs * A.sw.seg, p1 = min(p0 + A.sw.seg, hi);
+  int p0 = lo + bs * A.sw.seg, p1 = min(p0 + A.sw.seg, hi);
+  // (opaque, or what they are made from stays in registers along the march)
+  asm volatile("" : "+s"(p0), "+s"(p1));
   const bool act = L < A.sw.NL;
   const int j = (int)(L / A.sw.nzv), kc = (int)(L - (LI)j * A.sw.nzv), k = NV * kc;
   const int nz = A.nz, perz = A.per[2];
@@ -1001,8 +1013,20 @@ void go(SweepArgs& A, hipStream_t st) {
   // rows with a layer against those without; shorter ones load the three
   // planes of a segment's start too often (256^3 in 1 / 2 / 3 / 6 / 8 planes
   // FP32 338 / 311 / 296 / 298 / 310, FP16 251 / 212 / 196 / 192 / 191).
+  // A wave takes the rows beside its own from its XCD's L2, where they are only
+  // while the waves of these rows march abreast.  So planes larger than what the
+  // XCD's waves hold at once run in strips of that size, and segments end before
+  // waves drift far apart.  FP32, all steps over the whole grid, without that and
+  // so: 512x500x500 2215 (40.8 bytes a cell from beyond L2) and 2039, 512^3 2150
+  // and 2043, 300x512x1024 2747 and 2457, 100x1024x1024 1851 and 1690, 400^3 1066
+  // and 1001; FP16 512x500x500 1408 and 1190.  Segments of 4 / 6 / 8 / 12 planes
+  // there: FP32 2048 / 2039 / 2053 / 2071, FP16 1262 / 1219 / 1221 / 1211; strips of
+  // half that size, FP32: 2040 / 2044 / 2069 / 2097.
   const double share = (double)nlb * len / slots;
-  w.seg = share <= 6 ? std::max(1, (int)ceil(share)) : std::max(STORE == 1 ? 4 : 2, (int)(share / 6 + 0.5));
+  w.seg = share <= 6 ? std::max(1, (int)ceil(share))
+                     : std::min(std::max(STORE == 1 ? 4 : 2, (int)(share / 6 + 0.5)), STORE == 1 ? 12 : 6);
+  const int strips = share <= 6 ? 1 : (nlb * NXCD + slots - 1) / slots;
+  A.strip = (nlb + std::max(strips, 1) - 1) / std::max(strips, 1);
   auto segs = [&](int a, int b) { return (long long)((b - a + w.seg - 1) / w.seg); };
   const long long n[3] = {segs(w.i0, w.h0) * nlb, segs(w.h0, w.h1) * (nlb - nhb), segs(w.h1, w.i1) * nlb};
   const long long blocks = n[0] + n[1] + n[2];
