@@ -74,7 +74,7 @@ struct dtm_solver {
   void* H[3] = {};
   void* E2[3] = {};  // second buffers of the fused (torre) step
   void* H2[3] = {};
-  Fields<0> f32{}, f32n{};
+  Fields<0> f32{};
   Fields<1> f16{}, f16n{};
   Cpml pm{};         // current psi
   Cpml pmn{};        // second psi buffers (torre step)
@@ -678,8 +678,6 @@ static void field_structs(dtm_solver* s) {
     s->f32.H[c] = static_cast<float*>(s->H[c]);
     s->f16.E[c] = static_cast<__half*>(s->E[c]);
     s->f16.H[c] = static_cast<__half*>(s->H[c]);
-    s->f32n.E[c] = static_cast<float*>(s->E2[c]);
-    s->f32n.H[c] = static_cast<float*>(s->H2[c]);
     s->f16n.E[c] = static_cast<__half*>(s->E2[c]);
     s->f16n.H[c] = static_cast<__half*>(s->H2[c]);
   }
@@ -688,9 +686,7 @@ static void field_structs(dtm_solver* s) {
 static const void* fields_ptr(const dtm_solver* s) {
   return s->store == 0 ? static_cast<const void*>(&s->f32) : static_cast<const void*>(&s->f16);
 }
-static const void* fields_next_ptr(const dtm_solver* s) {
-  return s->store == 0 ? static_cast<const void*>(&s->f32n) : static_cast<const void*>(&s->f16n);
-}
+static const void* fields_next_ptr(const dtm_solver* s) { return &s->f16n; }  // (fused step: half storage)
 
 // After a fused step the new buffers become current.
 static void swap_buffers(dtm_solver* s) {
@@ -907,8 +903,8 @@ int dtm_create(const dtm_config* cfg, dtm_solver** out) {
     return fail(DTM_ERR_ARG, "the split-field layer runs with the two-pass sweeps");
   if (c.sweep == DTM_SWEEP_FUSED &&
       6ull * ((unsigned long long)c.nx * c.ny * c.nz + kPad) * (c.storage ? 2 : 4) >= (1ull << 32))
-    return fail(DTM_ERR_LIMIT, "the fused step addresses a field set (six arrays) with 32-bit byte offsets: "
-                               "at most 4 GiB, use the two-pass sweeps for larger grids");
+    return fail(DTM_ERR_LIMIT, "the fused schedule takes field sets (six arrays) of at most 4 GiB, which its "
+                               "half-storage kernel can address: use the two-pass sweeps for larger grids");
   const int n3[3] = {c.nx, c.ny, c.nz};
   for (int a = 0; a < 3; a++) {
     if (c.npml[2 * a] < 0 || c.npml[2 * a + 1] < 0 || c.npml[2 * a] + c.npml[2 * a + 1] > n3[a])
@@ -1269,7 +1265,7 @@ static int one_step(dtm_solver* s) {
   // Probes ride with the two sweeps: the H probes of a step with its E sweep,
   // its E probes with the next step's H sweep, or, at the end of a call or of
   // a block of the series, with a launch of their own.
-  const bool ride = !s->torre && !s->timing && (long long)np * std::max(s->nfreq, 1) < (1 << 30);
+  const bool ride = !s->torre && !s->timing;
   const Probes pr = rec ? probes_of(s, n, s->series_row, 0, c.nx) : Probes{};
   // Soft sources go into the E sweep, unless it does not run or k_tfsf adds to
   // the new E first.
