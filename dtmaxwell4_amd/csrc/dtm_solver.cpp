@@ -81,8 +81,8 @@ struct dtm_solver {
   // One kernel a step (dtm_torre.hip): the fused schedule in FP16 storage, where
   // its E update reads H before that is rounded.  In FP32 the two in-place
   // sweeps give the same update in less time and half the memory, so the
-  // schedule runs them (200^3: 131 us a step, that kernel's 228; 512x256x256:
-  // 572 and 614; 64^3: 17 and 29).
+  // schedule runs them (200^3: 123 us a step, that kernel's 227; 512x256x256:
+  // 531 and 606; 64^3: 12 and 26).
   bool torre = false;
   bool no_fold = false; // tabulated plane-wave TF/SF through k_tfsf instead of the sweeps
   float* fold_base = nullptr; // per-plane factors of a folded plane wave, kTableSteps x 2 half-steps
@@ -167,15 +167,18 @@ static int dalloc(dtm_solver* s, T** p, size_t bytes) {
   return 0;
 }
 
-// dalloc for buffers that hold time-stepped state.  64 bytes more are
+// dalloc for buffers that hold time-stepped state.  kStatePad bytes more are
 // allocated on either side: a lane of the sweeps reads whole chunks of cells,
 // the first or last one of an array past its ends where a slab or the z extent
-// is no multiple of a chunk.
+// is no multiple of a chunk.  A chunk's 16 bytes would do, but a whole number of
+// cache lines keeps the arrays' own alignment (with 64 bytes the fused FP16 step
+// took 595 us at 512x256x256, 590 so; the sweeps up to 1% more).
+static constexpr size_t kStatePad = 256;
 template <typename T>
 static int sdalloc(dtm_solver* s, T** p, size_t bytes) {
   char* base = nullptr;
-  if (int rc = dalloc(s, &base, bytes + 128)) return rc;
-  *p = reinterpret_cast<T*>(base + 64);
+  if (int rc = dalloc(s, &base, bytes + 2 * kStatePad)) return rc;
+  *p = reinterpret_cast<T*>(base + kStatePad);
   s->state.emplace_back(static_cast<void*>(*p), bytes == 0 ? 16 : bytes);
   return 0;
 }
