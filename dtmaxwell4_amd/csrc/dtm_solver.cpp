@@ -65,7 +65,6 @@ struct dtm_solver {
   hipStream_t stream = nullptr;
   char* ring = nullptr;  // pinned chunks of large field reads (read_back)
   size_t ring_bytes = 0;
-  int plain_reads = 0;  // of fields that the ring would take (read_back)
   hipEvent_t ring_ev[8] = {};
   Grid g{};
   Scales sc{};
@@ -1812,11 +1811,7 @@ static int zone_copy(dtm_solver* s, int comp, float* buf, bool to_host) {
 // 134 MB 12.8 and 3.6 | 7.4 and 3.6; 32 MB 3.3 and 1.3 | 1.8 and 1.1; 8 MB 0.97 and
 // 0.42 | 0.44 and 0.31; 4 MB 0.90 and 0.44 | 0.23 and 0.19; below, the warm copy
 // is as fast plain (2 MB: 0.11 and 0.12).  Six threads gain nothing more.
-// Making the ring takes about 1 ms: a solver's first read of 8 MB 1.5 ms with it
-// and 0.49 plain, of 16 MB 2.3 and 2.4.  So below kReadOnce the first kReadPlain
-// reads are plain, and programs that look at a field once never pay for it.
-static constexpr size_t kReadStaged = 4 << 20, kReadOnce = 15 << 20;
-static constexpr int kReadPlain = 2;
+static constexpr size_t kReadStaged = 4 << 20;
 static constexpr int kReaders = 4, kReadSlots = 8;
 static int read_back(dtm_solver* s, void* dst, const void* src, size_t bytes) {
   hipPointerAttribute_t at{};
@@ -1828,7 +1823,6 @@ static int read_back(dtm_solver* s, void* dst, const void* src, size_t bytes) {
     return 0;
   };
   if (known || bytes < kReadStaged) return plain();
-  if (!s->ring && bytes < kReadOnce && s->plain_reads++ < kReadPlain) return plain();
   HIPCHK(hipStreamSynchronize(s->stream));  // the readers spin: not while steps run
   const size_t chunk = bytes <= (32u << 20) ? 1u << 20 : 2u << 20;
   const long n = (long)((bytes + chunk - 1) / chunk);
