@@ -30,9 +30,10 @@ GROUPS_FUSED = ("fused step", "-", "-", "-", "TF/SF+ADE+sources+probes")
 # Algorithmic bytes per cell, the roofline basis: two-pass half-step sweep:
 # read 3E+3H, write 3 components (+1 class byte for E): 36 / 37 B in FP32.
 # Fused step of FP16 storage (H and E in one pass): read 3E+3H, write 3E+3H,
-# read the class byte: 25 B; in FP32 the fused schedule runs the two sweeps.  The CPML psi (two FP32 values read and written per half-step
-# for each slab a cell lies in: 16 B; 32 B per fused step) is region-local
-# and reported beside it (psi_bytes, roofline.extra_bytes), not in it.
+# read the class byte: 25 B; in FP32 the fused schedule runs the two sweeps.
+# The CPML psi (two FP32 values read and written per half-step for each slab a
+# cell lies in: 16 B; 32 B per fused step) is region-local and reported beside
+# it (psi_bytes, roofline.extra_bytes), not in it.
 WORDS_PER_HALF = 9
 WORDS_FUSED = 12
 PSI_BYTES_HALF = 2 * 2 * 4
@@ -323,6 +324,7 @@ def main():
             log(f"[bench] cpu baseline failed: {e}")
     dom = r32["groups"][r32["dominant"]]
     achieved = dom["gbs"]
+    step_bytes = sum(g["algorithmic_bytes"] + g["psi_bytes"] for g in r32["groups"].values())
     # measured HBM bytes of the dominant kernel, from the committed profile
     prefix = {"E sweep": "void dtm::k_sweep<1, 0,", "H sweep": "void dtm::k_sweep<0, 0,"}.get(r32["dominant"], "")
     tr = profiled_traffic(prefix) if prefix and (nx, ny, nz) == (512, 256, 256) else None
@@ -349,7 +351,10 @@ def main():
                      "kernel": r32["kernel"] + " " + r32["dominant"], "avg_launch_ms": dom["avg_ms"],
                      "algorithmic_bytes_per_launch": dom["algorithmic_bytes"], "cells_per_launch": dom["cells"],
                      "extra_bytes": dom["psi_bytes"], "extra": "CPML psi bytes per launch (not in achieved)",
-                     "achieved_with_extra": round(dom["gbs_with_psi"], 1)},
+                     "achieved_with_extra": round(dom["gbs_with_psi"], 1),
+                     "launches": "whole grid, one step at a time, as event timing runs them; the timed steps of "
+                                 "`value` advance slab by slab and take part of their traffic from the Infinity Cache",
+                     "timed_steps_gbs_with_extra": round(step_bytes / (r32["ms"] / args.steps * 1e-3) / 1e9, 1)},
         "effective_yee_gbs": round(r32["gcells"] * 72, 1),
         "effective_yee_frac": round(r32["gcells"] * 72 / HBM_PEAK_GBS, 4),
         "fp16_store": None if r16 is None else {

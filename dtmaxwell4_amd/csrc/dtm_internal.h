@@ -349,11 +349,6 @@ void launch_fold_weights(const Tfsf& tf, int2* out, const Grid& g, hipStream_t s
 // floats per half-step of the fold factor table: (nx + 1) * 8
 void launch_tfsf_fold(const Tfsf& tf, const double* tables, float* out, int nsteps, const Grid& g,
                       hipStream_t st);
-// TF/SF corrections applied after a sweep (half = 0: H, 1: E).  The update is
-// linear in the stencil sums, so the correction is additive, including its
-// CPML psi and ADE J terms.
-// mode 0: H post-correction, 1: E post-correction, 2: H pre-correction
-// (applied to H^{n-1/2} and psi before a fused step: psi += c D / b).
 // design-gradient adjoint (FP32 storage)
 // Both on the x planes [i0, i1).  Record: the design box's E into snap (null:
 // not) and Ez at the monitors into series (null: not).  Inject / grad: dJ/dE at
@@ -365,6 +360,10 @@ void launch_adj_inject_grad(const Grid& g, const void* fields, const Materials& 
                             const float* e1, double* acc, const long long* q, const float* inv_eps, const double* F,
                             int nmon, double w, double dt, long long n, hipStream_t st);
 void launch_tfsf_tables(const Tfsf& tf, double* out, long long n0, int nsteps, double dt, hipStream_t st);
+// TF/SF corrections applied after a sweep.  The update is linear in the stencil
+// sums, so the correction is additive, including its CPML psi and ADE J terms.
+// half 0: H post-correction, 1: E post-correction, 2: H pre-correction (applied to
+// H^{n-1/2} and psi before a fused step: psi += c D / b).
 void launch_tfsf(int store, int half, const Grid& g, const void* fields, const Scales& sc, const Cpml& pm,
                  const Materials& mt, const Ade& ade, const Tfsf& tf, const TfsfBands& bands, double t_inc,
                  hipStream_t st);

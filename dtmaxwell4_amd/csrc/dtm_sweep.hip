@@ -30,11 +30,12 @@
 // Bounds and figures (us a step of both sweeps, plane wave on a sphere, CPML;
 // in brackets the sweeps before these: 64 x 8 or 16 column tiles in LDS with a
 // barrier per plane, one cell per lane):
-//   512x256x256 FP32  564 (591)  HBM: 73 B/cell and psi at 5.1-5.4 TB/s, a copy 4.7-5.3
-//               FP16  353 (477)  HBM and issue: 37 B/cell and psi at 4.5-4.7 TB/s
-//   200^3       FP32  121 (161)  FP16  80 (152)  fields partly, or all, in the Infinity Cache
-//   128^3       FP32   38  (57)  FP16  30  (53)  one or two rounds of waves: latency and issue
-//    64^3       FP32   12  (33)  FP16  13  (35)  two launches of one plane per wave: latency
+//   512x256x256 FP32  557 (587)  HBM: 88 B/cell (Yee words 73, psi 7.5) at 5.1-5.4 TB/s, a copy 4.7-5.3
+//               FP16  348 (471)  HBM and issue: 48 B/cell (Yee words 37, psi 7.5) at 4.5-4.7 TB/s
+//   256^3       FP32  302 (316)  FP16 192 (250)
+//   200^3       FP32  122 (160)  FP16  82 (148)  fields partly, or all, in the Infinity Cache
+//   128^3       FP32   37  (54)  FP16  30  (49)  one or two rounds of waves: latency and issue
+//    64^3       FP32   12  (29)  FP16  12  (31)  two launches of one plane per wave: latency
 // (whole grid; several steps of a large grid run slab by slab, see skewed_steps).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -370,7 +371,9 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
   // A wave's first loads (fold weights, layer coefficients, the queues) go out
   // before the rest of its start is worked out, without a branch, in the order
   // of their use: waiting for one after the other took 1.3 of 13.9 us a step at
-  // 64^3 and 1.6 of 39 at 128^3.
+  // 64^3 and 1.6 of 39 at 128^3.  The first plane's own loads follow only after
+  // waits: for the coefficients on their way to LDS, for the fold weights, and in
+  // E for class 0's flag, a load after the queues and so for all of them.
   // packed TF/SF weights of the cells (k_fold_weights)
   int fz = 0, fi = 0;
   if constexpr (TF) {
@@ -958,8 +961,9 @@ __global__ __launch_bounds__(64, XZ || SP || AD == kHuge ? 2 : (STORE == 1 ? 4 :
     constexpr unsigned ALL = (1u << NV) - 1u;
     // whole chunks with one store per component for every lane (a lane that
     // stores only some cells addresses none here), so that the number of
-    // stores in flight is known and the wait for the next plane's loads does
-    // not reach them
+    // stores in flight is known and, in E, the wait for the next plane's loads
+    // does not reach them.  (In H the loop's head waits for all that is under way,
+    // these stores too: on the first way in that is the queues.)
     const O whole = put == ALL ? own : OUT;
     using H = Vec<Word<STORE, false>, NV>;
     auto word = [&](F v, float sc) {

@@ -358,7 +358,10 @@ int dtm_time_steps(dtm_solver* s, int nsteps, double* ms);
 /* Name of the kernel variant used for the E/H sweep. */
 const char* dtm_kernel_name(const dtm_solver* s);
 /* Per-launch HIP-event timing of the sweep kernels, recorded on the solver's
- * stream while enabled.  Groups: 0 H sweep (fused schedule: the whole step),
+ * stream while enabled.  While it is on, every step is taken over the whole grid
+ * and probes are recorded by a launch of their own: a grid larger than the
+ * Infinity Cache otherwise advances several steps slab by slab within a call, in
+ * less time than the groups' sum (the results are the same bit for bit).  Groups: 0 H sweep (fused schedule: the whole step),
  * 1 unused, 2 E sweep, 3 unused, 4 TF/SF, ADE, sources and probes.
  * dtm_kernel_times returns the summed ms and launch counts per group and
  * resets them. */
